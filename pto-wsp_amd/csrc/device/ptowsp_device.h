@@ -146,6 +146,108 @@ __device__ inline float team_max(float x) {
     return x;
 }
 
+// Rows whose width does not split evenly over a wide enough team (row_layout
+// on the host): the team covers NV*G*VW >= C columns, and the chunks past
+// column C - 1 are absent.  Absent elements hold 0 and take no part in the
+// reductions.  With VW 4 the accesses are declared aligned to one element
+// only (the row pitch of an odd width is odd too; global memory takes
+// unaligned 128-bit accesses), and the one chunk that straddles the row's
+// end goes element by element.
+//
+// HBM bound.  Softmax over 32,768 rows of 1001 columns (262 MB): one lane per
+// row, the layout these widths had before, kept 1001 values per lane in
+// 14 KB of scratch and took 1006 us; a team of 64 lanes takes 47 us (5.6
+// TB/s).  Scalar accesses are level there (45 us) and slower for narrow rows
+// (19 columns: 25 against 13 us) and wide ones (8128: 544 against 133 us).
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef u32 u32x2h __attribute__((ext_vector_type(2), aligned(2)));
+
+// Whether element e of chunk k of lane j lies in the row (constant, after
+// unrolling, for the chunks that are whole for every lane).
+template <int VW, int G, int C>
+__device__ inline bool row_has(int k, int e, int j) {
+    return (k + 1) * G * VW <= C || (k * G + j) * VW + e < C;
+}
+
+template <int NV, int VW, int G, bool NT, int C>
+__device__ inline void row_load_m(RowSlice<NV, VW>& r, const float* p, i64 s4, int j) {
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+        if constexpr (VW == 4) {
+            const int q = (k * G + j) * 4;
+            f32x4u x = {0.0f, 0.0f, 0.0f, 0.0f};
+            if (row_has<4, G, C>(k, 3, j)) {
+                const f32x4u* a = reinterpret_cast<const f32x4u*>(p + q);
+                x = NT ? __builtin_nontemporal_load(a) : *a;
+            } else if constexpr (C % 4 != 0) {
+                if (q < C) {
+#pragma unroll
+                    for (int e = 0; e < C % 4; ++e) x[e] = p[q + e];
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) r.v[k * 4 + e] = x[e];
+        } else {
+            static_assert(VW == 1, "masked rows: 4 or 1 elements per access");
+            r.v[k] = row_has<1, G, C>(k, 0, j) ? p[static_cast<i64>(k * G + j) * s4] : 0.0f;
+        }
+    }
+}
+
+template <int NV, int VW, int G, int C>
+__device__ inline void row_load_strided_m(RowSlice<NV, VW>& r, const float* p, i64 stride, int j) {
+#pragma unroll
+    for (int k = 0; k < NV; ++k)
+#pragma unroll
+        for (int e = 0; e < VW; ++e)
+            r.v[k * VW + e] = row_has<VW, G, C>(k, e, j) ? p[static_cast<i64>((k * G + j) * VW + e) * stride] : 0.0f;
+}
+
+template <int NV, int VW, int G, bool NT, int C>
+__device__ inline void row_store_m(float* p, const RowSlice<NV, VW>& r, i64 s4, int j) {
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+        if constexpr (VW == 4) {
+            const int q = (k * G + j) * 4;
+            if (row_has<4, G, C>(k, 3, j)) {
+                const f32x4u x = {r.v[k * 4], r.v[k * 4 + 1], r.v[k * 4 + 2], r.v[k * 4 + 3]};
+                f32x4u* a = reinterpret_cast<f32x4u*>(p + q);
+                if (NT) __builtin_nontemporal_store(x, a);
+                else *a = x;
+            } else if constexpr (C % 4 != 0) {
+                if (q < C) {
+#pragma unroll
+                    for (int e = 0; e < C % 4; ++e) p[q + e] = r.v[k * 4 + e];
+                }
+            }
+        } else {
+            if (row_has<1, G, C>(k, 0, j)) p[static_cast<i64>(k * G + j) * s4] = r.v[k];
+        }
+    }
+}
+
+// Sum over the row's elements.  A lane without elements starts from -0, the
+// identity of fp addition.
+template <int NV, int VW, int G, int C>
+__device__ inline float row_sum_m(const RowSlice<NV, VW>& r, int j) {
+    float a = -0.0f;
+#pragma unroll
+    for (int i = 0; i < NV * VW; ++i) a = row_has<VW, G, C>(i / VW, i % VW, j) ? a + r.v[i] : a;
+    return team_sum<G>(a);
+}
+
+// Maximum with the oracle's left-to-right `x > acc ? x : acc`: a NaN is kept
+// only as the row's first element, so lane 0 of the team, which holds it,
+// has the result.
+template <int NV, int VW, int G, int C>
+__device__ inline float row_max_m(const RowSlice<NV, VW>& r, int j) {
+    float a = j == 0 ? r.v[0] : -__builtin_inff();
+#pragma unroll
+    for (int i = 0; i < NV * VW; ++i) a = row_has<VW, G, C>(i / VW, i % VW, j) && r.v[i] > a ? r.v[i] : a;
+    a = team_max<G>(a);
+    return G == 1 ? a : __shfl(a, static_cast<int>(threadIdx.x & 63) & ~(G - 1), 64);
+}
+
 // Elementwise binary ops with the cpu_sim operator semantics (a>b?a:b for max).
 struct OpAdd { template <class T> __device__ static T f(T a, T b) { return a + b; } };
 struct OpSub { template <class T> __device__ static T f(T a, T b) { return a - b; } };
@@ -245,6 +347,29 @@ __device__ inline void row_store_h(u16* p, const RowSlice<NV, VW>& r, i64 s4, in
     } else {
 #pragma unroll
         for (int k = 0; k < NV; ++k) p[static_cast<i64>(k * G + j) * s4] = f32_to_h16_bits<DT>(r.v[k]);
+    }
+}
+
+template <int NV, int VW, int G, int DT, int C>
+__device__ inline void row_store_h_m(u16* p, const RowSlice<NV, VW>& r, i64 s4, int j) {
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+        if constexpr (VW == 4) {
+            const int q = (k * G + j) * 4;
+            if (row_has<4, G, C>(k, 3, j)) {
+                u32x2h x;
+                x.x = f32_to_h16_bits<DT>(r.v[k * 4 + 0]) | (static_cast<u32>(f32_to_h16_bits<DT>(r.v[k * 4 + 1])) << 16);
+                x.y = f32_to_h16_bits<DT>(r.v[k * 4 + 2]) | (static_cast<u32>(f32_to_h16_bits<DT>(r.v[k * 4 + 3])) << 16);
+                *reinterpret_cast<u32x2h*>(p + q) = x;
+            } else if constexpr (C % 4 != 0) {
+                if (q < C) {
+#pragma unroll
+                    for (int e = 0; e < C % 4; ++e) p[q + e] = f32_to_h16_bits<DT>(r.v[k * 4 + e]);
+                }
+            }
+        } else {
+            if (row_has<1, G, C>(k, 0, j)) p[static_cast<i64>(k * G + j) * s4] = f32_to_h16_bits<DT>(r.v[k]);
+        }
     }
 }
 

@@ -113,7 +113,7 @@ std::string offset_expr(int p, int nvars, int first_term, int nterms) {
 
 }  // namespace
 
-RowLayout row_layout(int cols, int vw, int up_cap) {
+RowLayout row_layout(int cols, int vw, int up_cap, bool unit_cols) {
     RowLayout l;
     l.vw = vw;
     const int n = cols / vw;
@@ -121,7 +121,23 @@ RowLayout row_layout(int cols, int vw, int up_cap) {
     while (g < 64 && n % (g * 2) == 0) g *= 2;
     l.g = g;
     l.nv = n / g;
-    int up = 32 / (l.nv * vw);
+    // The even split serves a row well when the team is full, when it reads
+    // runs of 64 bytes or more and a lane holds at most 32 values, or when
+    // the row is a few values per lane.  Other widths (odd ones above all:
+    // one lane per row) take a team of up to 64 lanes that reaches past the
+    // row's end, its last chunks absent.  Device time, even split against
+    // masked: 1001 columns 1006 / 47 us, 446 (16k rows) 87 / 16, 100 (64k
+    // rows) 52 / 16, 19 (262k rows) 33 / 13, 24 15.8 / 12.6.
+    const bool even = g == 64 || (g * vw >= 16 && l.nv * vw <= 32) || l.nv * vw <= 4;
+    if (!even) {
+        l.vw = unit_cols ? 4 : 1;
+        const int chunks = (cols + l.vw - 1) / l.vw;
+        l.g = 1;
+        while (l.g < 64 && l.g < chunks) l.g *= 2;
+        l.nv = (chunks + l.g - 1) / l.g;
+        l.masked = true;
+    }
+    int up = 32 / (l.nv * l.vw);
     if (up_cap < 1) up_cap = 1;
     l.up = up < 1 ? 1 : (up > up_cap ? up_cap : up);
     return l;
@@ -135,8 +151,19 @@ namespace {
 EmittedKernel emit_row(const Module& m, const KernelAnalysis& a, const LaunchSpec& L, const EmitSpec& spec) {
     (void)m;
     const KernelDef& k = *a.def;
-    const RowLayout lay = row_layout(a.cols, spec.vec_width, spec.row_up);
-    const char* nt = spec.nontemporal ? ", true" : "";
+    const RowLayout lay = row_layout(a.cols, spec.vec_width, spec.row_up, spec.row_unit_cols);
+    // Template arguments and suffixes of the row accesses: masked layouts
+    // carry the column count.
+    const std::string cm = std::to_string(a.cols);
+    const std::string sfx = lay.masked ? "_m" : "";
+    // Streaming accesses pay where a row is whole 128-byte lines (2880
+    // columns: 130 against 141 us without); a masked row that ends inside a
+    // line shares it with the next row's accesses and is better left cached
+    // (1000 columns: 48.6 us streaming, 42.7 us not; 1001: 51.1 and 47.5).
+    const std::string ntb = spec.nontemporal && a.cols % 32 == 0 ? "true" : "false";
+    const std::string nt = lay.masked ? ", " + ntb + ", " + cm : spec.nontemporal ? ", true" : "";
+    const std::string nont = lay.masked ? ", false, " + cm : "";
+    const std::string cmx = lay.masked ? ", " + cm : "";
     const int R = a.rows, C = a.cols, ng = static_cast<int>(L.grid.size());
     const int rpw = 64 / lay.g, ch = rpw * lay.up;
     const bool chunk_in_task = R % ch == 0;
@@ -240,10 +267,10 @@ EmittedKernel emit_row(const Module& m, const KernelAnalysis& a, const LaunchSpe
         const DType dt = a.by_id[dparam]->dtype;
         const std::string ps = std::to_string(p);
         if (full && dt == DType::F32)
-            o << ind << "if (ok[u]) row_store<NV, VW, G" << nt << ">((float*)" << basep << " + (i64)rr[u] * A.s3[" << ps << "], " << val
+            o << ind << "if (ok[u]) row_store" << sfx << "<NV, VW, G" << nt << ">((float*)" << basep << " + (i64)rr[u] * A.s3[" << ps << "], " << val
               << ", A.s4[" << ps << "], j);\n";
         else if (full)
-            o << ind << "if (ok[u]) row_store_h<NV, VW, G, " << dt_code(dt) << ">((u16*)" << basep << " + (i64)rr[u] * A.s3[" << ps
+            o << ind << "if (ok[u]) row_store_h" << sfx << "<NV, VW, G, " << dt_code(dt) << cmx << ">((u16*)" << basep << " + (i64)rr[u] * A.s3[" << ps
               << "], " << val << ", A.s4[" << ps << "], j);\n";
         else if (dt == DType::F32)
             o << ind << "if (ok[u] && j == 0) ((float*)" << basep << ")[(i64)rr[u] * A.s3[" << ps << "]] = " << val << ";\n";
@@ -259,7 +286,7 @@ EmittedKernel emit_row(const Module& m, const KernelAnalysis& a, const LaunchSpe
         const std::string tbp = base(p);
         switch (cls(id)) {
             case RowClass::Full:
-                o << ind1 << "RS ld" << id << "[UP];\n#pragma unroll\n" << ind1 << "for (int u = 0; u < UP; ++u) row_load<NV, VW, G" << nt << ">(ld" << id
+                o << ind1 << "RS ld" << id << "[UP];\n#pragma unroll\n" << ind1 << "for (int u = 0; u < UP; ++u) row_load" << sfx << "<NV, VW, G" << nt << ">(ld" << id
                   << "[u], (const float*)" << tbp << " + (i64)rr[u] * A.s3[" << p << "], A.s4[" << p << "], j);\n";
                 break;
             case RowClass::RowVec:
@@ -271,11 +298,11 @@ EmittedKernel emit_row(const Module& m, const KernelAnalysis& a, const LaunchSpe
                   << "[u] = ((const float*)" << tbp << ")[(i64)rr[u] * A.s4[" << p << "]];\n";
                 break;
             case RowClass::ColVec:
-                o << ind1 << "RS ld" << id << "[UP];\n#pragma unroll\n" << ind1 << "for (int u = 0; u < UP; ++u) row_load<NV, VW, G>(ld" << id
+                o << ind1 << "RS ld" << id << "[UP];\n#pragma unroll\n" << ind1 << "for (int u = 0; u < UP; ++u) row_load" << sfx << "<NV, VW, G" << nont << ">(ld" << id
                   << "[u], (const float*)" << tbp << ", A.s4[" << p << "], j);\n";
                 break;
             case RowClass::ColVecT:
-                o << ind1 << "RS ld" << id << "[UP];\n#pragma unroll\n" << ind1 << "for (int u = 0; u < UP; ++u) row_load_strided<NV, VW, G>(ld"
+                o << ind1 << "RS ld" << id << "[UP];\n#pragma unroll\n" << ind1 << "for (int u = 0; u < UP; ++u) row_load_strided" << sfx << "<NV, VW, G" << cmx << ">(ld"
                   << id << "[u], (const float*)" << tbp << ", A.s3[" << p << "], j);\n";
                 break;
             default: throw CompileError("row program: bad load class");
@@ -389,7 +416,8 @@ EmittedKernel emit_row(const Module& m, const KernelAnalysis& a, const LaunchSpe
                 const int src_cols = a.by_id[x]->cols;
                 o << "      const float v" << r << " = ";
                 if (cls(x) == RowClass::Full) {
-                    if (op.kind == OpKind::RowMax) o << "team_max<G>(lane_max<NV * VW>(" << vname(x) << ".v))";
+                    if (lay.masked) o << (op.kind == OpKind::RowMax ? "row_max_m" : "row_sum_m") << "<NV, VW, G, " << cm << ">(" << vname(x) << ", j)";
+                    else if (op.kind == OpKind::RowMax) o << "team_max<G>(lane_max<NV * VW>(" << vname(x) << ".v))";
                     else o << "team_sum<G>(lane_sum<NV * VW>(" << vname(x) << ".v))";
                 } else {
                     o << vname(x);

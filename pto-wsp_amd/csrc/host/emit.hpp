@@ -12,6 +12,7 @@ namespace ptowsp {
 // Launch-time facts a kernel is specialized on.
 struct EmitSpec {
     int vec_width = 1;                 // row programs: 4, 2 or 1 floats per access
+    bool row_unit_cols = false;        // row programs: full-row and column-vector params have unit column stride
     std::vector<int> indirect_count;   // per tensor ordinal: indirect index terms (in dim order)
     std::vector<int> inner_dyn_term;   // per inner loop: indirect term index of its extent, or -1
     int threads = 256;
@@ -94,7 +95,10 @@ EmittedKernel emit_launch(const Module& m, const KernelAnalysis& a, const Launch
 // accesses `vw` wide: lanes per row G, chunks per lane NV, unrolled passes UP.
 struct RowLayout {
     int vw = 1, g = 1, nv = 1, up = 1;
+    bool masked = false;  // the team's last chunks reach past the row's end
 };
-RowLayout row_layout(int cols, int vw, int up_cap = 8);
+// unit_cols: every full-row access has unit column stride, so that accesses
+// of 4 elements, aligned to one, may be used where the width is not even.
+RowLayout row_layout(int cols, int vw, int up_cap = 8, bool unit_cols = false);
 
 }  // namespace ptowsp

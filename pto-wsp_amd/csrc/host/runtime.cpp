@@ -431,19 +431,25 @@ struct BuiltLaunch {
     std::vector<int64_t> tasks;  // task-list launches: the grid tasks kept by the masks
 };
 
+// How param p of a row program is accessed: its own class, or that of a Load
+// of it.
+RowClass row_access_class(const KernelAnalysis& a, size_t p) {
+    const int id = a.def->params[a.tensor_param_index[p]].id;
+    RowClass c = a.row_class[id];
+    for (const auto& op : a.def->ops)
+        if (op.kind == OpKind::Load && op.operands[0] == id && op.result > 0 &&
+            (a.row_class[op.result] == RowClass::Full || a.row_class[op.result] == RowClass::ColVec))
+            c = a.row_class[op.result];
+    return c;
+}
+
 // Row-program vector width allowed by the actual strides and alignment.
 int pick_vec_width(const KernelAnalysis& a, const LaunchArgs& A, int nvars) {
     for (int vw : {4, 2}) {
         if (a.cols % vw) continue;
         bool ok = true;
         for (size_t p = 0; p < a.tensor_param_index.size() && ok; ++p) {
-            const int id = a.def->params[a.tensor_param_index[p]].id;
-            // The param's own class, or that of a Load of it, decides how it is accessed.
-            RowClass c = a.row_class[id];
-            for (const auto& op : a.def->ops)
-                if (op.kind == OpKind::Load && op.operands[0] == id && op.result > 0 &&
-                    (a.row_class[op.result] == RowClass::Full || a.row_class[op.result] == RowClass::ColVec))
-                    c = a.row_class[op.result];
+            const RowClass c = row_access_class(a, p);
             if (c != RowClass::Full && c != RowClass::ColVec) continue;
             if (A.s4[p] != 1) ok = false;
             if (reinterpret_cast<uintptr_t>(A.base[p]) % (vw * 4)) ok = false;
@@ -454,6 +460,14 @@ int pick_vec_width(const KernelAnalysis& a, const LaunchArgs& A, int nvars) {
         if (ok) return vw;
     }
     return 1;
+}
+
+bool row_unit_columns(const KernelAnalysis& a, const LaunchArgs& A) {
+    for (size_t p = 0; p < a.tensor_param_index.size(); ++p) {
+        const RowClass c = row_access_class(a, p);
+        if ((c == RowClass::Full || c == RowClass::ColVec) && A.s4[p] != 1) return false;
+    }
+    return true;
 }
 
 // Launch-shape defaults of the row-program family, from a sweep on MI355X
@@ -1076,6 +1090,7 @@ BuiltLaunch build_launch(RunEnv& E, const LaunchSpec& L) {
     B.spec.decode_waves = tuning().decode_waves ? tuning().decode_waves : decode_waves_for(a.decode.d, a.decode.g, a.decode.f32);
     B.spec.decode_ordered = tuning().decode_ordered;
     B.spec.vec_width = a.family == Family::RowProgram ? pick_vec_width(a, A, nvars) : 1;
+    B.spec.row_unit_cols = a.family == Family::RowProgram && row_unit_columns(a, A);
     B.spec.threads = tuning().tile_threads;
     B.spec.tile_mma = tuning().tile_mma;
     if (P->ka[L.kernel].family == Family::Custom) {
@@ -1088,7 +1103,7 @@ BuiltLaunch build_launch(RunEnv& E, const LaunchSpec& L) {
 
 std::string spec_key(const EmitSpec& s) {
     std::ostringstream o;
-    o << "vw" << s.vec_width << (s.serial ? ";serial" + std::to_string(s.seq_mask) : "") << (s.task_list ? ";tl" : "") << ";up" << s.row_up << (s.nontemporal ? ";nt" : "")
+    o << "vw" << s.vec_width << (s.row_unit_cols ? "u" : "") << (s.serial ? ";serial" + std::to_string(s.seq_mask) : "") << (s.task_list ? ";tl" : "") << ";up" << s.row_up << (s.nontemporal ? ";nt" : "")
       << (s.row_loops ? ";rl" : "") << (s.gemm ? ";gemm" : "") << ";m" << s.gemm_vm << ";n" << s.gemm_vn << ";f" << s.gemm_fm << "x" << s.gemm_fn << "x" << s.gemm_kf
       << (s.gemm_pingpong ? ";pp" : "")
       << (s.decode ? ";dec" : "")
@@ -1836,6 +1851,7 @@ int ptowsp_hip_precompile(ptowsp_program* P, int index, int flags, const char** 
                         while (vw > 1 && shape.back() % vw) vw /= 2;
                 }
                 spec.vec_width = vw;
+                spec.row_unit_cols = true;
             }
             const int ng = static_cast<int>(L.grid.size());
             if ((flags & 2) && spec.gemm && ng >= 2 && a.gemm.m <= 128 && a.gemm.n <= 128 &&
