@@ -1811,6 +1811,20 @@ struct DecodeSplit {
     static constexpr int kMaxUnits = 4096;  // prefixes held in LDS by every block
     static constexpr int kUnitCost = 3;
     __device__ static int cost(int pages) { return pages > 0 ? pages + kUnitCost : 0; }
+    // Waves to split the launch over, of AW resident ones (at most one per
+    // cost position, so that no wave's cost range is empty).  Splitting a unit
+    // further shortens each wave's share c and adds partials to fold (the
+    // unit's cost over c, by one wave); a page and a partial cost about the
+    // same, so c is the square root of the average unit's cost TC / U, and all
+    // waves are used once that leaves each of them as much (TC / AW >= c).
+    // Device time, C5 heads: two sequences of 512-8192 tokens 34 us (all 1024
+    // waves: 46), one of 8192 40 (47), 18 short ones at head dim 64 23 (36).
+    __device__ static i64 waves_for(i64 TC, int U, int AW) {
+        if (TC * U >= static_cast<i64>(AW) * AW) return AW < TC ? AW : TC;
+        const int c = static_cast<int>(sqrtf(static_cast<float>(static_cast<int>(TC)) / static_cast<float>(U)));
+        const u32 tw = c > 1 ? (static_cast<u32>(TC) + c - 1) / static_cast<u32>(c) : static_cast<u32>(TC);
+        return tw < static_cast<u32>(AW) ? tw : AW;
+    }
     // Wave holding cost position p: the largest w with w*TC/W <= p.
     __device__ static i64 wave_of(i64 p, i64 TC, i64 W) { return ((p + 1) * W - 1) / TC; }
     // Largest u in [0, U) with pre[u] <= s, for 0 <= s < pre[U] (a non-empty unit).
@@ -1846,17 +1860,18 @@ struct PageOffs {
 };
 
 // The addressing hooks of a decode launch (see DecodeStream), from lambdas.
-template <class P, class B, class Q, class S, class C>
+template <class P, class B, class Q, class S, class C, class M>
 struct DecodeFns {
     P page;
     B bases;
     Q q;
     S slot;
     C combine;
+    M combine_many;
 };
-template <class P, class B, class Q, class S, class C>
-__device__ inline DecodeFns<P, B, Q, S, C> decode_fns(P p, B b, Q q, S s, C c) {
-    return DecodeFns<P, B, Q, S, C>{p, b, q, s, c};
+template <class P, class B, class Q, class S, class C, class M>
+__device__ inline DecodeFns<P, B, Q, S, C, M> decode_fns(P p, B b, Q q, S s, C c, M m) {
+    return DecodeFns<P, B, Q, S, C, M>{p, b, q, s, c, m};
 }
 
 // One decode wave's pages [s, b) of the launch (units laid end to end, see
@@ -1879,7 +1894,8 @@ __device__ inline DecodeFns<P, B, Q, S, C> decode_fns(P p, B b, Q q, S s, C c) {
 // DW::kHalves plus the page's half (k < 0 for a half the unit does not
 // have); bases(PageOffs, kp, vp, mp);
 // q(u) (q tile of unit u, or null when out of range); slot(u) (this wave's
-// partial of unit u); combine(u, parts, first_slot).
+// partial of unit u); combine(u, parts, first_slot), and combine_many with the
+// same arguments for a unit of many partials.
 template <class DW, int NB, bool ORDERED>
 struct DecodeStream {
     struct Pending {
@@ -1908,10 +1924,46 @@ struct DecodeStream {
                 if (last) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         }
         if (last) {
-            f.combine(pd.unit, pd.parts, pd.first);
+            if (pd.parts > kManyParts) {
+                if ((threadIdx.x & 63) == 0) {
+                    int* q = many_queue();
+                    const int n = q[0];
+                    q[1 + 3 * n] = pd.unit;
+                    q[2 + 3 * n] = pd.parts;
+                    q[3 + 3 * n] = static_cast<int>(pd.first);
+                    q[0] = n + 1;
+                }
+            } else {
+                f.combine(pd.unit, pd.parts, pd.first);
+            }
             if (pd.parts > 1) reset_count(cnt + pd.unit);
         }
         pd.phase = 0;
+    }
+    // Units of more than kManyParts partials that this wave completes: folded
+    // after its stream, when the page ring's registers are free, by
+    // combine_many (deep loads), instead of two partials at a time in the
+    // middle of the stream.  A wave shares at most two units with other
+    // waves (its first and its last), so two records are enough; they wait in
+    // LDS, since the stream's loop has no scalar registers to spare.  A unit
+    // of up to 8 partials is folded in the stream, behind other waves' pages
+    // (C5 heads at head dim 64, 18 short sequences, 4-5 partials each: 23 us,
+    // with a limit of 4 28 us; 16 sequences at head dim 256, 8-9 partials: 65
+    // us, with a limit of 16 68 us).
+    static constexpr int kManyParts = 8;
+    __device__ static int* many_queue() {
+        __shared__ int q[8][8];
+        return q[wave_index()];
+    }
+    template <class F>
+    __device__ static void fold_many(F& f) {
+        wave_lds_barrier();
+        const int* q = many_queue();
+        const int n = __builtin_amdgcn_readfirstlane(q[0]);
+#pragma unroll 1
+        for (int i = 0; i < n; ++i)
+            f.combine_many(__builtin_amdgcn_readfirstlane(q[1 + 3 * i]), __builtin_amdgcn_readfirstlane(q[2 + 3 * i]),
+                           __builtin_amdgcn_readfirstlane(q[3 + 3 * i]));
     }
     // Completes a pending unit now.
     template <class F>
@@ -1948,6 +2000,7 @@ struct DecodeStream {
     __device__ static void run(F& f, const int* pre, const int* cpre, int U, i64 TC, i64 W, i64 w, i64 s, i64 b, int* cnt,
                                float scale, i64 ks, i64 vs, i64 qs) {
         const int lane = threadIdx.x & 63;
+        if (lane == 0) many_queue()[0] = 0;
         const typename DW::Lanes ln = DW::lanes(ks, vs);
         // Page-table runs: lane i holds the offsets of page i%HS of step
         // r0 + i/HS (f.page takes that half-step index, HS*step + half).
@@ -2057,7 +2110,7 @@ struct DecodeStream {
                     pd.wait = NB;
                     if (eu >= b) {
                         flush(pd, cnt, f);
-                        return;
+                        goto done;  // one copy of what follows, outside the unrolled steps
                     }
                     if constexpr (DW::kPrefetchQ) {
                         u = un;
@@ -2083,6 +2136,8 @@ struct DecodeStream {
                 }
             }
         }
+    done:
+        fold_many(f);
     }
 };
 
@@ -2173,6 +2228,116 @@ struct DecodeCombine {
 #pragma unroll
                         for (int j = 0; j < DPL; ++j) out[g * us3 + part_dim<D>(DPL * lane + j) * us4] = oo[r][j] / ll[r];
                     }
+                }
+            }
+        }
+    }
+    // run() for a unit of many partials (few units over all the waves): one
+    // wave folds them, so what bounds it is the chain of its memory round
+    // trips.  A pass takes 256 / D rows.  m and l are read 64 partials at a
+    // time, a partial per lane, which gives every partial's weight up front;
+    // the o rows, 128 bits per lane, then have no chain between them, and the
+    // first KB partials' are on their way before the weights are known.  Two
+    // sequences of 512-8192 tokens at the C5 heads (16 units): the launch takes
+    // 34 us, where folding 64 partials two at a time took 78.
+    static constexpr int KB = 16;
+    static constexpr int RP = 256 / D;
+    __device__ static f32x4v_t load_o(buf_rsrc rp, int voff, int soff) {
+        return __builtin_bit_cast(f32x4v_t, __builtin_amdgcn_raw_buffer_load_b128(rp, voff, soff, 16));
+    }
+    // Reduction over the wave: within 16 lanes by DPP (quad permutes, half
+    // and full row mirrors), then cross4_reduce; every lane has the result.
+    template <int CTRL>
+    __device__ static float dpp(float x) {
+        return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xF, 0xF, true));
+    }
+    template <class Op>
+    __device__ static float wave_reduce(float x, Op op) {
+        x = op(x, dpp<0xB1>(x));
+        x = op(x, dpp<0x4E>(x));
+        x = op(x, dpp<0x141>(x));
+        x = op(x, dpp<0x140>(x));
+        return cross4_reduce(x, op);
+    }
+    __device__ static void run_many(int nch, const float* part, int pstride, float* m, i64 ms3, float* l, i64 ls3, float* o,
+                                    i64 os3, i64 os4, float* out, i64 us3, i64 us4) {
+        const int lane = threadIdx.x & 63, rr = lane / (D / 4), p0 = 4 * (lane % (D / 4));
+        const buf_rsrc rp = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(part), 0, -1, 0x00020000);
+#pragma unroll 1
+        for (int g0 = 0; g0 < G; g0 += RP) {
+            const int g = g0 + rr < G ? g0 + rr : G - 1;  // a lane past the last row folds it again and stores nothing
+            const int voff = (g * D + p0) * 4;
+            float mm[RP], ll[RP];
+            f32x4v_t oo;
+            // Partials past the end read the last one again, with weight 0.
+            auto load_batch = [&](f32x4v_t(&x)[KB], int c) {
+#pragma unroll
+                for (int b = 0; b < KB; ++b) x[b] = load_o(rp, voff, (c + b < nch ? c + b : nch - 1) * pstride * 4);
+            };
+            f32x4v_t x[KB];
+            load_batch(x, 0);
+#pragma unroll
+            for (int r = 0; r < RP; ++r) {
+                const int gr = g0 + r < G ? g0 + r : G - 1;
+                mm[r] = m[gr * ms3];
+                ll[r] = l[gr * ls3];
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) oo[e] = o[g * os3 + part_dim<D>(p0 + e) * os4];
+#pragma unroll 1
+            for (int c0 = 0; c0 < nch; c0 += 64) {
+                const bool have = c0 + lane < nch;
+                float mc[RP], lc[RP], w[RP], a[RP];
+                const float* pc = part + static_cast<i64>(have ? c0 + lane : nch - 1) * pstride;
+#pragma unroll
+                for (int r = 0; r < RP; ++r) {
+                    const int gr = g0 + r < G ? g0 + r : G - 1;
+                    mc[r] = coherent_load(pc + G * D + gr);
+                    lc[r] = coherent_load(pc + G * D + G + gr);
+                }
+#pragma unroll
+                for (int r = 0; r < RP; ++r) {
+                    const float mn = fmaxf(mm[r], wave_reduce(mc[r], [](float p, float q) { return fmaxf(p, q); }));
+                    a[r] = expf(mm[r] - mn);
+                    w[r] = have ? expf(mc[r] - mn) : 0.0f;
+                    ll[r] = ll[r] * a[r] + wave_reduce(have ? lc[r] * w[r] : 0.0f, [](float p, float q) { return p + q; });
+                    mm[r] = mn;
+                }
+                auto mine = [&](const float (&v)[RP]) {  // the value of this lane's row
+                    float y = v[0];
+#pragma unroll
+                    for (int r = 1; r < RP; ++r) y = rr == r ? v[r] : y;
+                    return y;
+                };
+                oo = oo * mine(a);
+                const int nc = nch - c0 < 64 ? nch - c0 : 64;
+#pragma unroll 1
+                for (int c = 0; c < nc; c += KB) {
+                    if (c0 + c > 0) load_batch(x, c0 + c);
+#pragma unroll
+                    for (int b = 0; b < KB; ++b) {
+                        float wc[RP];
+#pragma unroll
+                        for (int r = 0; r < RP; ++r) wc[r] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w[r]), (c + b) & 63));
+                        if (c + b < nc) oo = oo + x[b] * mine(wc);
+                    }
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < RP; ++r)
+                if (lane == 0 && g0 + r < G) {
+                    m[(g0 + r) * ms3] = mm[r];
+                    l[(g0 + r) * ls3] = ll[r];
+                }
+            if (g0 + rr < G) {
+                float lr = ll[0];
+#pragma unroll
+                for (int r = 1; r < RP; ++r) lr = rr == r ? ll[r] : lr;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int dim = part_dim<D>(p0 + e);
+                    o[g * os3 + dim * os4] = oo[e];
+                    if (out) out[g * us3 + dim * us4] = oo[e] / lr;
                 }
             }
         }

@@ -1251,11 +1251,12 @@ EmittedKernel emit_decode(const Module& m, const KernelAnalysis& a, const Launch
     // Values read from LDS are wave-uniform: readfirstlane keeps the page
     // loop's control and addresses in scalar registers.
     o << "  const i64 TC = __builtin_amdgcn_readfirstlane(cpre[U]);\n";
-    // Active waves: at most one per cost position, so that no wave's cost
-    // range is empty and a unit's partials fill consecutive slots (a wave
-    // whose range holds only cost positions, and no page, returns here).
-    o << "  const i64 W = (i64)gridDim.x * " << nw << " < TC ? (i64)gridDim.x * " << nw << " : TC, w = (i64)blockIdx.x * " << nw
-      << " + wave;\n";
+    // Active waves (a wave whose range holds only cost positions, and no
+    // page, returns here; a unit's partials fill consecutive slots).  When not
+    // all are active they are spread over the blocks.
+    o << "  const int AW = static_cast<int>(gridDim.x) * " << nw << ";\n";
+    o << "  const i64 W = DecodeSplit::waves_for(TC, U, AW);\n";
+    o << "  const i64 w = W < AW ? static_cast<int>(blockIdx.x + gridDim.x * wave) : static_cast<int>(blockIdx.x * " << nw << " + wave);\n";
     o << "  if (w < W) {\n";
     o << "  const i64 s = DecodeSplit::page_at(pre, cpre, U, w * TC / W);\n";
     o << "  const i64 b = DecodeSplit::page_at(pre, cpre, U, (w + 1) * TC / W);\n";
@@ -1324,7 +1325,9 @@ EmittedKernel emit_decode(const Module& m, const KernelAnalysis& a, const Launch
     o << "  auto f_slot = [&](int u) { return partials + ((i64)u + w) * DW::kPartFloats; };\n";
     // Folds unit u's partials (slots first .. first+parts-1, in page order)
     // into its accumulators.
-    o << "  auto f_combine = [&](int u, int parts, i64 first) {\n";
+    // f_many: the same for a unit of many partials.
+    for (const bool many : {false, true}) {
+    o << "  auto " << (many ? "f_many" : "f_combine") << " = [&](int u, int parts, i64 first) {\n";
     o << "    i64 vars[" << nvars << "];\n";
     decode_vars("u", "    ");
     o << "    vars[" << ng << "] = 0;\n";
@@ -1339,14 +1342,15 @@ EmittedKernel emit_decode(const Module& m, const KernelAnalysis& a, const Launch
     o << "    if (!bad_acc)\n";
     // Accumulators per lane of one combine pass: half as many with two waves
     // per SIMD (half the registers per wave).
-    o << "      DecodeCombine<" << d.g << ", " << d.d << ", " << (nw == 8 ? 8 : 16) << ">::run(parts, partials + first * DW::kPartFloats, DW::kPartFloats, "
+    o << "      DecodeCombine<" << d.g << ", " << d.d << ", " << (nw == 8 ? 8 : 16) << ">::" << (many ? "run_many" : "run") << "(parts, partials + first * DW::kPartFloats, DW::kPartFloats, "
       << ptr(d.m, "float*", 4) << ", A.s3[" << d.m << "], " << ptr(d.l, "float*", 4) << ", A.s3[" << d.l << "], "
       << ptr(d.o, "float*", 4) << ", A.s3[" << d.o << "], A.s4[" << d.o << "], "
       << (spec.decode_norm ? "out_, A.s3[" + std::to_string(ntens + 1) + "], A.s4[" + std::to_string(ntens + 1) + "]"
                            : std::string("nullptr, 0, 0"))
       << ");\n";
     o << "  };\n";
-    o << "  auto fns = decode_fns(f_page, f_bases, f_q, f_slot, f_combine);\n";
+    }
+    o << "  auto fns = decode_fns(f_page, f_bases, f_q, f_slot, f_combine, f_many);\n";
     o << "  DecodeStream<DW, " << spec.decode_ring << ", " << (spec.decode_ordered ? "true" : "false") << ">::run(fns, pre, cpre, U, TC, W, w, s, b, cnt, " << scale.str() << ", A.s4[" << d.kt
       << "], A.s3[" << d.v << "], A.s3[" << d.q << "]);\n";
     o << "  }\n";

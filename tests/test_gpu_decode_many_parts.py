@@ -1,0 +1,64 @@
+"""Paged decode with few units over all the waves: each unit is split into many partials, which
+one wave folds after its stream (DecodeCombine::run_many, DecodeSplit::waves_for).
+
+Against float64 attention.  A page's scores and p @ v carry about 2^-17 relative for 16-bit pages
+(p enters as two 16-bit parts) and 2^-24 for f32, and the fold of n partials adds a rounding per
+partial, so the decode tests' bound of 1e-5 relative Frobenius holds whatever the split."""
+
+import numpy as np
+import pytest
+
+import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("lengths,hkv,G,D,page,kind", [
+    ([2100], 1, 1, 128, 16, "bf16"),          # one row: the lanes past it fold it again
+    ([3000, 17], 1, 3, 64, 32, "f16"),        # four rows per pass, three used; a unit of one partial beside it
+    ([4000], 2, 4, 128, 16, "bf16"),          # two passes of two rows
+    ([1500, 0, 900], 1, 7, 64, 8, "bf16"),    # two passes of four, the last one short; an empty unit
+    ([2500], 1, 16, 256, 16, "f16"),          # one row per pass
+    ([1800], 2, 20, 128, 32, "bf16"),         # more than 16 rows
+    ([1700], 1, 5, 64, 16, "f32"),
+    ([1025], 1, 16, 128, 16, "f32"),          # a square score tile, unmasked
+    ([90000], 1, 2, 64, 64, "bf16"),          # more than 64 partials: two rounds of weights
+    ([16 * 8 + 3] * 3, 1, 4, 128, 16, "bf16"),  # about as many partials as the limit between the two folds
+])
+def test_many_partials(gpu, lengths, hkv, G, D, page, kind):
+    import torch
+
+    a = W.paged_decode_arrays(lengths, hkv, G, D, page, seed=len(lengths) + G, f16=kind == "f16", f32=kind == "f32")
+    dt = {"bf16": W.BF16, "f16": W.F16, "f32": W.F32}[kind]
+
+    def dev(x):
+        if x.dtype == np.uint16:
+            return torch.from_numpy(x.view(np.int16)).to(gpu).view(torch.bfloat16)
+        return torch.from_numpy(x).to(gpu)
+
+    t = {k: dev(v) for k, v in a.items() if k != "lengths"}
+    masked = not (G == page)  # a square score tile reads the mask by rows
+    wl = W.rr4(W.paged_decode(t, masked=masked, dtype=dt))
+    prog = wl.compile(target="hip_gfx950")
+    assert prog._native.kernel_family("decode_page") == "decode"
+    for _ in range(3):  # the counters return to zero; the accumulators start afresh
+        t["m"].fill_(float("-inf"))
+        t["l"].zero_()
+        t["o"].zero_()
+        prog.execute()
+        prog.synchronize()
+    ref = W.paged_decode_ref(a) if masked else _ref_all_tokens(a)
+    got = t["out"].cpu().numpy()
+    live = np.asarray(lengths) > 0
+    assert np.isfinite(got[live]).all()
+    assert np.linalg.norm(got[live] - ref[live]) <= 1e-5 * np.linalg.norm(ref[live])
+    o, l = t["o"].cpu().numpy(), t["l"].cpu().numpy()
+    np.testing.assert_array_equal(got[live], (o / l)[live])
+
+
+def _ref_all_tokens(a):
+    """Without a mask the last page's padding tokens take part."""
+    b = dict(a)
+    page = a["k_cache"].shape[2]
+    b["lengths"] = ((a["lengths"] + page - 1) // page) * page
+    return W.paged_decode_ref(b)
