@@ -456,9 +456,8 @@ __device__ inline void tsort32_rank(float* dst, const float* sc, const i64* ix) 
 // (bf16 or f16) on MFMA v_mfma_f32_32x32x16
 // ---------------------------------------------------------------------------
 //
-// A workgroup of WM x WN waves owns a BM x BN block of C (one task's tile, or
-// several neighbouring tasks' tiles merged by the host).  Wave (wm, wn) holds
-// its (BM/WM) x (BN/WN) quadrant in registers as 32x32 MFMA blocks for the
+// A workgroup of WM x WN waves owns a BM x BN block of C, cut by the host
+// regardless of the task tiles.  Wave (wm, wn) holds its (BM/WM) x (BN/WN) quadrant in registers as 32x32 MFMA blocks for the
 // whole K loop; for an accumulating kernel the block starts from C.
 //
 // K steps go through two LDS stages filled by direct buffer->LDS loads (each
@@ -546,6 +545,14 @@ __device__ inline void wait_vmcnt() {
     __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
 }
 
+// Waits for this wave's stores (see the coherence notes at the decode
+// partials, which coherent_store introduces).
+__device__ inline void publish() {
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    wait_vmcnt<0>();
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+}
+
 // Position of workgroup w among n workgroups dispatched round-robin over the
 // 8 XCDs, so that each XCD (own L2) gets a contiguous run of tiles.
 __device__ inline i64 xcd_order(i64 w, i64 n) {
@@ -553,9 +560,29 @@ __device__ inline i64 xcd_order(i64 w, i64 n) {
     return x * q + (x < r ? x : r) + l;
 }
 
-// NS: LDS stages in the ring (DMA issued NS-1 stages ahead); KSPLIT: LDS
-// stages per task K step (a stage holds BK of the task's BK*KSPLIT columns).
-template <int BM, int BN, int BK, int WM, int WN, bool F16, int NS = 2, int KSPLIT = 1>
+// Where a block's sum goes besides its C block.  EDGE blocks hold only the
+// first `rows` rows and `cols` columns of their C block (the last ones along
+// M and N); their loads are clamped into the operands and what lies outside
+// is not stored.  SPLIT blocks sum part `s` of `ns` of the K range of tile
+// `tile`: each writes its partial block, and the last to arrive adds the
+// tile's partials in order and finishes C.
+struct GemmOut {
+    int rows, cols;
+    float* part;
+    int* cnt;
+    int tile, s, ns;
+};
+
+// The stages of part s of ns of [st0, st1).
+__device__ inline void gemm_split_range(i64& st0, i64& st1, int s, int ns) {
+    const u32 n = static_cast<u32>(st1 - st0), u = static_cast<u32>(s), d = static_cast<u32>(ns);
+    const i64 b = st0;
+    st0 = b + n / d * u + (n % d) * u / d;
+    st1 = b + n / d * (u + 1) + (n % d) * (u + 1) / d;
+}
+
+// NS: LDS stages in the ring (DMA issued NS-1 stages ahead).
+template <int BM, int BN, int BK, int WM, int WN, bool F16, int NS = 2>
 struct GemmBlock {
     static constexpr int NW = WM * WN, NT = 64 * NW, KS = BK / 16;
     static constexpr int TM = BM / WM, TN = BN / WN, FI = TM / 32, FJ = TN / 32;
@@ -586,19 +613,23 @@ struct GemmBlock {
     __device__ static int swb(int k) { return BN >= 128 ? (k & 3) << 1 : k & 3; }
 
     // Per-lane byte offsets, from the block's A / B origin at the first K step,
-    // of the chunks this wave moves (lda / ldb: row pitch in elements).
-    __device__ static void offsets(Offs& o, int lda, int ldb) {
+    // of the chunks this wave moves (lda / ldb: row pitch in elements).  EDGE:
+    // rows past the last one read it again, chunks past the last column (a
+    // multiple of 16) read the first one.
+    template <bool EDGE>
+    __device__ static void offsets(Offs& o, int lda, int ldb, const GemmOut& g) {
         const int lane = threadIdx.x & 63, w = wave_index();
 #pragma unroll
         for (int q = 0; q < AQ; ++q) {
             const int m = (w * AQ + q) * ARPB + lane / CH, p = lane % CH;
-            o.a[q] = (m * lda + ((p ^ swa(m)) << 3)) * 2;
+            const int mr = EDGE && m >= g.rows ? g.rows - 1 : m;
+            o.a[q] = (mr * lda + ((p ^ swa(m)) << 3)) * 2;
         }
 #pragma unroll
         for (int q = 0; q < BQ; ++q) {
             const int k = (w * BQ + q) * BRPB + lane / BCPR, p = lane % BCPR;
             const int c = (((p >> 1) ^ swb(k)) << 1) | (p & 1);
-            o.b[q] = (k * ldb + c * 8) * 2;
+            o.b[q] = (k * ldb + (EDGE && c * 8 >= g.cols ? 0 : c * 8)) * 2;
         }
     }
 
@@ -645,44 +676,27 @@ struct GemmBlock {
         }
     }
 
-    // C block I/O in the accumulator layout (ldc: row pitch in elements).
-    template <bool STORE>
-    __device__ static void c_io(Acc& acc, buf_rsrc rc, int ldc) {
-        const int lane = threadIdx.x & 63, wave = wave_index();
-        const int wm = wave / WN, wn = wave % WN;
-        const int vc = ((lane >> 5) * 4 * ldc + (lane & 31)) * 4;
-        const int so = (wm * TM * ldc + wn * TN) * 4;
-#pragma unroll
-        for (int i = 0; i < FI; ++i)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int s = so + (i * 32 + (e >> 2) * 8 + (e & 3)) * ldc * 4;
-#pragma unroll
-                for (int j = 0; j < FJ; ++j) {
-                    if constexpr (STORE)
-                        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc.v[i][j][e]), rc, vc + j * 128, s, 2);
-                    else
-                        acc.v[i][j][e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rc, vc + j * 128, s, 2));
-                }
-            }
-    }
-
     // Writes the block (plus C when ADD_C) in the accumulator layout, one
     // 32x32 accumulator at a time: the next accumulator's C is read while
     // this one is added and stored, and scheduling barriers keep the
     // accumulators apart so that few values sit in VGPRs at once.
-    template <bool ADD_C>
-    __device__ static void c_out(Acc& acc, buf_rsrc rc, int ldc) {
+    template <bool ADD_C, bool EDGE>
+    __device__ static void c_out(Acc& acc, buf_rsrc rc, int ldc, const GemmOut& g) {
         const int lane = threadIdx.x & 63, wave = wave_index();
         const int wm = wave / WN, wn = wave % WN;
+        const int r0 = wm * TM + (lane >> 5) * 4, c0 = wn * TN + (lane & 31);
         const int vc = ((lane >> 5) * 4 * ldc + (lane & 31)) * 4;
         const int so = (wm * TM * ldc + wn * TN) * 4;
         auto row = [&](int i, int e) { return so + (i * 32 + (e >> 2) * 8 + (e & 3)) * ldc * 4; };
+        auto in = [&](int i, int j, int e) {
+            return !EDGE || (r0 + i * 32 + (e >> 2) * 8 + (e & 3) < g.rows && c0 + j * 32 < g.cols);
+        };
         float t[2][16];
         auto fetch = [&](int n, float (&d)[16]) {
             const int i = n / FJ, j = n % FJ;
 #pragma unroll
-            for (int e = 0; e < 16; ++e) d[e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rc, vc + j * 128, row(i, e), 2));
+            for (int e = 0; e < 16; ++e)
+                if (in(i, j, e)) d[e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rc, vc + j * 128, row(i, e), 2));
         };
         if constexpr (ADD_C) fetch(0, t[0]);
 #pragma unroll
@@ -694,10 +708,66 @@ struct GemmBlock {
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
                 const float x = ADD_C ? t[n & 1][e] + acc.v[i][j][e] : acc.v[i][j][e];
-                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x), rc, vc + j * 128, row(i, e), 2);
+                if (in(i, j, e)) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x), rc, vc + j * 128, row(i, e), 2);
             }
             __builtin_amdgcn_sched_barrier(0);
         }
+    }
+
+    // SPLIT: writes this block's partial (128 bits per lane, one accumulator
+    // quarter of 1 KiB per instruction) and counts it; true in the last block
+    // of the tile to arrive, whose acc then holds the sum of the tile's
+    // partials in K order.  The partials are agent-coherent (sc1) stores,
+    // complete (vmcnt 0) in every wave before the workgroup barrier that
+    // precedes the count, and agent-coherent loads behind the count's value:
+    // the ordering of the decode partials (publish).
+    __device__ static bool reduce_split(Acc& acc, u16* lds, const GemmOut& g) {
+        const int lane = threadIdx.x & 63, wave = wave_index();
+        float* tile = g.part + static_cast<i64>(g.tile) * g.ns * (BM * BN);
+        const buf_rsrc rp = __builtin_amdgcn_make_buffer_rsrc(tile, 0, -1, 0x00020000);
+        auto at = [&](int n, int q) { return ((wave * FI * FJ + n) * 4 + q) * 1024 + lane * 16; };
+#pragma unroll
+        for (int n = 0; n < FI * FJ; ++n)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const f32x16& v = acc.v[n / FJ][n % FJ];
+                const u32x4 x = {__float_as_uint(v[4 * q]), __float_as_uint(v[4 * q + 1]), __float_as_uint(v[4 * q + 2]),
+                                 __float_as_uint(v[4 * q + 3])};
+                __builtin_amdgcn_raw_buffer_store_b128(x, rp, at(n, q), g.s * (BM * BN * 4), 16);
+            }
+        publish();
+        __syncthreads();
+        int* last = reinterpret_cast<int*>(lds);
+        if (threadIdx.x == 0) {
+            const int old = __hip_atomic_fetch_add(g.cnt + g.tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            *last = old == g.ns - 1;
+        }
+        __syncthreads();
+        if (!*last) return false;
+        if (threadIdx.x == 0) __hip_atomic_store(g.cnt + g.tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        constexpr int SB = FI * FJ >= 8 ? 1 : 4;  // partials read together
+#pragma unroll
+        for (int n = 0; n < FI * FJ; ++n) {
+            f32x16 sum = {};
+            for (int s0 = 0; s0 < g.ns; s0 += SB) {
+                u32x4 x[SB][4];
+#pragma unroll
+                for (int b = 0; b < SB; ++b)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        x[b][q] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                                rp, at(n, q), (s0 + b < g.ns ? s0 + b : g.ns - 1) * (BM * BN * 4), 16));
+#pragma unroll
+                for (int b = 0; b < SB; ++b)
+                    if (s0 + b < g.ns) {
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) sum[e] = sum[e] + __uint_as_float(x[b][e >> 2][e & 3]);
+                    }
+            }
+            acc.v[n / FJ][n % FJ] = sum;
+        }
+        return true;
     }
 
     // Waits until at most `ahead` stages of this wave's DMA are in flight.
@@ -711,30 +781,28 @@ struct GemmBlock {
         }
     }
 
-    // Task K steps it0 .. iters-1, as (iters-it0)*KSPLIT LDS stages; off(it,
-    // soa, sob) gives task step it's byte offsets from the step-0 origins pa /
-    // pb.  The block sums A x B from zero; ACC: then adds C, as c + sum.
-    template <bool ACC, class Off>
-    __device__ static void run(u16* lds, const u16* pa, int lda, const u16* pb, int ldb, float* pc, int ldc, i64 it0,
-                               i64 iters, Off off) {
+    // K stages st0 .. st1-1; off(st, soa, sob) gives stage st's byte offsets
+    // from the stage-0 origins pa / pb.  The block sums A x B from zero; ACC:
+    // then adds C, as c + sum.
+    template <bool ACC, bool EDGE, bool SPLIT, class Off>
+    __device__ static void run(u16* lds, const u16* pa, int lda, const u16* pb, int ldb, float* pc, int ldc, i64 st0, i64 st1,
+                               Off off, const GemmOut& g) {
         const u32x4 ra = buffer_words(pa), rb = buffer_words(pb);
         const buf_rsrc rc = __builtin_amdgcn_make_buffer_rsrc(pc, 0, -1, 0x00020000);
+        if constexpr (SPLIT) gemm_split_range(st0, st1, g.s, g.ns);
         Offs o;
-        offsets(o, lda, ldb);
+        offsets<EDGE>(o, lda, ldb, g);
         Acc acc;
 #pragma unroll
         for (int i = 0; i < FI; ++i)
 #pragma unroll
             for (int j = 0; j < FJ; ++j) acc.v[i][j] = f32x16{};
-        const i64 nst = (iters - it0) * KSPLIT;
+        const i64 nst = st1 - st0;
         auto issue = [&](i64 st) {
             int soa, sob;
-            off(it0 + st / KSPLIT, soa, sob);
-            const int h = static_cast<int>(st % KSPLIT);
-            load(lds + static_cast<int>(st & (NS - 1)) * STAGE, o, ra, soa + h * BK * 2, rb, sob + h * BK * ldb * 2);
+            off(st0 + st, soa, sob);
+            load(lds + static_cast<int>(st & (NS - 1)) * STAGE, o, ra, soa, rb, sob);
         };
-        wait_vmcnt<0>();
-        __syncthreads();  // the previous block's last stage reads are done
 #pragma unroll
         for (int p = 0; p < NS - 1; ++p)
             if (p < nst) issue(p);
@@ -745,7 +813,9 @@ struct GemmBlock {
             if (st + NS - 1 < nst) issue(st + NS - 1);
             mma(acc, lds + static_cast<int>(st & (NS - 1)) * STAGE);
         }
-        c_out<ACC>(acc, rc, ldc);
+        if constexpr (SPLIT)
+            if (!reduce_split(acc, lds, g)) return;
+        c_out<ACC, EDGE>(acc, rc, ldc, g);
     }
 };
 
@@ -767,7 +837,7 @@ struct GemmBlock {
 // a product is free, so for the 8 columns kk..kk+7 half-wave h reads
 // A[m][kk+4h .. +3] as one 16-byte chunk, and MFMA q (0..3) pairs column
 // kk+q (half 0) with kk+4+q (half 1).
-template <int BM, int BN, int BK, int WM, int WN, int NS = 2, int KSPLIT = 1>
+template <int BM, int BN, int BK, int WM, int WN, int NS = 2>
 struct GemmF32 {
     static constexpr int NW = WM * WN, NT = 64 * NW;
     static constexpr int TM = BM / WM, TN = BN / WN, FI = TM / 32, FJ = TN / 32;
@@ -781,7 +851,8 @@ struct GemmF32 {
     static constexpr int AQ = (ABLK + NW - 1) / NW, BQ = (BBLK + NW - 1) / NW;
     static constexpr int ASZ = BM * BK, STAGE = ASZ + BK * BN;  // floats
     static constexpr int kLdsElems = NS * STAGE * 2;            // 16-bit units (the kernel's LDS array)
-    static_assert(NS == 2, "two-stage ring");
+    static constexpr int kStageOps = AQ + BQ;  // DMA instructions of one wave per stage
+    static_assert(NS == 2 || (NS == 4 && AQ * NW == ABLK && BQ * NW == BBLK), "stage ring: every wave moves the same share");
     static_assert(TM % 32 == 0 && TN % 32 == 0 && (BK == 16 || BK == 32), "f32 GEMM block shape");
     static_assert(BN >= 64 && BN <= 256 && (BM * BK * 4) % 1024 == 0 && (BK * BN * 4) % 1024 == 0, "f32 GEMM block shape");
     typedef GemmBlock<BM, BN, 16, WM, WN, false> Out;  // the C epilogue (same accumulator layout)
@@ -795,18 +866,21 @@ struct GemmF32 {
     __device__ static int swb(int k) { return ((k >> 2) & 1) << 3; }
 
     // Per-lane byte offsets, from the block's A / B origin at the first K
-    // step, of the chunks this wave moves (lda / ldb: row pitch in elements).
-    __device__ static void offsets(Offs& o, int lda, int ldb) {
+    // step, of the chunks this wave moves (lda / ldb: row pitch in elements;
+    // EDGE as in GemmBlock).
+    template <bool EDGE>
+    __device__ static void offsets(Offs& o, int lda, int ldb, const GemmOut& g) {
         const int lane = threadIdx.x & 63, w = wave_index();
 #pragma unroll
         for (int q = 0; q < AQ; ++q) {
             const int m = (w * AQ + q) * ARPB + lane / CH, p = lane % CH;
-            o.a[q] = (m * lda + ((p ^ swa(m)) << 2)) * 4;
+            const int mr = EDGE && m >= g.rows ? g.rows - 1 : m;
+            o.a[q] = (mr * lda + ((p ^ swa(m)) << 2)) * 4;
         }
 #pragma unroll
         for (int q = 0; q < BQ; ++q) {
-            const int k = (w * BQ + q) * BRPB + lane / BCPR, p = lane % BCPR;
-            o.b[q] = (k * ldb + ((p ^ swb(k)) << 2)) * 4;
+            const int k = (w * BQ + q) * BRPB + lane / BCPR, p = lane % BCPR, c = (p ^ swb(k)) << 2;
+            o.b[q] = (k * ldb + (EDGE && c >= g.cols ? 0 : c)) * 4;
         }
     }
 
@@ -850,38 +924,46 @@ struct GemmF32 {
         }
     }
 
-    // Task K steps it0 .. iters-1, as (iters-it0)*KSPLIT LDS stages (see
-    // GemmBlock::run); pa / pb point at f32 data.
-    template <bool ACC, class Off>
-    __device__ static void run(u16* lds, const u16* pa, int lda, const u16* pb, int ldb, float* pc, int ldc, i64 it0,
-                               i64 iters, Off off) {
+    // K stages st0 .. st1-1 (see GemmBlock::run); pa / pb point at f32 data.
+    template <bool ACC, bool EDGE, bool SPLIT, class Off>
+    __device__ static void run(u16* lds, const u16* pa, int lda, const u16* pb, int ldb, float* pc, int ldc, i64 st0, i64 st1,
+                               Off off, const GemmOut& g) {
         float* ring = reinterpret_cast<float*>(lds);
         const u32x4 ra = buffer_words(pa), rb = buffer_words(pb);
         const buf_rsrc rc = __builtin_amdgcn_make_buffer_rsrc(pc, 0, -1, 0x00020000);
+        if constexpr (SPLIT) gemm_split_range(st0, st1, g.s, g.ns);
         Offs o;
-        offsets(o, lda, ldb);
+        offsets<EDGE>(o, lda, ldb, g);
         Acc acc;
 #pragma unroll
         for (int i = 0; i < FI; ++i)
 #pragma unroll
             for (int j = 0; j < FJ; ++j) acc.v[i][j] = f32x16{};
-        const i64 nst = (iters - it0) * KSPLIT;
+        const i64 nst = st1 - st0;
         auto issue = [&](i64 st) {
             int soa, sob;
-            off(it0 + st / KSPLIT, soa, sob);
-            const int hs = static_cast<int>(st % KSPLIT);
-            load(ring + static_cast<int>(st & 1) * STAGE, o, ra, soa + hs * BK * 4, rb, sob + hs * BK * ldb * 4);
+            off(st0 + st, soa, sob);
+            load(ring + static_cast<int>(st & (NS - 1)) * STAGE, o, ra, soa, rb, sob);
         };
-        wait_vmcnt<0>();
-        __syncthreads();  // the previous block's last stage reads are done
-        if (nst > 0) issue(0);
+#pragma unroll
+        for (int p = 0; p < NS - 1; ++p)
+            if (p < nst) issue(p);
         for (i64 st = 0; st < nst; ++st) {
-            wait_vmcnt<0>();
+            const i64 ahead = nst - 1 - st < NS - 2 ? nst - 1 - st : NS - 2;
+            if constexpr (NS == 2) {
+                wait_vmcnt<0>();
+            } else {
+                if (ahead >= 2) wait_vmcnt<2 * kStageOps>();
+                else if (ahead == 1) wait_vmcnt<kStageOps>();
+                else wait_vmcnt<0>();
+            }
             __syncthreads();
-            if (st + 1 < nst) issue(st + 1);
-            mma(acc, ring + static_cast<int>(st & 1) * STAGE);
+            if (st + NS - 1 < nst) issue(st + NS - 1);
+            mma(acc, ring + static_cast<int>(st & (NS - 1)) * STAGE);
         }
-        Out::template c_out<ACC>(acc, rc, ldc);
+        if constexpr (SPLIT)
+            if (!Out::reduce_split(acc, lds, g)) return;
+        Out::template c_out<ACC, EDGE>(acc, rc, ldc, g);
     }
 };
 
@@ -1011,7 +1093,7 @@ __device__ inline void dma4(u32x4 rsrc, int voff, int soff, u32 lds_addr) {
 
 template <int BK, bool F16>
 struct GemmPingPong {
-    typedef GemmBlock<256, 256, BK, 2, 4, F16, 2, 1> GB;
+    typedef GemmBlock<256, 256, BK, 2, 4, F16, 2> GB;
     static constexpr int NS = BK == 64 ? 2 : 4;        // LDS stages (128 KiB)
     static constexpr int PF = 3;                       // L2 touch distance in stages
     static constexpr int WN = 4, TM = 128, TN = 64, FI = 4, FJ = 2, KS = BK / 16;
@@ -1314,7 +1396,7 @@ struct GemmPingPong {
         if (grp == 0) block_barrier();
     }
 
-    // Task K steps it0 .. iters-1 (off(it, soa, sob): step it's byte offsets
+    // K stages it0 .. iters-1 (off(it, soa, sob): stage it's byte offsets
     // from the step-0 origins pa / pb).  The block sums A x B from zero; ACC:
     // then adds C, as c + sum.  pfa_row / pfb_row (< 0: no L2 touches): the
     // A rows pfa_row..+31 and B rows pfb_row..+15 of each stage that wave 0
@@ -1438,11 +1520,6 @@ __device__ inline float cross4_reduce(float x, Op op) {
 __device__ inline void coherent_store(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ inline float coherent_load(const float* p) {
     return __hip_atomic_load(const_cast<float*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ inline void publish() {
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);
-    wait_vmcnt<0>();
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);
 }
 // The wave that brings a unit's completion count to `parts` folds the unit
 // and sets the count back to zero for the next launch.

@@ -969,129 +969,132 @@ EmittedKernel emit_gemm(const Module& m, const KernelAnalysis& a, const LaunchSp
     const GemmInfo& g = a.gemm;
     const int ng = static_cast<int>(L.grid.size()), ni = static_cast<int>(L.inner.size());
     const int nvars = ng + ni;
-    const int fm = spec.gemm_vm >= 0 ? spec.gemm_fm : 1, fn = spec.gemm_vn >= 0 ? spec.gemm_fn : 1;
-    // Task tiles above 256 rows / columns run as sm x sn blocks of 256.
-    const int sm = g.m > 256 ? g.m / 256 : 1, sn = g.n > 256 ? g.n / 256 : 1;
-    const int bm = gemm_block_dim(g.m) * fm, bn = gemm_block_dim(g.n) * fn;
+    const int bm = spec.gemm_bm, bn = spec.gemm_bn;
     // One LDS stage per kf task K steps (kf consecutive steps are adjacent
-    // columns of A and rows of B), two stages (a 4-stage ring of 32-wide
-    // stages measured slower on 256x256 blocks: twice the barriers).
-    const int wm = gemm_waves_m(), wn = gemm_waves_n(bn);
+    // columns of A and rows of B), in a ring of ns stages (a 4-stage ring of
+    // 32-wide stages measured slower on 256x256 blocks: twice the barriers).
+    const int wm = gemm_waves_m(bm), wn = gemm_waves_n(bm, bn);
     const int kf = ni == 1 ? spec.gemm_kf : 1, kstep = g.k * kf;
-    // f32 A / B: stages of at most 32 K columns (GemmF32), a K step split
-    // over ksplit stages; element size es bytes.
-    const int bk = gemm_stage_k(kstep, g.f32), ns = 2, es = g.f32 ? 4 : 2;
-    // Stages per K step: GemmF32 takes them as its KSPLIT; the bf16 / f16
-    // blocks see each stage as one step of a stage-level offset function
-    // (sks stages per task step).
-    const int ksplit = g.f32 ? kstep / bk : 1, sks = g.f32 ? 1 : kstep / bk;
+    // f32 A / B: stages of at most 32 K columns (GemmF32); element size es
+    // bytes.  A K step of several stages: sks stages per task step.
+    const int bk = gemm_stage_k(kstep, g.f32), ns = spec.gemm_ring, es = g.f32 ? 4 : 2;
+    const int sks = kstep / bk;
     // Ping-pong block: 256x256, K step 32 / 64, row pitches checked on the host.
     const bool pp = !g.f32 && spec.gemm_pingpong && bm == 256 && bn == 256 && (bk == 64 || bk == 32);
+    const bool split = spec.gemm_split > 1;
     EmittedKernel ek;
     ek.threads = 64 * wm * wn;
     ek.row_program = false;
-    ek.tasks_per_block = fm * fn;
-    ek.blocks_per_task = sm * sn;
     std::ostringstream o;
     o << "#include \"ptowsp_device.h\"\nusing namespace ptowsp;\n";
     o << "// gemm program: kernel " << k.name << ", task tile " << g.m << "x" << g.n << "x" << g.k
       << (g.f32 ? " f32" : g.f16 ? " f16" : " bf16")
-      << (g.accumulate ? ", accumulate" : "") << "; block " << bm << "x" << bn << " (" << fm * fn << " tasks)"
-      << (kf > 1 ? "; " + std::to_string(kf) + " K steps per stage" : "")
-      << (pp ? ", ping-pong" : "") << "\n";
+      << (g.accumulate ? ", accumulate" : "") << "; block " << bm << "x" << bn
+      << (kf > 1 ? "; " + std::to_string(kf) + " K steps per stage" : "") << (spec.gemm_edge ? "; edges" : "")
+      << (split ? "; K in " + std::to_string(spec.gemm_split) + " parts" : "") << (pp ? ", ping-pong" : "") << "\n";
     ek.entry = entry_name("gemm", k);
     o << "extern \"C\" __global__ void __launch_bounds__(" << ek.threads << ") "
       << ek.entry << "(const LaunchArgs A) {\n";
     if (pp)
         o << "  typedef GemmPingPong<" << bk << ", " << (g.f16 ? "true" : "false") << "> GB;\n";
     else if (g.f32)
-        o << "  typedef GemmF32<" << bm << ", " << bn << ", " << bk << ", " << wm << ", " << wn << ", " << ns << ", " << ksplit
-          << "> GB;\n";
+        o << "  typedef GemmF32<" << bm << ", " << bn << ", " << bk << ", " << wm << ", " << wn << ", " << ns << "> GB;\n";
     else
         o << "  typedef GemmBlock<" << bm << ", " << bn << ", " << bk << ", " << wm << ", " << wn << ", "
-          << (g.f16 ? "true" : "false") << ", " << ns << ", " << ksplit << "> GB;\n";
+          << (g.f16 ? "true" : "false") << ", " << ns << "> GB;\n";
     o << "  __shared__ __attribute__((aligned(1024))) u16 lds[GB::kLdsElems];\n";
     o << "  i64 vars[" << (nvars > 0 ? nvars : 1) << "];\n  (void)vars;\n";
-    // One workgroup per block (the host launches every block): nothing of
-    // the launch arguments stays live through the K loop.
-    o << "  const i64 nblk = A.ntasks / " << fm * fn << " * " << sm * sn << ";\n";
-    o << "  {\n    const i64 w = blockIdx.x;\n    if (w >= nblk) return;\n";
-    o << "    i64 q_ = xcd_order(w, nblk);\n";
-    if (sm * sn > 1) {
-        // The block's 256 x 256 sub-tile of its task.
-        o << "    const i64 sn_ = q_ % " << sn << "; q_ /= " << sn << ";\n";
-        o << "    const i64 sm_ = q_ % " << sm << "; q_ /= " << sm << ";\n";
-    }
-    // Decode the block index over the grid with the merged extents divided.
+    // One workgroup per block (the host launches every block, fewer than
+    // 2^31): nothing of the launch arguments stays live through the K loop.
+    // C is rows_ x cols_ per problem: the task tile, extended over the grid
+    // variable whose tasks continue it downwards (gemm_vm) and to the right
+    // (gemm_vn); the other grid variables number the problems.
+    const int vm = spec.gemm_vm, vn = spec.gemm_vn;
+    auto extent = [&](int t, int v) {
+        return v >= 0 ? std::to_string(t) + "u * static_cast<u32>(A.ext[" + std::to_string(v) + "])" : std::to_string(t) + "u";
+    };
+    o << "  const u32 rows_ = " << extent(g.m, vm) << ", cols_ = " << extent(g.n, vn) << ";\n";
+    o << "  const u32 mb_ = (rows_ + " << bm - 1 << "u) / " << bm << "u, nb_ = (cols_ + " << bn - 1 << "u) / " << bn << "u;\n";
+    o << "  u32 q_ = static_cast<u32>(xcd_order(blockIdx.x, gridDim.x));\n";
+    if (split) o << "  const u32 sp_ = q_ % " << spec.gemm_split << "u; q_ /= " << spec.gemm_split << "u;\n  const u32 tile_ = q_;\n";
+    o << "  const u32 n_ = q_ % nb_; q_ /= nb_;\n  const u32 m_ = q_ % mb_; q_ /= mb_;\n";
     for (int v = ng - 1; v >= 0; --v) {
-        const int f = v == spec.gemm_vm ? fm : (v == spec.gemm_vn ? fn : 1);
-        const std::string ext = f > 1 ? "(A.ext[" + std::to_string(v) + "] / " + std::to_string(f) + ")" : "A.ext[" + std::to_string(v) + "]";
-        if (v > 0) o << "    vars[" << v << "] = q_ % " << ext << "; q_ /= " << ext << ";\n";
-        else o << "    vars[0] = q_;\n";
-        if (f > 1) o << "    vars[" << v << "] *= " << f << ";\n";
+        if (v == vm || v == vn) {
+            o << "  vars[" << v << "] = 0;\n";
+            continue;
+        }
+        o << "  { const u32 e_ = static_cast<u32>(A.ext[" << v << "]); vars[" << v << "] = q_ % e_; q_ /= e_; }\n";
     }
-    o << "    i64 iters = 1;\n";
-    for (int i = 0; i < ni; ++i) o << "    iters *= A.ext[" << ng + i << "];\n";
+    o << "  i64 iters = 1;\n";
+    for (int i = 0; i < ni; ++i) o << "  iters *= A.ext[" << ng + i << "];\n";
     // Merged K steps: iterations count stages of kf task steps (the host has
     // checked that kf divides the loop).
-    if (kf > 1) o << "    iters /= " << kf << ";\n";
-    o << "    if (iters <= 0) return;\n";
-    for (int i = 0; i < ni; ++i) o << "    vars[" << ng + i << "] = 0;\n";
-    o << "    const u16* pa = reinterpret_cast<const u16*>(A.base[" << g.a << "] + (" << offset_expr(g.a, nvars, 0, 0) << ") * " << es
-      << ");\n";
-    o << "    const u16* pb = reinterpret_cast<const u16*>(A.base[" << g.b << "] + (" << offset_expr(g.b, nvars, 0, 0) << ") * " << es
-      << ");\n";
+    if (kf > 1) o << "  iters /= " << kf << ";\n";
+    o << "  if (iters <= 0) return;\n";
+    for (int i = 0; i < ni; ++i) o << "  vars[" << ng + i << "] = 0;\n";
+    o << "  const u16* pa = reinterpret_cast<const u16*>(A.base[" << g.a << "] + (" << offset_expr(g.a, nvars, 0, 0) << " + (i64)(m_ * "
+      << bm << "u) * A.s3[" << g.a << "]) * " << es << ");\n";
+    o << "  const u16* pb = reinterpret_cast<const u16*>(A.base[" << g.b << "] + (" << offset_expr(g.b, nvars, 0, 0) << " + (i64)(n_ * "
+      << bn << "u)) * " << es << ");\n";
     // The output view does not move with the in-kernel loops (checked on the host).
-    o << "    float* pc = reinterpret_cast<float*>(A.base[" << g.c << "] + (" << offset_expr(g.c, nvars, 0, 0) << ") * 4);\n";
-    if (sm * sn > 1) {
-        o << "    pa = reinterpret_cast<const u16*>(reinterpret_cast<const char*>(pa) + sm_ * 256 * A.s3[" << g.a << "] * " << es << ");\n";
-        o << "    pb = reinterpret_cast<const u16*>(reinterpret_cast<const char*>(pb) + sn_ * 256 * " << es << ");\n";
-        o << "    pc += sm_ * 256 * A.s3[" << g.c << "] + sn_ * 256;\n";
-    }
+    o << "  float* pc = reinterpret_cast<float*>(A.base[" << g.c << "] + (" << offset_expr(g.c, nvars, 0, 0) << " + (i64)(m_ * " << bm
+      << "u) * A.s3[" << g.c << "] + (i64)(n_ * " << bn << "u)) * 4);\n";
     // Byte offsets of in-kernel iteration `it` from iteration 0 (mixed radix over the inner loops).
     if (ni == 1) {
         // One in-kernel loop: 32-bit byte steps (the host bounds every
         // offset below 2^31).
-        o << "    const int da_ = static_cast<int>(A.coef[" << g.a << "][" << ng << "] * " << es * kf << "), db_ = static_cast<int>(A.coef["
+        o << "  const int da_ = static_cast<int>(A.coef[" << g.a << "][" << ng << "] * " << es * kf << "), db_ = static_cast<int>(A.coef["
           << g.b << "][" << ng << "] * " << es * kf << ");\n";
-        o << "    auto off = [=](i64 it, int& soa, int& sob) { soa = static_cast<int>(it) * da_; sob = static_cast<int>(it) * db_; };\n";
+        o << "  auto off = [=](i64 it, int& soa, int& sob) { soa = static_cast<int>(it) * da_; sob = static_cast<int>(it) * db_; };\n";
     } else {
-        o << "    auto off = [&](i64 it, int& soa, int& sob) {\n";
-        o << "      i64 oa = 0, ob = 0;\n";
+        o << "  auto off = [&](i64 it, int& soa, int& sob) {\n";
+        o << "    i64 oa = 0, ob = 0;\n";
         for (int i = ni - 1; i >= 0; --i) {
             const int v = ng + i;
-            o << "      { const i64 x = it % A.ext[" << v << "]; it /= A.ext[" << v << "]; oa += A.coef[" << g.a << "][" << v
+            o << "    { const i64 x = it % A.ext[" << v << "]; it /= A.ext[" << v << "]; oa += A.coef[" << g.a << "][" << v
               << "] * x; ob += A.coef[" << g.b << "][" << v << "] * x; }\n";
         }
-        o << "      soa = static_cast<int>(oa * " << es << "); sob = static_cast<int>(ob * " << es << ");\n";
-        o << "    };\n";
+        o << "    soa = static_cast<int>(oa * " << es << "); sob = static_cast<int>(ob * " << es << ");\n";
+        o << "  };\n";
     }
     if (sks > 1) {
         // Stage st: task step st / sks, columns (st % sks) * BK of it.
-        o << "    const i64 ldb_ = A.s3[" << g.b << "];\n";
-        o << "    auto offs = [=](i64 st, int& soa, int& sob) {\n";
-        o << "      off(st / " << sks << ", soa, sob);\n";
-        o << "      const int h_ = static_cast<int>(st % " << sks << ");\n";
-        o << "      soa += h_ * " << bk * es << "; sob += h_ * static_cast<int>(ldb_) * " << bk * es << ";\n";
-        o << "    };\n";
+        o << "  const int ldb_ = static_cast<int>(A.s3[" << g.b << "]);\n";
+        o << "  auto offs = [=](i64 st, int& soa, int& sob) {\n";
+        o << "    off(static_cast<u32>(st) / " << sks << "u, soa, sob);\n";
+        o << "    const int h_ = static_cast<int>(static_cast<u32>(st) % " << sks << "u);\n";
+        o << "    soa += h_ * " << bk * es << "; sob += h_ * ldb_ * " << bk * es << ";\n";
+        o << "  };\n";
     }
+    const std::string its = sks > 1 ? "iters * " + std::to_string(sks) : "iters";
+    const std::string it0 = g.accumulate ? "0" : (sks > 1 ? "(iters - 1) * " + std::to_string(sks) : "iters - 1");
+    const std::string head = std::string(g.accumulate ? "true" : "false");
+    const std::string args = "(lds, pa, static_cast<int>(A.s3[" + std::to_string(g.a) + "]), pb, static_cast<int>(A.s3[" + std::to_string(g.b) +
+                             "]), pc, static_cast<int>(A.s3[" + std::to_string(g.c) + "]), " + it0 + ", " + its + ", " +
+                             (sks > 1 ? "offs" : "off");
     if (pp) {
         // L2 touches: the blocks that share an A panel (same m block) split its
         // rows by their n block (8 x 32 rows); those that share a B panel
         // split the stage's K rows by their m block (BK/16 x 16 rows).
-        if (spec.gemm_vm >= 0 && spec.gemm_vn >= 0)
-            o << "    const int pfa_row = static_cast<int>((vars[" << spec.gemm_vn << "] / " << fn << ") % 8) * 32;\n"
-              << "    const int pfb_row = static_cast<int>((vars[" << spec.gemm_vm << "] / " << fm << ") % " << bk / 16
-              << ") * 16;\n";
+        if (vm >= 0 && vn >= 0)
+            o << "  const int pfa_row = static_cast<int>(n_ % 8u) * 32, pfb_row = static_cast<int>(m_ % " << bk / 16 << "u) * 16;\n";
         else
-            o << "    const int pfa_row = -1, pfb_row = -1;\n";
+            o << "  const int pfa_row = -1, pfb_row = -1;\n";
+        o << "  GB::template run<" << head << ">" << args << ", pfa_row, pfb_row);\n";
+    } else {
+        const int nt = static_cast<int>(a.tensor_param_index.size());
+        o << "  GemmOut go;\n";
+        o << "  go.rows = static_cast<int>(rows_ - m_ * " << bm << "u); go.cols = static_cast<int>(cols_ - n_ * " << bn << "u);\n";
+        // Split K: base[ntens] is the scratch (int32 counters, one per tile,
+        // zero between launches, then the partial blocks).
+        if (split)
+            o << "  go.cnt = reinterpret_cast<int*>(A.base[" << nt << "]); go.part = reinterpret_cast<float*>(A.base[" << nt << "] + "
+              << kScratchCounters * 4 << ");\n  go.tile = static_cast<int>(tile_); go.s = static_cast<int>(sp_); go.ns = " << spec.gemm_split
+              << ";\n";
+        o << "  GB::template run<" << head << ", " << (spec.gemm_edge ? "true" : "false") << ", " << (split ? "true" : "false") << ">" << args
+          << ", go);\n";
     }
-    const std::string its = sks > 1 ? "iters * " + std::to_string(sks) : "iters";
-    const std::string it0 = g.accumulate ? "0" : (sks > 1 ? "(iters - 1) * " + std::to_string(sks) : "iters - 1");
-    o << "    GB::template run<" << (g.accumulate ? "true" : "false") << ">(lds, pa, static_cast<int>(A.s3[" << g.a
-      << "]), pb, static_cast<int>(A.s3[" << g.b << "]), pc, static_cast<int>(A.s3[" << g.c << "]), "
-      << it0 << ", " << its << ", " << (sks > 1 ? "offs" : "off") << (pp ? ", pfa_row, pfb_row" : "") << ");\n";
-    o << "  }\n}\n";
+    o << "}\n";
     ek.source = o.str();
     ek.lds_bytes = pp ? static_cast<size_t>((bk == 64 ? 2 : 4) * 512 * bk * 2 + 256) : static_cast<size_t>(ns * (bm + bn) * bk * es);
     return ek;

@@ -39,13 +39,16 @@ struct EmitSpec {
     bool tile_mma = true;
     // GEMM family on MFMA (only when strides and alignment allow it).
     bool gemm = false;
-    // GEMM: grid variables whose neighbouring tasks are merged into one
-    // workgroup block (factor 2 along rows / columns of C), or -1.
+    // GEMM: the grid variables along which the tasks continue one C matrix
+    // downwards / to the right (-1: none); C is cut into blocks of gemm_bm x
+    // gemm_bn whatever the task tiles are (gemm_edge: the last ones are not
+    // whole), in rings of gemm_ring LDS stages, each holding gemm_kf task K
+    // steps (consecutive ones, adjacent in A's columns and B's rows, in the
+    // accumulate form).  gemm_split: parts of the K range summed by blocks of
+    // their own.
     int gemm_vm = -1, gemm_vn = -1;
-    // GEMM: tasks per block along those variables (powers of two), and task
-    // K steps per LDS stage (consecutive steps whose A columns and B rows
-    // are adjacent, in the accumulate form).
-    int gemm_fm = 1, gemm_fn = 1, gemm_kf = 1;
+    int gemm_bm = 256, gemm_bn = 256, gemm_kf = 1, gemm_ring = 2, gemm_split = 1;
+    bool gemm_edge = false;
     // GEMM: 256x256 blocks with K step 32 or 64 and A / B row pitches that
     // are multiples of 64 elements run as a two-group ping-pong block.
     bool gemm_pingpong = false;
@@ -68,9 +71,14 @@ constexpr int kDecodeMaxUnits = 4096;
 // Scheduling cost of starting a unit, in pages (DecodeSplit::kUnitCost).
 constexpr int kDecodeUnitCost = 3;
 
-// Waves of a GEMM block: 2 along M, 4 along N for 256-wide blocks, else 2.
-inline int gemm_waves_n(int bn) { return bn >= 256 ? 4 : 2; }
-inline int gemm_waves_m() { return 2; }
+// Counters at the start of a program's launch scratch: one per decode unit,
+// or per C block of a GEMM launch with split K.
+constexpr int kScratchCounters = kDecodeMaxUnits;
+
+// Waves of a GEMM block: 2 along M (1 for 32-row blocks), 4 along N for
+// 256-wide and 32-row blocks, else 2.
+inline int gemm_waves_n(int bm, int bn) { return bn >= 256 || (bm == 32 && bn >= 128) ? 4 : 2; }
+inline int gemm_waves_m(int bm) { return bm == 32 ? 1 : 2; }
 
 struct EmittedKernel {
     std::string source;
@@ -79,8 +87,6 @@ struct EmittedKernel {
     int rows_per_chunk = 0;     // row programs: rows handled per wave iteration
     int waves_per_block = 4;
     bool row_program = false;
-    int tasks_per_block = 1;    // GEMM: tasks merged into one workgroup
-    int blocks_per_task = 1;    // GEMM: 256-wide blocks of a task tile above 256
     int part_floats = 0;        // decode: floats per partial (m, l, o of one unit)
     size_t lds_bytes = 0;
     // Tile programs: bytes of global scratch per workgroup for the tiles that

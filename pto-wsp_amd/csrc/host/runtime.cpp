@@ -226,6 +226,10 @@ struct RunEnv {
     int* err = nullptr;
     char* nscratch = nullptr;
     size_t nscratch_limit = 0;
+    // Bytes of launch scratch that a no-allocation run of the program would
+    // have: every run stays below it where it has a choice, so that both
+    // entry points run the same kernels.
+    size_t scratch_limit = 0;
 };
 
 // Workgroups of a tile-program launch whose tiles exceed LDS (each has its
@@ -429,6 +433,7 @@ struct BuiltLaunch {
     int64_t ntasks = 0;
     bool host_checked = false;
     std::vector<int64_t> tasks;  // task-list launches: the grid tasks kept by the masks
+    int64_t gemm_tiles = 0;      // GEMM launches: C blocks (each gemm_split workgroups)
 };
 
 // How param p of a row program is accessed: its own class, or that of a Load
@@ -628,19 +633,98 @@ uint32_t grid_write_hazard(const KernelAnalysis& a, const LaunchSpec& L, const L
     return best;
 }
 
+// C blocks of a GEMM launch and the parts its K range is split into.
+struct GemmShape {
+    int bm = 256, bn = 256, split = 1, ring = 2;
+    int64_t tiles = 0;
+};
+
+// Scratch of a GEMM launch with split K: the counters, then the partial blocks.
+size_t gemm_scratch_bytes(int64_t tiles, int split, int bm, int bn) {
+    return kScratchCounters * sizeof(int32_t) + static_cast<size_t>(tiles) * split * bm * bn * sizeof(float);
+}
+
+// Chooses the C blocks by an estimate of the launch's time.  256x256 blocks
+// use the matrix cores best but leave CUs idle when there are few of them;
+// smaller blocks, and blocks that sum only a part of K, spread the work.  The
+// constants are fits to sweeps of all shapes on one MI355X, in us at K = 2048:
+// `alone` for a block with a CU to itself, `shared` per block of a CU that
+// runs several.  The C traffic is added (a block's epilogue does not overlap
+// its own K loop); a split K costs its partial blocks.  Measured, best shape
+// against the 256x256 blocks (or the tile program) used for everything before:
+//   4 x 1024^3 f16        18 us (128x64; estimate picks 64x128, 18.3)  30
+//   1024^3 bf16           10 (64x64)                                   24
+//   2 x 2048^3 bf16       42 (128x128)                                 53
+//   32 x 4096 x 4096      14 (32x128, 4 parts)                         673
+//   128 x 4096 x 4096     19 (64x64, 4 parts)                          108
+//   1024^3 f32            27 (64x64, 2 parts)                          250
+//   13 x 128 x 5440 x 2944 f32  454 (128x64, 2 parts; picks 1 part, 475)  473
+// False: a product too small for the blocks (below 64 rows or columns with
+// fewer than 128 of the other, or K below 128), left to the tile program.
+bool gemm_shape(int64_t rows, int64_t cols, int64_t problems, int64_t stages, int bk, const GemmInfo& g, bool pp_ok,
+                size_t scratch_limit, GemmShape& sh) {
+    struct Block {
+        int bm, bn;
+        double alone, shared;
+    };
+    static const Block b16[] = {{256, 256, 41, 41},   {128, 128, 22, 13.6}, {64, 128, 14.2, 9.7},
+                                {128, 64, 14.2, 9.7}, {64, 64, 12.2, 5.8},  {32, 128, 11.8, 9}};
+    static const Block b32[] = {{256, 256, 490, 458}, {128, 128, 135, 120}, {64, 128, 71, 62},
+                                {128, 64, 71, 62},    {64, 64, 49, 36},     {32, 128, 46, 33}};
+    const double k = static_cast<double>(stages) * bk;
+    if ((rows < 64 || cols < 64) && (std::max(rows, cols) < 128 || k < 128)) return false;
+    if (stages <= 0) return false;
+    const int es = g.f32 ? 4 : 2;
+    const double bytes_per_us = 5.5e6;
+    const double ab = static_cast<double>(problems) * (rows + cols) * k * es / bytes_per_us;
+    const double c = static_cast<double>(problems) * rows * cols * (g.accumulate ? 8 : 4) / bytes_per_us;
+    double best = 0.0;
+    for (const Block& b : g.f32 ? b32 : b16) {
+        if (b.bm == 32 && rows > 32) continue;
+        // 256x256 blocks only where they are whole (15 x 224 x 6144 x 320 with
+        // a last block row of 224: 71 us, 128x64 blocks 58).
+        if (b.bm == 256 && (rows % 256 || cols % 256)) continue;
+        if (2 * (b.bm + b.bn) * bk * es > 160 * 1024) continue;
+        const int64_t tiles = problems * ((rows + b.bm - 1) / b.bm) * ((cols + b.bn - 1) / b.bn);
+        for (int split = 1; split <= 16; split *= 2) {
+            if (split > 1 && (split > stages / 2 || tiles * split > 1024 || tiles > kScratchCounters ||
+                              gemm_scratch_bytes(tiles, split, b.bm, b.bn) > scratch_limit))
+                break;
+            const double per_cu = std::ceil(static_cast<double>(tiles) * split / 256.0);
+            // The block without the ping-pong schedule is a seventh slower.
+            const double slow = b.bm == 256 && !g.f32 && (!pp_ok || split > 1) ? 1.15 : 1.0;
+            const double work = slow * k / 2048.0 / split * std::max(b.alone, b.shared * per_cu);
+            double t = std::max(work, ab) + c;
+            if (split > 1) t += 1.5 + 0.6 * split + 0.35e-6 * tiles * split * b.bm * b.bn * 4;
+            if (best > 0.0 && t >= best) continue;
+            best = t;
+            sh.bm = b.bm;
+            sh.bn = b.bn;
+            sh.split = split;
+            sh.tiles = tiles;
+        }
+    }
+    if (best == 0.0) return false;
+    // Few workgroups: a ring of four stages keeps more of the operands in
+    // flight (64 x 4096 x 4096 in 4 parts: 13.7 against 16.1 us); several per
+    // CU do so by themselves and lose the LDS (2048^3, 64x64: 35.7 against 33).
+    // Every wave moves the same share of a 4-stage ring's loads, which needs
+    // 4 KiB of A per stage.
+    if (sh.bm <= 64 && sh.bm * bk * es >= 4096 && sh.tiles * sh.split <= 512 && 4 * (sh.bm + sh.bn) * bk * es <= 80 * 1024) sh.ring = 4;
+    return true;
+}
+
 // The MFMA GEMM template needs unit column strides, 16-byte aligned operand
 // rows at every task and K step, an output tile that stays put across the
 // in-kernel loops, and operands that the launch does not write.
-// Chooses the MFMA GEMM path for a launch of a GEMM-family kernel and, where
-// neighbouring tasks' tiles are contiguous in A, B and C, the grid variables
-// whose task pairs are merged into one workgroup block.  Returns false (tile
-// program fallback) when strides, alignment or offset ranges do not allow the
-// direct buffer->LDS loads of the GEMM block.
-bool gemm_allowed(const KernelAnalysis& a, const LaunchSpec& L, const LaunchArgs& A, EmitSpec& spec, int ng, int nvars) {
-    spec.gemm_vm = spec.gemm_vn = -1;
-    spec.gemm_fm = spec.gemm_fn = spec.gemm_kf = 1;
-    spec.gemm_pingpong = false;
-    if (a.family != Family::Gemm || spec.serial) return false;
+// Chooses the MFMA GEMM path for a launch of a GEMM-family kernel: the grid
+// variables along which neighbouring tasks' tiles continue one C matrix (its
+// blocks are then cut regardless of the task tiles), and the blocks' shape.
+// Returns false (tile program) when strides, alignment or offset ranges do
+// not allow the direct buffer->LDS loads of the GEMM block.
+bool gemm_allowed(const KernelAnalysis& a, const LaunchSpec& L, const LaunchArgs& A, EmitSpec& spec, int ng, int nvars,
+                  size_t scratch_limit, int64_t& tiles) {
+    if (a.family != Family::Gemm || spec.serial || A.ntasks <= 0) return false;
     for (int c : spec.indirect_count)
         if (c) return false;
     for (int t : spec.inner_dyn_term)
@@ -659,16 +743,17 @@ bool gemm_allowed(const KernelAnalysis& a, const LaunchSpec& L, const LaunchArgs
     }
     const int tc = L.targs[g.c]->tid;
     if (L.targs[g.a]->tid == tc || L.targs[g.b]->tid == tc) return false;
-    // Merge candidates: rows of C move with A's rows, columns with B's.
+    // Tasks that continue C: its rows move with A's rows, its columns with B's.
     const int64_t M = g.m, N = g.n;
     int vm = -1, vn = -1;
     for (int v = 0; v < ng; ++v) {
-        if (A.ext[v] <= 0 || A.ext[v] % 2) continue;
+        if (A.ext[v] <= 1) continue;
         if (vm < 0 && A.coef[g.a][v] == M * A.s3[g.a] && A.coef[g.c][v] == M * A.s3[g.c] && A.coef[g.b][v] == 0)
             vm = v;
         else if (vn < 0 && A.coef[g.b][v] == N && A.coef[g.c][v] == N && A.coef[g.a][v] == 0)
             vn = v;
     }
+    const int64_t rows = M * (vm >= 0 ? A.ext[vm] : 1), cols = N * (vn >= 0 ? A.ext[vn] : 1);
     // Task K steps per LDS stage: in the accumulate form with one in-kernel
     // loop whose consecutive steps are adjacent A columns and B rows, steps
     // are merged up to 64 columns per stage (32 for f32), dividing the loop.
@@ -679,31 +764,18 @@ bool gemm_allowed(const KernelAnalysis& a, const LaunchSpec& L, const LaunchArgs
         if (A.coef[g.a][v] == g.k && A.coef[g.b][v] == g.k * A.s3[g.b])
             while (g.k * kf * 2 <= kmax && A.ext[v] % (kf * 2) == 0) kf *= 2;
     }
-    const int64_t bk = g.k * kf;
-    auto lds_fits = [&](int64_t bm, int64_t bn) {
-        return bm <= 256 && bn <= 256 && 2 * (bm + bn) * gemm_stage_k(static_cast<int>(bk), g.f32) * es <= 160 * 1024;
-    };
-    // Tasks per block: powers of two along the merge variables (dividing
-    // their extents), growing the smaller side first, up to 256 x 256.
-    // Tiles above 256 are split into 256-wide blocks instead.
-    const int64_t M0 = gemm_block_dim(static_cast<int>(M)), N0 = gemm_block_dim(static_cast<int>(N));
-    int64_t fm = 1, fn = 1;
-    for (;;) {
-        const bool gm = vm >= 0 && M0 * fm * 2 <= 256 && A.ext[vm] % (fm * 2) == 0 && lds_fits(M0 * fm * 2, N0 * fn);
-        const bool gn = vn >= 0 && N0 * fn * 2 <= 256 && A.ext[vn] % (fn * 2) == 0 && lds_fits(M0 * fm, N0 * fn * 2);
-        if (gm && (M0 * fm <= N0 * fn || !gn)) fm *= 2;
-        else if (gn) fn *= 2;
-        else break;
-    }
-    const int64_t bm = M0 * fm, bn = N0 * fn;
-    // Blocks below the MFMA block shape (64 rows / columns) stay on the tile program.
-    if (bm % 64 || bn % 64 || !lds_fits(bm, bn)) return false;
-    spec.gemm_vm = fm > 1 ? vm : -1;
-    spec.gemm_vn = fn > 1 ? vn : -1;
-    spec.gemm_fm = static_cast<int>(fm);
-    spec.gemm_fn = static_cast<int>(fn);
-    spec.gemm_kf = static_cast<int>(kf);
-    // Buffer offsets (32-bit) from a block's step-0 origins.
+    const int64_t kstep = g.k * kf;
+    const int bk = gemm_stage_k(static_cast<int>(kstep), g.f32);
+    int64_t steps = 1;
+    for (int v = ng; v < nvars; ++v) steps *= std::max<int64_t>(0, A.ext[v]);
+    const int64_t stages = (g.accumulate ? steps / kf : std::min<int64_t>(steps, 1)) * (kstep / bk);
+    if (steps * (kstep / bk) >= (int64_t(1) << 31) || rows >= (int64_t(1) << 31) || cols >= (int64_t(1) << 31)) return false;
+    const int64_t problems = A.ntasks / ((vm >= 0 ? A.ext[vm] : 1) * (vn >= 0 ? A.ext[vn] : 1));
+    const bool pp_ok = tuning().gemm_pingpong && !g.f32 && (bk == 64 || bk == 32) && A.s3[g.a] % 64 == 0 && A.s3[g.b] % 64 == 0;
+    GemmShape sh;
+    if (!gemm_shape(rows, cols, problems, stages, bk, g, pp_ok, scratch_limit, sh)) return false;
+    const bool edge = rows % sh.bm != 0 || cols % sh.bn != 0;
+    // Buffer offsets (32-bit) from a block's stage-0 origins.
     int64_t ka = 0, kb = 0;
     for (int v = ng; v < nvars; ++v) {
         ka += A.coef[g.a][v] * std::max<int64_t>(0, A.ext[v] - 1);
@@ -711,11 +783,20 @@ bool gemm_allowed(const KernelAnalysis& a, const LaunchSpec& L, const LaunchArgs
     }
     const int64_t lim = int64_t(1) << 31;
     if (A.s3[g.a] >= lim || A.s3[g.b] >= lim || A.s3[g.c] >= lim) return false;
-    if (((bm - 1) * A.s3[g.a] + g.k) * es + ka * es >= lim) return false;
-    if (((bk - 1) * A.s3[g.b] + bn) * es + kb * es >= lim) return false;
-    if (((bm - 1) * A.s3[g.c] + bn) * 4 >= lim) return false;
-    spec.gemm_pingpong = tuning().gemm_pingpong && !g.f32 && bm == 256 && bn == 256 && (bk == 64 || bk == 32) &&
-                         A.s3[g.a] % 64 == 0 && A.s3[g.b] % 64 == 0;
+    if (((sh.bm - 1) * A.s3[g.a] + g.k) * es + ka * es >= lim) return false;
+    if (((kstep - 1) * A.s3[g.b] + sh.bn) * es + kb * es >= lim) return false;
+    if (((sh.bm - 1) * A.s3[g.c] + sh.bn) * 4 >= lim) return false;
+    if (sh.tiles * sh.split >= lim) return false;
+    spec.gemm_vm = vm;
+    spec.gemm_vn = vn;
+    spec.gemm_bm = sh.bm;
+    spec.gemm_bn = sh.bn;
+    spec.gemm_kf = static_cast<int>(kf);
+    spec.gemm_ring = sh.ring;
+    spec.gemm_split = sh.split;
+    spec.gemm_edge = edge;
+    spec.gemm_pingpong = pp_ok && sh.bm == 256 && sh.bn == 256 && !edge && sh.split == 1;
+    tiles = sh.tiles;
     return true;
 }
 
@@ -874,10 +955,7 @@ void apply_masks(RunEnv& E, const LaunchSpec& L, BuiltLaunch& B) {
     B.spec.task_list = true;
     // The GEMM and decode programs map several tasks or a cost-balanced
     // split onto a workgroup; a task list runs on the row or tile program.
-    B.spec.gemm = false;
-    B.spec.gemm_pingpong = false;
-    B.spec.gemm_vm = B.spec.gemm_vn = -1;
-    B.spec.gemm_fm = B.spec.gemm_fn = B.spec.gemm_kf = 1;
+    B.spec.gemm = B.spec.gemm_pingpong = false;
     B.spec.decode = false;
 }
 
@@ -1078,12 +1156,7 @@ BuiltLaunch build_launch(RunEnv& E, const LaunchSpec& L) {
     if (B.spec.serial && !tuning().serial_groups) B.spec.seq_mask = 0;  // 0: every grid variable, one workgroup
     B.spec.row_up = tuning().row_up;
     B.spec.nontemporal = tuning().nontemporal;
-    B.spec.gemm = gemm_allowed(a, L, A, B.spec, ng, nvars);
-    if (!B.spec.gemm) {
-        B.spec.gemm_vm = B.spec.gemm_vn = -1;
-        B.spec.gemm_fm = B.spec.gemm_fn = B.spec.gemm_kf = 1;
-        B.spec.gemm_pingpong = false;
-    }
+    B.spec.gemm = gemm_allowed(a, L, A, B.spec, ng, nvars, E.scratch_limit, B.gemm_tiles);
     B.spec.decode = decode_allowed(a, L, A, B.spec, ng);
     B.spec.row_loops = tuning().row_loops && row_loops_allowed(a, L, A, B.spec, ng, nvars);
     B.spec.decode_ring = tuning().decode_ring ? tuning().decode_ring : decode_ring_for(a.decode.d, a.decode.g, a.decode.f32);
@@ -1104,8 +1177,8 @@ BuiltLaunch build_launch(RunEnv& E, const LaunchSpec& L) {
 std::string spec_key(const EmitSpec& s) {
     std::ostringstream o;
     o << "vw" << s.vec_width << (s.row_unit_cols ? "u" : "") << (s.serial ? ";serial" + std::to_string(s.seq_mask) : "") << (s.task_list ? ";tl" : "") << ";up" << s.row_up << (s.nontemporal ? ";nt" : "")
-      << (s.row_loops ? ";rl" : "") << (s.gemm ? ";gemm" : "") << ";m" << s.gemm_vm << ";n" << s.gemm_vn << ";f" << s.gemm_fm << "x" << s.gemm_fn << "x" << s.gemm_kf
-      << (s.gemm_pingpong ? ";pp" : "")
+      << (s.row_loops ? ";rl" : "") << (s.gemm ? ";gemm" : "") << ";m" << s.gemm_vm << ";n" << s.gemm_vn << ";b" << s.gemm_bm << "x" << s.gemm_bn << "x" << s.gemm_kf << "x" << s.gemm_ring
+      << "s" << s.gemm_split << (s.gemm_edge ? ";edge" : "") << (s.gemm_pingpong ? ";pp" : "")
       << (s.decode ? ";dec" : "")
       << (s.decode_norm ? ";norm" : "") << (s.tile_mma ? ";mma" : "") << ";t" << s.threads << ";r" << s.decode_ring << ";w" << s.decode_waves << (s.decode_ordered ? ";ord" : "")
       << ";i";
@@ -1157,11 +1230,33 @@ DecodeShape decode_shape(hipFunction_t f, int threads) {
     return r;
 }
 
+// A launch's scratch: kScratchCounters int32 counters, zeroed when the scratch
+// is allocated (a no-allocation run: at its start, in the fixed device
+// scratch) and left at zero by every launch, then partials.  A program's
+// launches run one after the other on its stream and share it.
+bool scratch_fits(const RunEnv& E, size_t need) { return !E.nscratch || kNoAllocHeaderBytes + need <= E.nscratch_limit; }
+char* launch_scratch(RunEnv& E, size_t need) {
+    if (E.nscratch) return E.nscratch + kNoAllocHeaderBytes;
+    ptowsp_program* P = E.P;
+    if (need > P->scratch_bytes) {
+        if (P->scratch) {
+            // Earlier launches of this run may still use the smaller one.
+            check(hipDeviceSynchronize(), "hipDeviceSynchronize");
+            check(hipFree(P->scratch), "hipFree(scratch)");
+        }
+        P->scratch = nullptr;
+        P->scratch_bytes = 0;
+        check(hipMalloc(&P->scratch, need), "hipMalloc(launch scratch)");
+        check(hipMemset(P->scratch, 0, kScratchCounters * sizeof(int32_t)), "hipMemset(scratch counters)");
+        check(hipDeviceSynchronize(), "hipDeviceSynchronize");
+        P->scratch_bytes = need;
+    }
+    return static_cast<char*>(P->scratch);
+}
+
 // One launch of the balanced decode kernel (emit_decode): one block per
-// CU.  The program's scratch starts with kDecodeMaxUnits int32
-// counters, zeroed when the scratch is allocated and left at zero by every
-// launch; the partials follow, one slot per (unit, wave) pair: units + waves
-// slots.
+// CU.  Counters: one per unit; partials: one slot per (unit, wave) pair,
+// units + waves slots.
 void enqueue_decode(RunEnv& E, int li, BuiltLaunch& B, const EmittedKernel& ek, const JitKernel& jk, hipStream_t stream,
                     uint64_t& launches) {
     ptowsp_program* P = E.P;
@@ -1173,31 +1268,15 @@ void enqueue_decode(RunEnv& E, int li, BuiltLaunch& B, const EmittedKernel& ek, 
     const DecodeShape shape = decode_shape(jk.function, ek.threads);
     const int64_t grid = shape.blocks;
     const int64_t waves = static_cast<int64_t>(ek.threads / 64) * grid;
-    const size_t count_bytes = static_cast<size_t>(kDecodeMaxUnits) * sizeof(int32_t);
     const size_t part_bytes = static_cast<size_t>(B.ntasks + waves) * static_cast<size_t>(ek.part_floats) * sizeof(float);
-    const size_t need = count_bytes + part_bytes;
+    const size_t need = kScratchCounters * sizeof(int32_t) + part_bytes;
     const int ntens = static_cast<int>(a.tensor_param_index.size());
     if (ntens >= kMaxParams) throw std::runtime_error("decode launch: no argument slot for its scratch");
-    if (E.nscratch) {
-        // No-allocation run: counters (zeroed at the start of the run) and
-        // partials in the fixed device scratch.
-        char* base = E.nscratch + kNoAllocHeaderBytes;
-        if (kNoAllocHeaderBytes + need > E.nscratch_limit)
-            throw std::runtime_error("ptowsp_hip_launch_noalloc: the decode launch needs " +
-                                     std::to_string(kNoAllocHeaderBytes + need) + " bytes of scratch, more than the " +
-                                     std::to_string(E.nscratch_limit) + " bytes available (the fixed scratch holds " +
-                                     std::to_string(kNoAllocScratchBytes) + " bytes)");
-        B.args.base[ntens] = base;
-    } else if (need > P->scratch_bytes) {
-        if (P->scratch) check(hipFree(P->scratch), "hipFree(scratch)");
-        P->scratch = nullptr;
-        P->scratch_bytes = 0;
-        check(hipMalloc(&P->scratch, need), "hipMalloc(decode scratch)");
-        check(hipMemset(P->scratch, 0, count_bytes), "hipMemset(decode counters)");
-        check(hipDeviceSynchronize(), "hipDeviceSynchronize");
-        P->scratch_bytes = need;
-    }
-    if (!E.nscratch) B.args.base[ntens] = static_cast<char*>(P->scratch);
+    if (E.nscratch && !scratch_fits(E, need))
+        throw std::runtime_error("ptowsp_hip_launch_noalloc: the decode launch needs " + std::to_string(kNoAllocHeaderBytes + need) +
+                                 " bytes of scratch, more than the " + std::to_string(E.nscratch_limit) +
+                                 " bytes available (the fixed scratch holds " + std::to_string(kNoAllocScratchBytes) + " bytes)");
+    B.args.base[ntens] = launch_scratch(E, need);
     B.args.span[ntens] = static_cast<int64_t>(need / sizeof(float));
     B.args.scal[kMaxScalars - 1] = static_cast<uint64_t>(maxp);
     void* params[] = {&B.args};
@@ -1233,6 +1312,12 @@ void enqueue_built(RunEnv& E, int li, BuiltLaunch& B, hipStream_t stream, uint64
     }
     if (B.spec.task_list) B.args.tlist = reinterpret_cast<const i64*>(upload_task_list(E, B.tasks, stream));
     const LaunchSpec& L = P->plan.launches[li];
+    if (B.spec.gemm && B.spec.gemm_split > 1) {
+        const size_t need = gemm_scratch_bytes(B.gemm_tiles, B.spec.gemm_split, B.spec.gemm_bm, B.spec.gemm_bn);
+        const int ntens = static_cast<int>(P->ka[L.kernel].tensor_param_index.size());
+        B.args.base[ntens] = launch_scratch(E, need);
+        B.args.span[ntens] = static_cast<int64_t>(need / sizeof(float));
+    }
     if (P->ka[L.kernel].family == Family::Custom) {
         ptowsp_program::CustomRun run;
         size_t grid = 1;
@@ -1264,14 +1349,10 @@ void enqueue_built(RunEnv& E, int li, BuiltLaunch& B, hipStream_t stream, uint64
             for (size_t v = 0; v < L.grid.size(); ++v)
                 if (!((seq >> v) & 1u)) blocks *= std::max<int64_t>(1, B.args.ext[v]);
     } else {
-        blocks = B.ntasks / ek.tasks_per_block * ek.blocks_per_task;
+        blocks = B.ntasks;
     }
-    if (B.spec.gemm && !B.spec.serial) {
-        // GEMM kernels run exactly one block per workgroup.
-        if (blocks > 0x7FFFFFFF) throw std::runtime_error("GEMM launch: more than 2^31-1 blocks");
-    } else {
-        blocks = std::min<int64_t>(blocks, int64_t(1) << 20);
-    }
+    if (B.spec.gemm && !B.spec.serial) blocks = B.gemm_tiles * B.spec.gemm_split;  // exactly one block per workgroup
+    else blocks = std::min<int64_t>(blocks, int64_t(1) << 20);
     blocks = std::max<int64_t>(1, blocks);
     if (ek.gtile_bytes > 0) {
         // Tiles beyond LDS live in global scratch, one region per workgroup;
@@ -1710,19 +1791,21 @@ int launch_impl(ptowsp_program* P, RuntimeContext* ctx, void* hip_stream, ptowsp
     // replays the values the run read, after the run.
     const bool slot_loads = module_loads_slots(P->m) || custom;
     const std::vector<int> dev_ext = device_extent_tensors(E);
+    // The extent copies of a no-allocation run sit at the tail of the scratch;
+    // its launches may use everything before them.
+    size_t ext_bytes = 0;
+    for (int tid : dev_ext) ext_bytes += static_cast<size_t>(std::max<int64_t>(E.ts[tid].span, 0)) * 4;
+    ext_bytes = (ext_bytes + 255) / 256 * 256;
+    const bool ext_fit = ext_bytes + kNoAllocHeaderBytes + kScratchCounters * sizeof(int32_t) <= kNoAllocScratchBytes;
+    E.scratch_limit = ext_fit ? kNoAllocScratchBytes - ext_bytes - kNoAllocHeaderBytes : 0;
     if (noalloc) {
-        // The extent copies sit at the tail of the scratch; the decode
-        // launches may use everything before them.
-        size_t ext_bytes = 0;
-        for (int tid : dev_ext) ext_bytes += static_cast<size_t>(std::max<int64_t>(E.ts[tid].span, 0)) * 4;
-        ext_bytes = (ext_bytes + 255) / 256 * 256;
-        if (ext_bytes + kNoAllocHeaderBytes + kDecodeMaxUnits * sizeof(int32_t) > kNoAllocScratchBytes)
+        if (!ext_fit)
             throw std::runtime_error("ptowsp_hip_launch_noalloc: the loop-extent tensors (" + std::to_string(ext_bytes) +
                                      " bytes) do not fit in the fixed scratch of " + std::to_string(kNoAllocScratchBytes) +
                                      " bytes");
         E.nscratch_limit = kNoAllocScratchBytes - ext_bytes;
-        // The error flag and the decode unit counters start at zero.
-        noalloc_zero(E.nscratch, kNoAllocHeaderBytes + kDecodeMaxUnits * sizeof(int32_t), stream);
+        // The error flag and the counters start at zero.
+        noalloc_zero(E.nscratch, kNoAllocHeaderBytes + kScratchCounters * sizeof(int32_t), stream);
     }
     CycleResult cyc{};
     bool ext_written = false;
@@ -1854,18 +1937,23 @@ int ptowsp_hip_precompile(ptowsp_program* P, int index, int flags, const char** 
                 spec.row_unit_cols = true;
             }
             const int ng = static_cast<int>(L.grid.size());
-            if ((flags & 2) && spec.gemm && ng >= 2 && a.gemm.m <= 128 && a.gemm.n <= 128 &&
-                2 * (2 * a.gemm.m + 2 * a.gemm.n) * a.gemm.k * 2 <= 160 * 1024) {
-                spec.gemm_vm = ng - 2;
-                spec.gemm_vn = ng - 1;
-                spec.gemm_fm = spec.gemm_fn = 2;
-                spec.gemm_pingpong = (flags & 4) && a.gemm.m == 128 && a.gemm.n == 128 && (a.gemm.k == 64 || a.gemm.k == 32);
+            if (spec.gemm) {
+                // One block per task, or one per 2 x 2 tasks (merged).
+                int f = 1;
+                if ((flags & 2) && ng >= 2 && a.gemm.m <= 128 && a.gemm.n <= 128 &&
+                    2 * (2 * a.gemm.m + 2 * a.gemm.n) * a.gemm.k * 2 <= 160 * 1024) {
+                    f = 2;
+                    spec.gemm_vm = ng - 2;
+                    spec.gemm_vn = ng - 1;
+                    spec.gemm_pingpong = (flags & 4) && a.gemm.m == 128 && a.gemm.n == 128 && (a.gemm.k == 64 || a.gemm.k == 32);
+                }
+                spec.gemm_bm = gemm_block_dim(a.gemm.m) * f;
+                spec.gemm_bn = gemm_block_dim(a.gemm.n) * f;
             }
             // Blocks below the MFMA block shape: the tile program.
-            if (spec.gemm && ((a.gemm.m * spec.gemm_fm) % 64 || (a.gemm.n * spec.gemm_fn) % 64)) {
+            if (spec.gemm && (spec.gemm_bm % 64 || spec.gemm_bn % 64)) {
                 spec.gemm = spec.gemm_pingpong = false;
                 spec.gemm_vm = spec.gemm_vn = -1;
-                spec.gemm_fm = spec.gemm_fn = 1;
             }
             const EmittedKernel& ek = emitted_for(P, static_cast<int>(li), spec);
             (void)jit_compile(ek.source);
