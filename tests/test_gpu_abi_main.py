@@ -85,6 +85,8 @@ def test_slot_branch_through_module_main(gpu, tmp_path, value, want):
 
 
 def test_paged_decode_through_module_main(gpu, tmp_path):
+    if cases.artifact("paged_decode") is None:
+        pytest.skip("integration artifacts not built (reference headers absent at build time)")
     a = cases.decode_arrays()
     # Tensor ids in the bridge's first-use order (the page counts bound the page loop first);
     # K is read through its transposed view.
