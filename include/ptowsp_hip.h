@@ -124,7 +124,8 @@ int ptowsp_hip_kernel_family(const ptowsp_program* prog, const char* kernel);
  * ping-pong GEMM block; bit 4: build row-program launches with in-kernel
  * loops as row programs that run the loops inside each row's lane team;
  * bit 5: build decode launches with the following `out = o / l` launch
- * folded into them (the form a run uses when that launch follows). */
+ * folded into them (the form a run uses when that launch follows); bit 6:
+ * build launches with matmuls whose rows are independent as row blocks. */
 int ptowsp_hip_precompile(ptowsp_program* prog, int index, int flags, const char** source);
 
 /* Evaluates only the cpu_sim cycle model (total_cycles, task_count) for the

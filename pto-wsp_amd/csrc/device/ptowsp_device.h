@@ -1041,6 +1041,183 @@ __device__ inline void tile_mma16(FA a, FB b, float* c, float* scratch) {
     }
 }
 
+// Reduction over the lanes l%16 + 16*i (i = 0..3), the four lanes that hold
+// one row of a transposed value: a swap of the wave's halves, then
+// of its odd and even 16-lane rows.  Every lane ends with the result, and
+// computes it with the same operand order (lower lane's value first).
+template <class Op>
+__device__ inline float cross4_reduce(float x, Op op) {
+    const u32 b = __float_as_uint(x);
+    const auto h = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+    x = op(__uint_as_float(h[0]), __uint_as_float(h[1]));
+    const u32 c = __float_as_uint(x);
+    const auto r = __builtin_amdgcn_permlane16_swap(c, c, false, false);
+    return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+// ---------------------------------------------------------------------------
+// Row blocks: 16 rows of a task per wave, values in registers
+// ---------------------------------------------------------------------------
+//
+// A [16, 16*NB] fp32 value is held transposed: lane l has row l%16, columns
+// 16*j + 4*(l/16) + e of register v[j][e].  That is at once
+//   * the result layout of v_mfma_f32_16x16x4_f32 when the rows are its N
+//     dimension (D = B^T A^T: lane l holds 4 consecutive D rows, i.e. columns
+//     of the value, of value row l%16), and
+//   * its operand layout for the next product: the K order of a product is
+//     free, so MFMA (j, e) takes column 16*j + 4*(l/16) + e from every lane
+//     group's own register, against the same rows of the right operand.
+// So a chain of products, elementwise ops and row reductions (over the lane's
+// registers, then the row's 4 lanes) never leaves the registers; only the
+// right operands of products go through LDS (row pitch N + 4: the 4 lane
+// groups of a read hit distinct quarters of the banks).
+//
+// What bounds it: attention tiles of 64 rows at head dim 64 (4 x 16 x 2048)
+// move 134 MB and need 2.1 GFLOP of fp32 MFMA, 22 and 14 us; as a tile
+// program (values in LDS, a workgroup barrier per op, sequential row
+// reductions on 64 of 256 threads) 86 us, as row blocks 38 us.
+template <int NB>
+struct RV {
+    f32x4v v[NB];
+};
+
+// Element (row, column) at p + row*s3 + column*s4; VEC: unit columns and
+// 16-byte aligned rows.
+template <int NB, bool VEC>
+__device__ inline RV<NB> rv_load(const float* p, i64 s3, i64 s4) {
+    const int lane = threadIdx.x & 63;
+    const float* q = p + (lane & 15) * s3 + 4 * (lane >> 4) * (VEC ? 1 : s4);
+    RV<NB> r;
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+        if constexpr (VEC) {
+            r.v[j] = *reinterpret_cast<const f32x4v*>(q + 16 * j);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) r.v[j][e] = q[(16 * j + e) * s4];
+        }
+    }
+    return r;
+}
+template <int NB, bool VEC>
+__device__ inline void rv_store(float* p, i64 s3, i64 s4, const RV<NB>& r) {
+    const int lane = threadIdx.x & 63;
+    float* q = p + (lane & 15) * s3 + 4 * (lane >> 4) * (VEC ? 1 : s4);
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+        if constexpr (VEC) {
+            *reinterpret_cast<f32x4v*>(q + 16 * j) = r.v[j];
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) q[(16 * j + e) * s4] = r.v[j][e];
+        }
+    }
+}
+template <class Op, int NB>
+__device__ inline RV<NB> rv_ew(const RV<NB>& a, const RV<NB>& b) {
+    RV<NB> r;
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) r.v[j][e] = Op::f(static_cast<float>(a.v[j][e]), static_cast<float>(b.v[j][e]));
+    return r;
+}
+template <class Op, int NB>
+__device__ inline RV<NB> rv_ew(const RV<NB>& a, float s) {
+    RV<NB> r;
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) r.v[j][e] = Op::f(static_cast<float>(a.v[j][e]), s);
+    return r;
+}
+template <class Op, int NB>
+__device__ inline RV<NB> rv_ew(float s, const RV<NB>& a) {
+    RV<NB> r;
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) r.v[j][e] = Op::f(s, static_cast<float>(a.v[j][e]));
+    return r;
+}
+template <int NB>
+__device__ inline RV<NB> rv_exp(const RV<NB>& a) {
+    RV<NB> r;
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) r.v[j][e] = expf(a.v[j][e]);
+    return r;
+}
+template <int NB>
+__device__ inline RV<NB> rv_rsqrt(const RV<NB>& a) {
+    RV<NB> r;
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) r.v[j][e] = rsqrt_cr(a.v[j][e]);
+    return r;
+}
+template <int NB>
+__device__ inline float rv_sum(const RV<NB>& a) {
+    float s = a.v[0][0];
+#pragma unroll
+    for (int i = 1; i < 4 * NB; ++i) s = s + a.v[i >> 2][i & 3];
+    return cross4_reduce(s, [](float x, float y) { return x + y; });
+}
+// The oracle's left-to-right maximum: a NaN is kept only as the row's first
+// element, which lane group 0 holds, and the lower lane's value comes first.
+template <int NB>
+__device__ inline float rv_max(const RV<NB>& a) {
+    float m = (threadIdx.x & 48) == 0 ? a.v[0][0] : -__builtin_inff();
+#pragma unroll
+    for (int i = 0; i < 4 * NB; ++i) m = a.v[i >> 2][i & 3] > m ? a.v[i >> 2][i & 3] : m;
+    return cross4_reduce(m, [](float x, float y) { return y > x ? y : x; });
+}
+
+// a [16, 16*KB] x b [16*KB, 16*NB], b in LDS with row pitch LDN.
+template <int KB, int NB, int LDN>
+__device__ inline RV<NB> rv_matmul(const RV<KB>& a, const float* b) {
+    const int lane = threadIdx.x & 63;
+    const float* q = b + 4 * (lane >> 4) * LDN + (lane & 15);
+    RV<NB> r;
+#pragma unroll
+    for (int n = 0; n < NB; ++n) r.v[n] = f32x4v{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int j = 0; j < KB; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int n = 0; n < NB; ++n)
+                r.v[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(q[(16 * j + e) * LDN + 16 * n], a.v[j][e], r.v[n], 0, 0, 0);
+    return r;
+}
+
+// Copies a [K, N] right operand (element (k, n) at p + k*s3 + n*s4) into LDS.
+// MODE 0: unit s4, 16-byte aligned rows; 1: unit s3, 16-byte aligned columns
+// (a transposed view); 2: any strides.
+template <int K, int N, int LDN, int MODE, int NT>
+__device__ inline void rv_stage(float* dst, const float* p, i64 s3, i64 s4) {
+    if constexpr (MODE == 0) {
+#pragma unroll 8
+        for (int e = threadIdx.x; e < K * N / 4; e += NT) {
+            const int k = e / (N / 4), n = e % (N / 4) * 4;
+            *reinterpret_cast<f32x4v*>(dst + k * LDN + n) = *reinterpret_cast<const f32x4v*>(p + k * s3 + n);
+        }
+    } else if constexpr (MODE == 1) {
+#pragma unroll 8
+        for (int e = threadIdx.x; e < K * N / 4; e += NT) {
+            const int n = e / (K / 4), k = e % (K / 4) * 4;
+            const f32x4v x = *reinterpret_cast<const f32x4v*>(p + n * s4 + k);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) dst[(k + i) * LDN + n] = x[i];
+        }
+    } else {
+#pragma unroll 8
+        for (int e = threadIdx.x; e < K * N; e += NT) dst[(e / N) * LDN + e % N] = p[(e / N) * s3 + (e % N) * s4];
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Ping-pong GEMM block: 256x256 C block, 8 waves in two groups of four
 // ---------------------------------------------------------------------------
@@ -1491,20 +1668,6 @@ __device__ inline f32x4v_t mfma_16x16x32(u32x4 a, u32x4 b, f32x4v_t c) {
     else
         return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0,
                                                        0);
-}
-
-// Reduction over the lanes l%16 + 16*i (i = 0..3), the four lanes that hold
-// one query row of the transposed scores: a swap of the wave's halves, then
-// of its odd and even 16-lane rows.  Every lane ends with the result, and
-// computes it with the same operand order (lower lane's value first).
-template <class Op>
-__device__ inline float cross4_reduce(float x, Op op) {
-    const u32 b = __float_as_uint(x);
-    const auto h = __builtin_amdgcn_permlane32_swap(b, b, false, false);
-    x = op(__uint_as_float(h[0]), __uint_as_float(h[1]));
-    const u32 c = __float_as_uint(x);
-    const auto r = __builtin_amdgcn_permlane16_swap(c, c, false, false);
-    return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
 
 // Partials pass between waves of different XCDs (each XCD has its own L2).

@@ -393,6 +393,94 @@ DecodeInfo classify_decode(const KernelDef& k, const KernelAnalysis& a) {
     return info;
 }
 
+// Row-block form of a kernel (see RowBlockInfo).
+RowBlockInfo classify_rowblock(const KernelDef& k, const KernelAnalysis& a) {
+    RowBlockInfo r, no;
+    int R = 0;
+    for (const auto& op : k.ops)
+        if (op.kind == OpKind::Matmul) {
+            r.matmul = true;
+            if (R == 0) R = a.by_id[op.result]->rows;
+        }
+    if (R == 0) {
+        if (a.family != Family::RowProgram) return no;
+        R = a.rows;
+    }
+    if (R < 16 || R % 16) return no;
+    r.rows = R;
+    r.cls.assign(a.max_id + 1, RowClass::None);
+    r.right.assign(a.tensor_param_index.size(), false);
+    // How each value is used besides as a matmul's right operand.
+    std::vector<int> row_bcast(a.max_id + 1, 0), col_bcast(a.max_id + 1, 0), other(a.max_id + 1, 0);
+    for (size_t i = 0; i < k.ops.size(); ++i) {
+        const auto& op = k.ops[i];
+        switch (op.kind) {
+            case OpKind::Constant: case OpKind::CpuSimAddCycles: case OpKind::Store: case OpKind::TMov: case OpKind::Exp:
+            case OpKind::Rsqrt: case OpKind::RowSum: case OpKind::RowMax: case OpKind::RowMean: case OpKind::Matmul:
+            case OpKind::Load: case OpKind::Add: case OpKind::Sub: case OpKind::Mul: case OpKind::Div: case OpKind::Max:
+            case OpKind::Min: break;
+            default: return no;
+        }
+        if (op.kind == OpKind::Matmul) {
+            const ValueInfo *x = a.by_id[op.operands[0]], *y = a.by_id[op.operands[1]];
+            const int pb = a.param_of[y->id];
+            if (op.operands.size() != 2 || pb < 0 || x->rows != R || x->cols % 16 || y->cols % 16) return no;
+            if (!tile_mma_kind(x->rows, x->cols, y->cols)) return no;
+            r.right[a.tensor_ordinal[pb]] = true;
+            ++other[x->id];
+            continue;
+        }
+        for (size_t j = 0; j < op.operands.size(); ++j) {
+            const int id = op.operands[j];
+            if (is_binary(op.kind) && j == 1 && a.bin_mode[i] == BinMode::RowExpand) ++row_bcast[id];
+            else if (is_binary(op.kind) && j == 1 && a.bin_mode[i] == BinMode::ColExpand) ++col_bcast[id];
+            else ++other[id];
+        }
+    }
+    for (const auto& v : k.values) {
+        if (!v.tile) {
+            r.cls[v.id] = RowClass::Scalar;
+            if (a.by_id[v.id]->dtype != DType::F32) return no;
+            continue;
+        }
+        if (v.dtype != DType::F32) return no;
+        const bool used = row_bcast[v.id] || col_bcast[v.id] || other[v.id];
+        const int p = a.param_of[v.id];
+        if (!used) {
+            // A right operand only, or a result nothing reads.
+            if (p >= 0 && r.right[a.tensor_ordinal[p]]) continue;
+            if (p >= 0) return no;
+        }
+        bool given = p >= 0;  // a param's tile, or a Load of one
+        for (const auto& op : k.ops) given = given || (op.kind == OpKind::Load && op.result == v.id);
+        RowClass c = RowClass::None;
+        if (v.rows == R && v.cols == 1 && !col_bcast[v.id]) c = RowClass::RowVec;
+        else if (v.rows == R && v.cols % 16 == 0 && !row_bcast[v.id] && !col_bcast[v.id]) c = RowClass::Full;
+        else if (given && v.rows == 1 && v.cols == R && row_bcast[v.id] && !col_bcast[v.id] && !other[v.id]) c = RowClass::RowVecT;
+        else if (given && v.rows == 1 && v.cols % 16 == 0 && col_bcast[v.id] && !row_bcast[v.id] && !other[v.id]) c = RowClass::ColVec;
+        else if (given && v.cols == 1 && v.rows % 16 == 0 && col_bcast[v.id] && !row_bcast[v.id] && !other[v.id]) c = RowClass::ColVecT;
+        if (c == RowClass::None) return no;
+        r.cls[v.id] = c;
+    }
+    for (const auto& op : k.ops) {
+        if (op.kind == OpKind::RowSum || op.kind == OpKind::RowMax || op.kind == OpKind::RowMean)
+            if (r.cls[op.operands[0]] != RowClass::Full) return no;
+        if (op.kind == OpKind::Store) {
+            const RowClass c = r.cls[op.operands[1]];
+            if (c != RowClass::Full && c != RowClass::RowVec) return no;
+            if (r.cls[op.operands[0]] != c) return no;
+        }
+        if ((op.kind == OpKind::Load || op.kind == OpKind::TMov) && r.cls[op.operands[0]] != r.cls[op.result]) return no;
+        if (is_binary(op.kind) || op.kind == OpKind::Exp || op.kind == OpKind::Rsqrt) {
+            const RowClass c = r.cls[op.result];
+            if (c != RowClass::Full && c != RowClass::RowVec) return no;
+        }
+        if (op.kind == OpKind::Matmul && (r.cls[op.operands[0]] != RowClass::Full || r.cls[op.result] != RowClass::Full)) return no;
+    }
+    r.ok = true;
+    return r;
+}
+
 }  // namespace
 
 KernelAnalysis analyze_kernel(const KernelDef& k) {
@@ -720,6 +808,7 @@ KernelAnalysis analyze_kernel(const KernelDef& k) {
         a.decode = a.gemm.ok ? DecodeInfo{} : classify_decode(k, a);
         a.family = a.gemm.ok ? Family::Gemm : (a.decode.ok ? Family::Decode : Family::TileProgram);
     }
+    if (a.family == Family::RowProgram || a.family == Family::TileProgram) a.rowblock = classify_rowblock(k, a);
     return a;
 }
 

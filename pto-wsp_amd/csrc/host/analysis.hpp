@@ -65,6 +65,29 @@ struct NormInfo {
     int g = 0, d = 0;
 };
 
+// A kernel whose rows are independent once its matmuls' right operands are
+// given: every value is [rows, n] (or a vector broadcast over them), computed
+// row by row, and matmuls multiply such a value by a param tile.  Its blocks
+// of 16 rows run as waves that hold their values in registers (RV on the
+// device), alone or chained with the launches that follow.
+struct RowBlockInfo {
+    bool ok = false;
+    bool matmul = false;           // has matmuls, all of them of MFMA shape
+    int rows = 0;                  // a multiple of 16
+    std::vector<RowClass> cls;     // value id -> class (Full: [rows, 16*n]); None for right operands only
+    std::vector<bool> right;       // tensor ordinal: a matmul's right operand
+};
+
+// MFMA block size of a tile-program matmul [m,k] x [k,n]: 32 (m, n multiples
+// of 32, k even), 16 (m, n multiples of 16, k a multiple of 4, at least 32^3
+// products) or 0 (the scalar loop, bit for bit the oracle's); k at most 32 or
+// a multiple of 32.
+inline int tile_mma_kind(int64_t m, int64_t k, int64_t n) {
+    if (k > 32 && k % 32 != 0) return 0;
+    if (m % 32 == 0 && n % 32 == 0 && k % 2 == 0) return 32;
+    return m % 16 == 0 && n % 16 == 0 && k % 4 == 0 && m * n * k >= 32 * 32 * 32 ? 16 : 0;
+}
+
 struct KernelAnalysis {
     const KernelDef* def = nullptr;
     int max_id = 0;
@@ -92,6 +115,7 @@ struct KernelAnalysis {
     GemmInfo gemm;
     DecodeInfo decode;
     NormInfo norm;
+    RowBlockInfo rowblock;
 };
 
 // Throws CompileError for kernels the reference lowering cannot compute.

@@ -594,20 +594,10 @@ EmittedKernel emit_tile(const Module& m, const KernelAnalysis& a, const LaunchSp
     size_t staged_bytes = 0;
     for (const auto& p : k.params)
         if (staged_id(p.id)) staged_bytes += static_cast<size_t>(SB) * a.by_id[p.id]->rows * a.by_id[p.id]->cols * (is_int_v(p.id) ? 8 : 4);
-    // 32: 32x32 blocks (M, N multiples of 32, K even); 16: 16x16 blocks (M, N
-    // multiples of 16, K a multiple of 4, at least 32^3 products); K at most
-    // 32 or a multiple of 32.
     auto mma_kind = [&](const OpInfo& op) {
-        if (op.kind != OpKind::Matmul || op.result <= 0) return 0;
-        const ValueInfo* av = a.by_id[op.operands[0]];
-        const ValueInfo* bv = a.by_id[op.operands[1]];
-        const int M = av->rows, K = av->cols, N = bv->cols;
-        if (is_int_v(op.result) || is_int_v(op.operands[0]) || is_int_v(op.operands[1]) || spec.threads % 64 != 0) return 0;
-        if (K > 32 && K % 32 != 0) return 0;
-        if (M % 32 == 0 && N % 32 == 0 && K % 2 == 0) return 32;
-        // (smaller products keep the scalar loop, bit for bit the oracle's)
-        if (M % 16 == 0 && N % 16 == 0 && K % 4 == 0 && M * N * K >= 32 * 32 * 32) return 16;
-        return 0;
+        if (op.kind != OpKind::Matmul || op.result <= 0 || spec.threads % 64 != 0) return 0;
+        if (is_int_v(op.result) || is_int_v(op.operands[0]) || is_int_v(op.operands[1])) return 0;
+        return tile_mma_kind(a.by_id[op.operands[0]]->rows, a.by_id[op.operands[0]]->cols, a.by_id[op.operands[1]]->cols);
     };
     auto mma_shape = [&](const OpInfo& op) { return mma_kind(op) != 0; };
     const size_t mma_scratch = static_cast<size_t>(spec.threads / 64) * 32 * kTileMmaPitchHost * 4;
@@ -1486,6 +1476,221 @@ EmittedKernel emit_custom(const Module& m, const KernelAnalysis& a, const Launch
     o << "    A.cyc[g] = " << (k.custom_tu ? k.name : std::string("ptowsp_body")) << "(&d, nullptr);\n  }\n}\n";
     ek.source = o.str();
     return ek;
+}
+
+// ---------------------------------------------------------------------------
+// Row-block chains
+// ---------------------------------------------------------------------------
+bool emit_rowblock(const RowBlockChain& c, EmittedKernel& ek) {
+    const int R = c.segs[0].a->rowblock.rows, nslots = static_cast<int>(c.vec.size());
+    // Waves of a workgroup: up to 4 blocks of 16 rows of one task.
+    const int blocks = R / 16, nw = blocks % 4 == 0 ? 4 : blocks % 2 == 0 ? 2 : 1, nt = 64 * nw;
+    // Right operands in LDS, one copy per slot.
+    struct Right {
+        int k = 0, n = 0;
+        size_t off = 0;
+    };
+    std::map<int, Right> right;
+    size_t lds = 0;
+    long mfma = 0;
+    for (const auto& sg : c.segs)
+        for (const auto& op : sg.a->def->ops) {
+            if (op.kind != OpKind::Matmul) continue;
+            const ValueInfo* b = sg.a->by_id[op.operands[1]];
+            const int slot = sg.slot[sg.a->tensor_ordinal[sg.a->param_of[b->id]]];
+            mfma += static_cast<long>(b->rows) / 4 * (b->cols / 16);
+            Right& r = right[slot];
+            if (r.k) {
+                if (r.k != b->rows || r.n != b->cols) return false;
+                continue;
+            }
+            r.k = b->rows;
+            r.n = b->cols;
+            r.off = lds;
+            lds += static_cast<size_t>(r.k) * (r.n + 4);
+        }
+    if (lds * 4 > 150 * 1024 || mfma > 4096) return false;
+    // The chain's values in order, each with its registers, and the lines that
+    // compute them.  cur: the value a slot holds.
+    struct Line {
+        std::string text;
+        std::vector<int> uses;
+        int def = -1;
+    };
+    std::vector<Line> lines;
+    std::vector<int> regs;
+    auto vn = [](int v) { return "v" + std::to_string(v); };
+    auto emit = [&](int cost, std::vector<int> uses, const std::string& type, const std::string& expr) {
+        const int v = static_cast<int>(regs.size());
+        regs.push_back(cost);
+        lines.push_back({"  const " + type + " " + vn(v) + " = " + expr + ";\n", std::move(uses), v});
+        return v;
+    };
+    std::map<int, int> cur;
+    std::ostringstream scalars;
+    size_t barrier = 0;  // line before which the right operands must be in LDS
+    for (size_t si = 0; si < c.segs.size(); ++si) {
+        const RowBlockChain::Seg& sg = c.segs[si];
+        const KernelAnalysis& a = *sg.a;
+        const KernelDef& k = *a.def;
+        const RowBlockInfo& rb = a.rowblock;
+        std::vector<int> val(a.max_id + 1, -1);
+        auto sname = [&](int id) { return "s" + std::to_string(si) + "_" + std::to_string(id); };
+        for (size_t i = 0; i < k.params.size(); ++i)
+            if (!a.by_id[k.params[i].id]->tile)
+                scalars << "  const float " << sname(k.params[i].id) << " = bits_f32(A.scal[" << sg.scal0 + a.scalar_ordinal[i] << "]);\n";
+        for (const auto& op : k.ops)
+            if (op.kind == OpKind::Constant && op.result > 0 && op.has_value)
+                scalars << "  const float " << sname(op.result) << " = " << flt(op.value) << ";\n";
+        auto nb = [&](int id) { return a.by_id[id]->cols / 16; };
+        auto rvt = [&](int n) { return "RV<" + std::to_string(n) + ">"; };
+        auto is_full = [&](RowClass x) { return x == RowClass::Full || x == RowClass::ColVec || x == RowClass::ColVecT; };
+        // The value of param `id` as its slot holds it now.
+        auto read = [&](int id) {
+            const int s = sg.slot[a.tensor_ordinal[a.param_of[id]]];
+            auto it = cur.find(s);
+            if (it != cur.end()) return it->second;
+            const std::string p = "P" + std::to_string(s), s3 = "A.s3[" + std::to_string(s) + "]", s4 = "A.s4[" + std::to_string(s) + "]";
+            const std::string vec = c.vec[s] ? "true" : "false";
+            int v = -1;
+            switch (rb.cls[id]) {
+                case RowClass::Full:
+                    v = emit(4 * nb(id), {}, rvt(nb(id)), "rv_load<" + std::to_string(nb(id)) + ", " + vec + ">(" + p + " + r0 * " + s3 + ", " + s3 + ", " + s4 + ")");
+                    break;
+                case RowClass::ColVec:  // every row reads the same one
+                    v = emit(4 * nb(id), {}, rvt(nb(id)), "rv_load<" + std::to_string(nb(id)) + ", false>(" + p + ", 0, " + s4 + ")");
+                    break;
+                case RowClass::ColVecT: {
+                    const int n = a.by_id[id]->rows / 16;
+                    v = emit(4 * n, {}, rvt(n), "rv_load<" + std::to_string(n) + ", false>(" + p + ", 0, " + s3 + ")");
+                    break;
+                }
+                case RowClass::RowVec: v = emit(1, {}, "float", p + "[(r0 + row) * " + s3 + "]"); break;
+                default: v = emit(1, {}, "float", p + "[(r0 + row) * " + s4 + "]"); break;  // RowVecT
+            }
+            // Broadcast vectors are not a slot's [rows, n] value.
+            if (rb.cls[id] == RowClass::Full || rb.cls[id] == RowClass::RowVec) cur[s] = v;
+            return v;
+        };
+        // Preloaded params hold their value at the launch's start for the whole task.
+        for (const auto& p : k.params)
+            if (a.by_id[p.id]->tile && a.preload[p.id]) val[p.id] = read(p.id);
+        if (si == 0) {
+            for (const auto& op : k.ops)  // a left operand read from memory: ahead of the barrier too
+                if (op.kind == OpKind::Matmul && a.param_of[op.operands[0]] >= 0) read(op.operands[0]);
+            barrier = lines.size();
+        }
+        auto get = [&](int id) { return val[id] >= 0 ? val[id] : read(id); };
+        auto arg = [&](int id) { return a.by_id[id]->tile ? vn(get(id)) : sname(id); };
+        for (size_t oi = 0; oi < k.ops.size(); ++oi) {
+            const auto& op = k.ops[oi];
+            std::vector<int> uses;
+            auto use = [&](int id) {
+                if (a.by_id[id]->tile) uses.push_back(get(id));
+                return arg(id);
+            };
+            switch (op.kind) {
+                case OpKind::Constant: case OpKind::CpuSimAddCycles: break;
+                case OpKind::Load: val[op.result] = read(op.operands[0]); break;
+                case OpKind::TMov: val[op.result] = get(op.operands[0]); break;
+                case OpKind::Store: {
+                    const int d = op.operands[0], s = sg.slot[a.tensor_ordinal[a.param_of[d]]], v = get(op.operands[1]);
+                    const std::string p = "P" + std::to_string(s), s3 = "A.s3[" + std::to_string(s) + "]", s4 = "A.s4[" + std::to_string(s) + "]";
+                    if (rb.cls[d] == RowClass::Full)
+                        lines.push_back({"  rv_store<" + std::to_string(nb(d)) + ", " + (c.vec[s] ? "true" : "false") + ">(" + p + " + r0 * " + s3 + ", " + s3 +
+                                             ", " + s4 + ", " + vn(v) + ");\n",
+                                         {v}, -1});
+                    else
+                        lines.push_back({"  if (lane < 16) " + p + "[(r0 + row) * " + s3 + "] = " + vn(v) + ";\n", {v}, -1});
+                    cur[s] = v;
+                    break;
+                }
+                case OpKind::Matmul: {
+                    const int x = op.operands[0], y = op.operands[1];
+                    const Right& r = right[sg.slot[a.tensor_ordinal[a.param_of[y]]]];
+                    const std::string xa = use(x);
+                    val[op.result] = emit(r.n / 4, uses, rvt(r.n / 16), "rv_matmul<" + std::to_string(r.k / 16) + ", " + std::to_string(r.n / 16) + ", " +
+                                                                            std::to_string(r.n + 4) + ">(" + xa + ", lb + " + std::to_string(r.off) + ")");
+                    break;
+                }
+                case OpKind::Add: case OpKind::Sub: case OpKind::Mul: case OpKind::Div: case OpKind::Max: case OpKind::Min: {
+                    int x = op.operands[0], y = op.operands[1];
+                    // As the other families: a scalar left operand keeps its side only for Div.
+                    if (a.bin_mode[oi] == BinMode::ScalarLeft && op.kind != OpKind::Div) std::swap(x, y);
+                    const std::string xa = use(x), ya = use(y);
+                    const bool full = is_full(rb.cls[op.result]);
+                    val[op.result] = full ? emit(4 * nb(op.result), uses, rvt(nb(op.result)), std::string("rv_ew<") + op_functor(op.kind) + ">(" + xa + ", " + ya + ")")
+                                          : emit(1, uses, "float", std::string(op_functor(op.kind)) + "::f(" + xa + ", " + ya + ")");
+                    break;
+                }
+                case OpKind::Exp:
+                case OpKind::Rsqrt: {
+                    const std::string xa = use(op.operands[0]);
+                    const bool full = is_full(rb.cls[op.result]), ex = op.kind == OpKind::Exp;
+                    val[op.result] = full ? emit(4 * nb(op.result), uses, rvt(nb(op.result)), std::string(ex ? "rv_exp(" : "rv_rsqrt(") + xa + ")")
+                                          : emit(1, uses, "float", std::string(ex ? "expf(" : "rsqrt_cr(") + xa + ")");
+                    break;
+                }
+                case OpKind::RowSum:
+                case OpKind::RowMax:
+                case OpKind::RowMean: {
+                    const std::string xa = use(op.operands[0]);
+                    std::string e = std::string(op.kind == OpKind::RowMax ? "rv_max(" : "rv_sum(") + xa + ")";
+                    if (op.kind == OpKind::RowMean) e += " / " + flt(static_cast<double>(a.by_id[op.operands[0]]->cols));
+                    val[op.result] = emit(1, uses, "float", e);
+                    break;
+                }
+                default: return false;
+            }
+        }
+    }
+    // Registers live at once (a wave has 512; half of them leave room for the
+    // products' operands, addresses and a second wave).
+    std::vector<int> last(regs.size(), -1);
+    for (size_t i = 0; i < lines.size(); ++i)
+        for (int v : lines[i].uses) last[v] = static_cast<int>(i);
+    int live = 0, most = 0;
+    for (size_t i = 0; i < lines.size(); ++i) {
+        if (lines[i].def >= 0) live += regs[lines[i].def];
+        most = std::max(most, live);
+        if (lines[i].def >= 0 && last[lines[i].def] < 0) live -= regs[lines[i].def];
+        std::set<int> u(lines[i].uses.begin(), lines[i].uses.end());
+        for (int v : u)
+            if (last[v] == static_cast<int>(i)) live -= regs[v];
+    }
+    if (most > 224) return false;
+
+    std::ostringstream o;
+    o << "#include \"ptowsp_device.h\"\nusing namespace ptowsp;\n// row-block program: kernels";
+    for (const auto& sg : c.segs) o << " " << sg.a->def->name;
+    o << ", " << R << " rows\n";
+    ek = EmittedKernel();
+    ek.entry = entry_name("block", *c.segs[0].a->def);
+    ek.threads = nt;
+    ek.blocks_per_task = blocks / nw;
+    ek.lds_bytes = lds * 4;
+    o << "extern \"C\" __global__ void __launch_bounds__(" << nt << ") " << ek.entry << "(const LaunchArgs A) {\n";
+    if (lds) o << "  __shared__ __attribute__((aligned(16))) float lb[" << lds << "];\n";
+    o << "  const int lane = threadIdx.x & 63, row = lane & 15, wave = wave_index();\n  (void)row; (void)lane;\n";
+    o << scalars.str();
+    o << "  i64 vars[" << std::max(1, c.ng) << "];\n  (void)vars;\n";
+    // A workgroup's rows are nw blocks of 16 of one task (fewer than 2^31 workgroups).
+    o << "  u32 q_ = blockIdx.x;\n";
+    o << "  const i64 r0 = ((q_ % " << ek.blocks_per_task << "u) * " << nw << " + wave) * 16; q_ /= " << ek.blocks_per_task << "u;\n";
+    for (int v = c.ng - 1; v >= 0; --v)
+        o << "  { const u32 e_ = static_cast<u32>(A.ext[" << v << "]); vars[" << v << "] = q_ % e_; q_ /= e_; }\n";
+    for (int s = 0; s < nslots; ++s)
+        o << "  float* const P" << s << " = reinterpret_cast<float*>(A.base[" << s << "]) + (" << offset_expr(s, c.ng, 0, 0) << ");\n";
+    for (const auto& [s, r] : right)
+        o << "  rv_stage<" << r.k << ", " << r.n << ", " << r.n + 4 << ", " << c.stage_mode[s] << ", " << nt << ">(lb + " << r.off << ", P" << s << ", A.s3["
+          << s << "], A.s4[" << s << "]);\n";
+    for (size_t i = 0; i < lines.size(); ++i) {
+        if (i == barrier && lds) o << "  __syncthreads();\n";
+        o << lines[i].text;
+    }
+    o << "}\n";
+    ek.source = o.str();
+    return true;
 }
 
 EmittedKernel emit_launch(const Module& m, const KernelAnalysis& a, const LaunchSpec& L, const EmitSpec& spec) {

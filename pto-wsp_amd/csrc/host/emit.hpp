@@ -88,6 +88,7 @@ struct EmittedKernel {
     int waves_per_block = 4;
     bool row_program = false;
     int part_floats = 0;        // decode: floats per partial (m, l, o of one unit)
+    int blocks_per_task = 1;    // row blocks: workgroups per task
     size_t lds_bytes = 0;
     // Tile programs: bytes of global scratch per workgroup for the tiles that
     // do not fit in LDS (base[ntens] of the launch; the grid is capped so
@@ -96,6 +97,26 @@ struct EmittedKernel {
 };
 
 EmittedKernel emit_launch(const Module& m, const KernelAnalysis& a, const LaunchSpec& L, const EmitSpec& spec);
+
+// A chain of launches over the same grid whose rows are independent
+// (RowBlockInfo), run as one kernel of row blocks.  Params that are the same
+// view share a slot: what one launch stores, the next reads from registers.
+struct RowBlockChain {
+    struct Seg {
+        const KernelAnalysis* a = nullptr;
+        std::vector<int> slot;  // tensor ordinal -> slot
+        int scal0 = 0;          // its first scalar argument
+    };
+    std::vector<Seg> segs;
+    int ng = 0;                      // grid loop variables
+    std::vector<bool> vec;           // slot: unit columns, 16-byte aligned rows
+    std::vector<int> stage_mode;     // slot: how rv_stage reads it as a right operand
+};
+
+// Emits the kernel of a chain; false when its values need more registers, or
+// its right operands more LDS, than a wave or workgroup has to give, or its
+// products more code than the instruction cache holds.
+bool emit_rowblock(const RowBlockChain& c, EmittedKernel& ek);
 
 // Parameters of the row-program layout for a row of `cols` floats with
 // accesses `vw` wide: lanes per row G, chunks per lane NV, unrolled passes UP.

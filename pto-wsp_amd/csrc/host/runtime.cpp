@@ -64,6 +64,13 @@ struct LaunchCache {
     std::map<std::string, EmittedKernel> emitted;
 };
 
+// A row-block chain of this program: its kernel, or that it has none.
+struct ChainEntry {
+    bool ok = false;
+    EmittedKernel ek;
+    const JitKernel* jk = nullptr;
+};
+
 }  // namespace
 
 struct ptowsp_program {
@@ -71,6 +78,7 @@ struct ptowsp_program {
     std::vector<KernelAnalysis> ka;
     Plan plan;
     std::vector<LaunchCache> cache;
+    std::map<std::string, ChainEntry> chains;  // by launches, slots and access modes
     std::vector<bool> tensor_written;
     std::vector<void*> stage_buf;
     std::vector<size_t> stage_bytes;
@@ -1440,6 +1448,153 @@ bool enqueue_decode_folded(RunEnv& E, int li, int lj, hipStream_t stream, uint64
     return true;
 }
 
+// Launches items[i], items[i+1], ... as one kernel of row blocks (RowBlockChain)
+// where they are consecutive launches over the same grid, at least one of
+// them with matmuls, and no memory links them except row by row: a tensor
+// that one of them writes is touched by any of them only through the very
+// same view, and not as a right operand.  In the llama example's block
+// (attention, add, rmsnorm, MLP, add over 8192 tokens) the five launches took
+// 68 us, 21 and 40 of them the two tile programs; one chain takes 18.
+// Returns the number of items launched (0: none).
+size_t enqueue_rowblock(RunEnv& E, const std::vector<PlanItem>& items, size_t i0, hipStream_t stream, uint64_t& launches) {
+    ptowsp_program* P = E.P;
+    if (!tuning().tile_mma) return 0;
+    auto usable = [&](const PlanItem& it, const LaunchSpec* first, int rows) {
+        if (it.ctl || it.is_loop) return false;
+        const LaunchSpec& L = P->plan.launches[it.launch];
+        const RowBlockInfo& rb = P->ka[L.kernel].rowblock;
+        if (!rb.ok || !L.inner.empty() || !L.masks.empty()) return false;
+        return !first || (L.grid.size() == first->grid.size() && rb.rows == rows);
+    };
+    if (!usable(items[i0], nullptr, 0)) return 0;
+    const LaunchSpec& L0 = P->plan.launches[items[i0].launch];
+    const int ng = static_cast<int>(L0.grid.size()), rows = P->ka[L0.kernel].rowblock.rows;
+    size_t n = 1, last_mm = P->ka[L0.kernel].rowblock.matmul ? 1 : 0;
+    while (i0 + n < items.size() && usable(items[i0 + n], &L0, rows)) {
+        ++n;
+        if (P->ka[P->plan.launches[items[i0 + n - 1].launch].kernel].rowblock.matmul) last_mm = n;
+    }
+    if (!last_mm) return 0;
+    // Build the launches; the chain ends before one that does not fit it.
+    std::vector<BuiltLaunch> B;
+    B.reserve(n);
+    for (size_t j = 0; j < n; ++j) {
+        BuiltLaunch b = build_launch(E, P->plan.launches[items[i0 + j].launch]);
+        bool ok = b.ntasks > 0 && b.host_checked && !b.spec.serial && b.ntasks * (rows / 16) < (int64_t(1) << 31);
+        for (int v = 0; v < ng && ok; ++v) ok = j == 0 || b.args.ext[v] == B[0].args.ext[v];
+        if (!ok) break;
+        B.push_back(std::move(b));
+    }
+    struct Slot {
+        int tid, launch, p, rows, cols;
+        bool written = false, right = false, row = false;  // stored; a right operand; read or written row by row
+    };
+    for (size_t len = B.size(); len > 0; --len) {
+        bool mm = false;
+        for (size_t j = 0; j < len; ++j) mm = mm || P->ka[P->plan.launches[items[i0 + j].launch].kernel].rowblock.matmul;
+        if (!mm) return 0;
+        RowBlockChain chain;
+        chain.ng = ng;
+        std::vector<Slot> slots;
+        LaunchArgs A{};
+        int nscal = 0;
+        bool ok = true;
+        std::ostringstream key;
+        for (size_t j = 0; j < len && ok; ++j) {
+            const int li = items[i0 + j].launch;
+            const LaunchSpec& L = P->plan.launches[li];
+            const KernelAnalysis& a = P->ka[L.kernel];
+            const LaunchArgs& X = B[j].args;
+            RowBlockChain::Seg sg;
+            sg.a = &a;
+            sg.scal0 = nscal;
+            key << li << ":";
+            for (size_t p = 0; p < a.tensor_param_index.size() && ok; ++p) {
+                const int id = a.def->params[a.tensor_param_index[p]].id;
+                const ValueInfo* v = a.by_id[id];
+                int s = -1;
+                for (size_t q = 0; q < slots.size() && s < 0; ++q) {
+                    const Slot& t = slots[q];
+                    if (t.tid != L.targs[p]->tid || t.rows != v->rows || t.cols != v->cols) continue;
+                    if (A.base[q] != X.base[p] || A.s3[q] != X.s3[p] || A.s4[q] != X.s4[p]) continue;
+                    bool same = true;
+                    for (int g = 0; g < ng; ++g) same = same && A.coef[q][g] == X.coef[p][g];
+                    if (same) s = static_cast<int>(q);
+                }
+                if (s < 0) {
+                    s = static_cast<int>(slots.size());
+                    if (s >= kMaxParams) {
+                        ok = false;
+                        break;
+                    }
+                    slots.push_back({L.targs[p]->tid, static_cast<int>(j), static_cast<int>(p), v->rows, v->cols});
+                    A.base[s] = X.base[p];
+                    A.s3[s] = X.s3[p];
+                    A.s4[s] = X.s4[p];
+                    A.span[s] = X.span[p];
+                    bool aligned = reinterpret_cast<uintptr_t>(X.base[p]) % 16 == 0;
+                    for (int g = 0; g < ng; ++g) {
+                        A.coef[s][g] = X.coef[p][g];
+                        aligned = aligned && X.coef[p][g] % 4 == 0;
+                    }
+                    chain.vec.push_back(aligned && X.s4[p] == 1 && X.s3[p] % 4 == 0);
+                    chain.stage_mode.push_back(chain.vec.back() ? 0 : aligned && X.s3[p] == 1 && X.s4[p] % 4 == 0 ? 1 : 2);
+                }
+                Slot& t = slots[s];
+                t.written = t.written || a.stored[p];
+                t.right = t.right || a.rowblock.right[p];
+                t.row = t.row || a.rowblock.cls[id] != RowClass::None;
+                // A vector broadcast over the rows is read by all of them.
+                if (a.rowblock.cls[id] == RowClass::ColVec || a.rowblock.cls[id] == RowClass::ColVecT) t.right = true;
+                sg.slot.push_back(s);
+                key << s << ",";
+            }
+            const size_t ns = L.task->scalar_args.size();
+            if (nscal + ns > static_cast<size_t>(kMaxScalars)) ok = false;
+            for (size_t q = 0; q < ns && ok; ++q) A.scal[nscal + q] = X.scal[q];
+            nscal += static_cast<int>(ns);
+            chain.segs.push_back(std::move(sg));
+        }
+        // Row-by-row dependences only.
+        for (size_t s = 0; s < slots.size() && ok; ++s) {
+            if (!slots[s].written) continue;
+            if (slots[s].right) ok = false;
+            const TensorState& T = E.ts[slots[s].tid];
+            for (size_t q = 0; q < slots.size() && ok; ++q) {
+                const TensorState& U = E.ts[slots[q].tid];
+                if (q != s && T.dev < U.dev + U.span * 4 && U.dev < T.dev + T.span * 4) ok = false;
+            }
+        }
+        if (!ok) continue;
+        for (size_t s = 0; s < slots.size(); ++s) key << (chain.vec[s] ? "v" : "s") << chain.stage_mode[s];
+        ChainEntry& e = P->chains.emplace(key.str(), ChainEntry{}).first->second;
+        if (!e.ok && e.ek.entry.empty()) {
+            e.ok = emit_rowblock(chain, e.ek);
+            if (!e.ok) e.ek.entry = "-";  // refused: remembered
+        }
+        if (!e.ok) continue;
+        if (!e.jk) {
+            if (E.nscratch) {
+                e.jk = jit_loaded(e.ek.source, e.ek.entry);
+                if (!e.jk)
+                    throw std::runtime_error("ptowsp_hip_launch_noalloc: the kernel of launch " + std::to_string(items[i0].launch) +
+                                             " is not loaded yet; run the program once through ptowsp_hip_launch, "
+                                             "which builds and loads its kernels");
+            } else {
+                e.jk = &jit_kernel(e.ek.source, e.ek.entry);
+            }
+        }
+        for (int v = 0; v < ng; ++v) A.ext[v] = B[0].args.ext[v];
+        A.ntasks = B[0].ntasks;
+        A.err = B[0].args.err;
+        void* params[] = {&A};
+        launch_kernel(E, e.jk->function, B[0].ntasks * e.ek.blocks_per_task, e.ek.threads, 0, stream, params, "hipModuleLaunchKernel(row blocks)");
+        ++launches;
+        return len;
+    }
+    return 0;
+}
+
 void run_host_step(RunEnv& E, const PlanItem& it, hipStream_t stream, uint64_t& launches);
 
 void run_items(RunEnv& E, const std::vector<PlanItem>& items, hipStream_t stream, uint64_t& launches) {
@@ -1450,6 +1605,10 @@ void run_items(RunEnv& E, const std::vector<PlanItem>& items, hipStream_t stream
             continue;
         }
         if (!it.is_loop) {
+            if (const size_t n = enqueue_rowblock(E, items, i, stream, launches)) {
+                i += n - 1;
+                continue;
+            }
             if (i + 1 < items.size() && !items[i + 1].is_loop && !items[i + 1].ctl &&
                 enqueue_decode_folded(E, it.launch, items[i + 1].launch, stream, launches)) {
                 ++i;
@@ -1954,6 +2113,25 @@ int ptowsp_hip_precompile(ptowsp_program* P, int index, int flags, const char** 
             if (spec.gemm && (spec.gemm_bm % 64 || spec.gemm_bn % 64)) {
                 spec.gemm = spec.gemm_pingpong = false;
                 spec.gemm_vm = spec.gemm_vn = -1;
+            }
+            if ((flags & 64) && a.rowblock.ok && a.rowblock.matmul && L.inner.empty()) {
+                // The launch alone as row blocks, every param a view of its own.
+                RowBlockChain chain;
+                chain.ng = ng;
+                RowBlockChain::Seg sg;
+                sg.a = &a;
+                for (size_t p = 0; p < a.tensor_param_index.size(); ++p) {
+                    sg.slot.push_back(static_cast<int>(p));
+                    chain.vec.push_back(true);
+                    chain.stage_mode.push_back(0);
+                }
+                chain.segs.push_back(std::move(sg));
+                EmittedKernel ek;
+                if (emit_rowblock(chain, ek)) {
+                    (void)jit_compile(ek.source);
+                    if (static_cast<int>(li) == index) P->precompiled_source = ek.source;
+                    continue;
+                }
             }
             const EmittedKernel& ek = emitted_for(P, static_cast<int>(li), spec);
             (void)jit_compile(ek.source);
