@@ -1478,11 +1478,37 @@ EmittedKernel emit_custom(const Module& m, const KernelAnalysis& a, const Launch
     return ek;
 }
 
+// One line of a chain's kernel: its text, the values it reads and the one it
+// defines (-1: none).
+struct ChainLine {
+    std::string text;
+    std::vector<int> uses;
+    int def = -1;
+};
+
+// Most registers live at once (regs: per value).
+static int most_live(const std::vector<ChainLine>& lines, const std::vector<int>& regs) {
+    std::vector<int> last(regs.size(), -1);
+    for (size_t i = 0; i < lines.size(); ++i)
+        for (int v : lines[i].uses) last[v] = static_cast<int>(i);
+    int live = 0, most = 0;
+    for (size_t i = 0; i < lines.size(); ++i) {
+        const int d = lines[i].def;
+        if (d >= 0) live += regs[d];
+        most = std::max(most, live);
+        if (d >= 0 && last[d] < 0) live -= regs[d];
+        const std::set<int> u(lines[i].uses.begin(), lines[i].uses.end());
+        for (int v : u)
+            if (last[v] == static_cast<int>(i)) live -= regs[v];
+    }
+    return most;
+}
+
 // ---------------------------------------------------------------------------
 // Row-block chains
 // ---------------------------------------------------------------------------
-bool emit_rowblock(const RowBlockChain& c, EmittedKernel& ek) {
-    const int R = c.segs[0].a->rowblock.rows, nslots = static_cast<int>(c.vec.size());
+bool emit_rowblock(const RowChain& c, EmittedKernel& ek) {
+    const int R = c.segs[0].a->rowblock.rows, nslots = static_cast<int>(c.slots.size());
     // Waves of a workgroup: up to 4 blocks of 16 rows of one task.
     const int blocks = R / 16, nw = blocks % 4 == 0 ? 4 : blocks % 2 == 0 ? 2 : 1, nt = 64 * nw;
     // Right operands in LDS, one copy per slot.
@@ -1512,12 +1538,7 @@ bool emit_rowblock(const RowBlockChain& c, EmittedKernel& ek) {
     if (lds * 4 > 150 * 1024 || mfma > 4096) return false;
     // The chain's values in order, each with its registers, and the lines that
     // compute them.  cur: the value a slot holds.
-    struct Line {
-        std::string text;
-        std::vector<int> uses;
-        int def = -1;
-    };
-    std::vector<Line> lines;
+    std::vector<ChainLine> lines;
     std::vector<int> regs;
     auto vn = [](int v) { return "v" + std::to_string(v); };
     auto emit = [&](int cost, std::vector<int> uses, const std::string& type, const std::string& expr) {
@@ -1530,7 +1551,7 @@ bool emit_rowblock(const RowBlockChain& c, EmittedKernel& ek) {
     std::ostringstream scalars;
     size_t barrier = 0;  // line before which the right operands must be in LDS
     for (size_t si = 0; si < c.segs.size(); ++si) {
-        const RowBlockChain::Seg& sg = c.segs[si];
+        const RowChain::Seg& sg = c.segs[si];
         const KernelAnalysis& a = *sg.a;
         const KernelDef& k = *a.def;
         const RowBlockInfo& rb = a.rowblock;
@@ -1551,7 +1572,7 @@ bool emit_rowblock(const RowBlockChain& c, EmittedKernel& ek) {
             auto it = cur.find(s);
             if (it != cur.end()) return it->second;
             const std::string p = "P" + std::to_string(s), s3 = "A.s3[" + std::to_string(s) + "]", s4 = "A.s4[" + std::to_string(s) + "]";
-            const std::string vec = c.vec[s] ? "true" : "false";
+            const std::string vec = c.slots[s].vec ? "true" : "false";
             int v = -1;
             switch (rb.cls[id]) {
                 case RowClass::Full:
@@ -1597,7 +1618,7 @@ bool emit_rowblock(const RowBlockChain& c, EmittedKernel& ek) {
                     const int d = op.operands[0], s = sg.slot[a.tensor_ordinal[a.param_of[d]]], v = get(op.operands[1]);
                     const std::string p = "P" + std::to_string(s), s3 = "A.s3[" + std::to_string(s) + "]", s4 = "A.s4[" + std::to_string(s) + "]";
                     if (rb.cls[d] == RowClass::Full)
-                        lines.push_back({"  rv_store<" + std::to_string(nb(d)) + ", " + (c.vec[s] ? "true" : "false") + ">(" + p + " + r0 * " + s3 + ", " + s3 +
+                        lines.push_back({"  rv_store<" + std::to_string(nb(d)) + ", " + (c.slots[s].vec ? "true" : "false") + ">(" + p + " + r0 * " + s3 + ", " + s3 +
                                              ", " + s4 + ", " + vn(v) + ");\n",
                                          {v}, -1});
                     else
@@ -1644,21 +1665,9 @@ bool emit_rowblock(const RowBlockChain& c, EmittedKernel& ek) {
             }
         }
     }
-    // Registers live at once (a wave has 512; half of them leave room for the
-    // products' operands, addresses and a second wave).
-    std::vector<int> last(regs.size(), -1);
-    for (size_t i = 0; i < lines.size(); ++i)
-        for (int v : lines[i].uses) last[v] = static_cast<int>(i);
-    int live = 0, most = 0;
-    for (size_t i = 0; i < lines.size(); ++i) {
-        if (lines[i].def >= 0) live += regs[lines[i].def];
-        most = std::max(most, live);
-        if (lines[i].def >= 0 && last[lines[i].def] < 0) live -= regs[lines[i].def];
-        std::set<int> u(lines[i].uses.begin(), lines[i].uses.end());
-        for (int v : u)
-            if (last[v] == static_cast<int>(i)) live -= regs[v];
-    }
-    if (most > 224) return false;
+    // A wave has 512 registers; half of them leave room for the products'
+    // operands, addresses and a second wave.
+    if (most_live(lines, regs) > 224) return false;
 
     std::ostringstream o;
     o << "#include \"ptowsp_device.h\"\nusing namespace ptowsp;\n// row-block program: kernels";
@@ -1682,12 +1691,199 @@ bool emit_rowblock(const RowBlockChain& c, EmittedKernel& ek) {
     for (int s = 0; s < nslots; ++s)
         o << "  float* const P" << s << " = reinterpret_cast<float*>(A.base[" << s << "]) + (" << offset_expr(s, c.ng, 0, 0) << ");\n";
     for (const auto& [s, r] : right)
-        o << "  rv_stage<" << r.k << ", " << r.n << ", " << r.n + 4 << ", " << c.stage_mode[s] << ", " << nt << ">(lb + " << r.off << ", P" << s << ", A.s3["
+        o << "  rv_stage<" << r.k << ", " << r.n << ", " << r.n + 4 << ", " << c.slots[s].stage_mode << ", " << nt << ">(lb + " << r.off << ", P" << s << ", A.s3["
           << s << "], A.s4[" << s << "]);\n";
     for (size_t i = 0; i < lines.size(); ++i) {
         if (i == barrier && lds) o << "  __syncthreads();\n";
         o << lines[i].text;
     }
+    o << "}\n";
+    ek.source = o.str();
+    return true;
+}
+
+// ---------------------------------------------------------------------------
+// Row-program chains
+// ---------------------------------------------------------------------------
+// Every row is a job of its lane team, as in a row program, for all launches
+// of the chain: what it reads it reads once, what it computes stays in
+// registers (a value of each iteration of the loops, which are unrolled), and
+// what it stores is stored once, at the end.
+bool emit_rowchain(const RowChain& c, EmittedKernel& ek) {
+    const KernelAnalysis& a0 = *c.segs[0].a;
+    const int R = a0.rows, C = a0.cols, nslots = static_cast<int>(c.slots.size());
+    const RowLayout lay = row_layout(C, c.vec_width, 1, c.unit_cols);
+    const std::string cm = std::to_string(C), sfx = lay.masked ? "_m" : "";
+    const std::string ntb = c.nontemporal && C % 32 == 0 ? "true" : "false";
+    const std::string nt = lay.masked ? ", " + ntb + ", " + cm : c.nontemporal ? ", true" : "";
+    const std::string nont = lay.masked ? ", false, " + cm : "", cmx = lay.masked ? ", " + cm : "";
+    const int full = lay.nv * lay.vw;
+    std::vector<ChainLine> lines;
+    std::vector<int> regs;
+    auto vn = [](int v) { return "v" + std::to_string(v); };
+    auto emit = [&](bool wide, std::vector<int> uses, const std::string& expr) {
+        const int v = static_cast<int>(regs.size());
+        regs.push_back(wide ? full : 1);
+        lines.push_back({std::string("  const ") + (wide ? "RS " : "float ") + vn(v) + " = " + expr + ";\n", std::move(uses), v});
+        return v;
+    };
+    std::map<std::pair<int, int>, int> cur;  // (slot, iteration) -> value
+    std::map<std::pair<int, int>, std::pair<int, bool>> out;  // stored: value, full row
+    std::ostringstream scalars;
+    for (size_t si = 0; si < c.segs.size(); ++si) {
+        const RowChain::Seg& sg = c.segs[si];
+        const KernelAnalysis& a = *sg.a;
+        const KernelDef& k = *a.def;
+        auto sname = [&](int id) { return "s" + std::to_string(si) + "_" + std::to_string(id); };
+        for (size_t i = 0; i < k.params.size(); ++i) {
+            const ValueInfo* v = a.by_id[k.params[i].id];
+            if (v->tile) continue;
+            if (v->dtype != DType::F32) return false;
+            scalars << "  const float " << sname(v->id) << " = bits_f32(A.scal[" << sg.scal0 + a.scalar_ordinal[i] << "]);\n";
+        }
+        for (const auto& op : k.ops)
+            if (op.kind == OpKind::Constant && op.result > 0 && op.has_value) {
+                if (a.by_id[op.result]->dtype != DType::F32) return false;
+                scalars << "  const float " << sname(op.result) << " = " << flt(op.value) << ";\n";
+            }
+        auto wide = [&](int id) {
+            const RowClass x = a.row_class[id];
+            return x == RowClass::Full || x == RowClass::ColVec || x == RowClass::ColVecT;
+        };
+        for (int it = 0; it < (sg.loops ? c.loop : 1); ++it) {
+            std::vector<int> val(a.max_id + 1, -1);
+            auto at = [&](int slot) { return std::make_pair(slot, c.slots[slot].moves ? it : 0); };
+            // Value `id` of the class it is read as (a param's own, or its Load's).
+            auto read = [&](int param, int id) {
+                const int s = sg.slot[a.tensor_ordinal[a.param_of[param]]];
+                const auto key = at(s);
+                auto f = cur.find(key);
+                if (f != cur.end()) return f->second;
+                std::string p = "P" + std::to_string(s);
+                if (c.slots[s].moves) p = "(" + p + " + " + std::to_string(it) + " * M" + std::to_string(s) + ")";
+                const std::string s3 = "A.s3[" + std::to_string(s) + "]", s4 = "A.s4[" + std::to_string(s) + "]";
+                int v = -1;
+                switch (a.row_class[id]) {
+                    case RowClass::Full:
+                        v = emit(true, {}, "chain_load([&](RS& x_) { row_load" + sfx + "<NV, VW, G" + nt + ">(x_, " + p + " + rr * " + s3 + ", " + s4 + ", j); }, RS())");
+                        break;
+                    case RowClass::ColVec:
+                        v = emit(true, {}, "chain_load([&](RS& x_) { row_load" + sfx + "<NV, VW, G" + nont + ">(x_, " + p + ", " + s4 + ", j); }, RS())");
+                        break;
+                    case RowClass::ColVecT:
+                        v = emit(true, {}, "chain_load([&](RS& x_) { row_load_strided" + sfx + "<NV, VW, G" + cmx + ">(x_, " + p + ", " + s3 + ", j); }, RS())");
+                        break;
+                    case RowClass::RowVec: v = emit(false, {}, p + "[rr * " + s3 + "]"); break;
+                    default: v = emit(false, {}, p + "[rr * " + s4 + "]"); break;
+                }
+                if (a.row_class[id] == RowClass::Full || a.row_class[id] == RowClass::RowVec) cur[key] = v;
+                return v;
+            };
+            for (const auto& p : k.params)
+                if (a.by_id[p.id]->tile && a.preload[p.id]) val[p.id] = read(p.id, p.id);
+            for (size_t oi = 0; oi < k.ops.size(); ++oi) {
+                const auto& op = k.ops[oi];
+                std::vector<int> uses;
+                auto use = [&](int id) {
+                    if (!a.by_id[id]->tile) return sname(id);
+                    uses.push_back(val[id]);
+                    return vn(val[id]);
+                };
+                switch (op.kind) {
+                    case OpKind::Constant: case OpKind::CpuSimAddCycles: break;
+                    case OpKind::Load: val[op.result] = read(op.operands[0], op.result); break;
+                    case OpKind::TMov: val[op.result] = val[op.operands[0]]; break;
+                    case OpKind::Store: {
+                        const int s = sg.slot[a.tensor_ordinal[a.param_of[op.operands[0]]]], v = val[op.operands[1]];
+                        // Row-column shapes of one slot are the same in every launch.
+                        cur[at(s)] = v;
+                        out[at(s)] = {v, a.row_class[op.operands[1]] == RowClass::Full};
+                        break;
+                    }
+                    case OpKind::Add: case OpKind::Sub: case OpKind::Mul: case OpKind::Div: case OpKind::Max: case OpKind::Min: {
+                        const bool left = a.bin_mode[oi] == BinMode::ScalarLeft;
+                        int x = op.operands[0], y = op.operands[1];
+                        if (left && op.kind != OpKind::Div) std::swap(x, y);
+                        const std::string xa = use(x), ya = use(y), F = op_functor(op.kind);
+                        const bool w = wide(op.result);
+                        if (!w) val[op.result] = emit(false, uses, F + "::f(" + xa + ", " + ya + ")");
+                        else if (left && op.kind == OpKind::Div) val[op.result] = emit(true, uses, "ew_sr<OpDiv>(" + xa + ", " + ya + ")");
+                        else if (a.bin_mode[oi] == BinMode::Same || a.bin_mode[oi] == BinMode::ColExpand)
+                            val[op.result] = emit(true, uses, "ew<" + F + ">(" + xa + ", " + ya + ")");
+                        else val[op.result] = emit(true, uses, "ew_rs<" + F + ">(" + xa + ", " + ya + ")");
+                        break;
+                    }
+                    case OpKind::Exp:
+                    case OpKind::Rsqrt: {
+                        const bool w = wide(op.result), ex = op.kind == OpKind::Exp;
+                        const std::string xa = use(op.operands[0]);
+                        val[op.result] = emit(w, uses, (w ? std::string(ex ? "ew_exp(" : "ew_rsqrt(") : std::string(ex ? "expf(" : "rsqrt_cr(")) + xa + ")");
+                        break;
+                    }
+                    case OpKind::RowSum:
+                    case OpKind::RowMax:
+                    case OpKind::RowMean: {
+                        const int x = op.operands[0];
+                        std::string e = use(x);
+                        if (a.row_class[x] == RowClass::Full) {
+                            const bool mx = op.kind == OpKind::RowMax;
+                            if (lay.masked) e = std::string(mx ? "row_max_m" : "row_sum_m") + "<NV, VW, G, " + cm + ">(" + e + ", j)";
+                            else e = mx ? "team_max<G>(lane_max<NV * VW>(" + e + ".v))" : "team_sum<G>(lane_sum<NV * VW>(" + e + ".v))";
+                        }
+                        if (op.kind == OpKind::RowMean) e += " / " + flt(static_cast<double>(a.by_id[x]->cols));
+                        val[op.result] = emit(false, uses, e);
+                        break;
+                    }
+                    default: return false;
+                }
+                if (lines.size() > 1500) return false;
+            }
+        }
+    }
+    for (const auto& [key, vf] : out) {
+        const auto [s, it] = key;
+        const std::string ss = std::to_string(s), v = vn(vf.first);
+        std::string p = "P" + ss;
+        if (c.slots[s].moves) p = "(" + p + " + " + std::to_string(it) + " * M" + ss + ")";
+        const DType dt = c.slots[s].dtype;
+        const std::string dc = std::to_string(dt_code(dt));
+        std::string t;
+        if (vf.second && dt == DType::F32) t = "  if (ok) row_store" + sfx + "<NV, VW, G" + nt + ">(" + p + " + rr * A.s3[" + ss + "], " + v + ", A.s4[" + ss + "], j);\n";
+        else if (vf.second) t = "  if (ok) row_store_h" + sfx + "<NV, VW, G, " + dc + cmx + ">(" + p + " + rr * A.s3[" + ss + "], " + v + ", A.s4[" + ss + "], j);\n";
+        else if (dt == DType::F32) t = "  if (ok && j == 0) " + p + "[rr * A.s3[" + ss + "]] = " + v + ";\n";
+        else t = "  if (ok && j == 0) " + p + "[rr * A.s3[" + ss + "]] = f32_to_h16_bits<" + dc + ">(" + v + ");\n";
+        lines.push_back({t, {vf.first}, -1});
+    }
+    // Registers for at least three waves per SIMD: rows are latency bound.
+    if (most_live(lines, regs) > 128) return false;
+
+    std::ostringstream o;
+    o << "#include \"ptowsp_device.h\"\nusing namespace ptowsp;\n// row chain: kernels";
+    for (const auto& sg : c.segs) o << " " << sg.a->def->name;
+    o << ", rows " << R << " x cols " << C << (c.loop > 1 ? ", " + std::to_string(c.loop) + " iterations" : "") << "\n";
+    ek = EmittedKernel();
+    ek.entry = entry_name("rows", *a0.def);
+    ek.threads = 256;
+    ek.row_program = true;
+    ek.rows_per_chunk = 64 / lay.g;
+    o << "template <class F, class X> __device__ inline X chain_load(F f, X x) { f(x); return x; }\n";
+    o << "extern \"C\" __global__ void __launch_bounds__(256) " << ek.entry << "(const LaunchArgs A) {\n";
+    o << "  constexpr int R = " << R << ", NV = " << lay.nv << ", VW = " << lay.vw << ", G = " << lay.g << ";\n";
+    o << "  typedef RowSlice<NV, VW> RS;\n";
+    o << "  const int lane = threadIdx.x & 63, j = lane % G;\n  (void)j;\n" << scalars.str();
+    // Rows number fewer than 2^31 (checked on the host); a lane past the last
+    // row computes row 0 and stores nothing.
+    o << "  u32 q_ = (blockIdx.x * 4 + (threadIdx.x >> 6)) * " << 64 / lay.g << "u + lane / G;\n";
+    o << "  const bool ok = q_ < static_cast<u32>(A.ntasks) * R;\n  if (!ok) q_ = 0;\n";
+    o << "  const i64 rr = q_ % R; q_ /= R;\n  i64 vars[" << std::max(1, c.ng) << "];\n  (void)vars;\n";
+    for (int v = c.ng - 1; v >= 0; --v)
+        o << "  { const u32 e_ = static_cast<u32>(A.ext[" << v << "]); vars[" << v << "] = q_ % e_; q_ /= e_; }\n";
+    for (int s = 0; s < nslots; ++s) {
+        o << "  " << (c.slots[s].dtype == DType::F32 ? "float" : "u16") << "* const P" << s << " = reinterpret_cast<"
+          << (c.slots[s].dtype == DType::F32 ? "float" : "u16") << "*>(A.base[" << s << "]) + (" << offset_expr(s, c.ng, 0, 0) << ");\n";
+        if (c.slots[s].moves) o << "  const i64 M" << s << " = A.coef[" << s << "][" << c.ng << "];\n";
+    }
+    for (const auto& l : lines) o << l.text;
     o << "}\n";
     ek.source = o.str();
     return true;

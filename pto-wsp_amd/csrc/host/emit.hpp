@@ -98,25 +98,39 @@ struct EmittedKernel {
 
 EmittedKernel emit_launch(const Module& m, const KernelAnalysis& a, const LaunchSpec& L, const EmitSpec& spec);
 
-// A chain of launches over the same grid whose rows are independent
-// (RowBlockInfo), run as one kernel of row blocks.  Params that are the same
-// view share a slot: what one launch stores, the next reads from registers.
-struct RowBlockChain {
+// A chain of launches over the same grid whose rows are independent, run as
+// one kernel.  Params that are the same view share a slot: what one launch
+// stores, the next reads from registers.  With matmuls the chain runs as row
+// blocks (RowBlockInfo, emit_rowblock), without as a row program
+// (emit_rowchain), whose launches may also loop, each `loop` times: over
+// their in-kernel loop, or over an innermost grid variable of their own.
+struct RowChain {
     struct Seg {
         const KernelAnalysis* a = nullptr;
         std::vector<int> slot;  // tensor ordinal -> slot
         int scal0 = 0;          // its first scalar argument
+        bool loops = false;
+    };
+    struct Slot {
+        DType dtype = DType::F32;
+        bool vec = false;        // unit columns, 16-byte aligned rows
+        bool moves = false;      // the loop moves it (coef[slot][ng])
+        bool written = false;
+        int stage_mode = 0;      // how rv_stage reads it as a right operand
     };
     std::vector<Seg> segs;
+    std::vector<Slot> slots;
     int ng = 0;                      // grid loop variables
-    std::vector<bool> vec;           // slot: unit columns, 16-byte aligned rows
-    std::vector<int> stage_mode;     // slot: how rv_stage reads it as a right operand
+    int loop = 1;
+    int vec_width = 1;               // row program: as EmitSpec
+    bool unit_cols = false, nontemporal = false;
 };
 
 // Emits the kernel of a chain; false when its values need more registers, or
 // its right operands more LDS, than a wave or workgroup has to give, or its
-// products more code than the instruction cache holds.
-bool emit_rowblock(const RowBlockChain& c, EmittedKernel& ek);
+// body more code than the instruction cache holds.
+bool emit_rowblock(const RowChain& c, EmittedKernel& ek);
+bool emit_rowchain(const RowChain& c, EmittedKernel& ek);
 
 // Parameters of the row-program layout for a row of `cols` floats with
 // accesses `vw` wide: lanes per row G, chunks per lane NV, unrolled passes UP.

@@ -64,7 +64,7 @@ struct LaunchCache {
     std::map<std::string, EmittedKernel> emitted;
 };
 
-// A row-block chain of this program: its kernel, or that it has none.
+// A chain of this program's launches: its kernel, or that it has none.
 struct ChainEntry {
     bool ok = false;
     EmittedKernel ek;
@@ -1448,106 +1448,157 @@ bool enqueue_decode_folded(RunEnv& E, int li, int lj, hipStream_t stream, uint64
     return true;
 }
 
-// Launches items[i], items[i+1], ... as one kernel of row blocks (RowBlockChain)
-// where they are consecutive launches over the same grid, at least one of
-// them with matmuls, and no memory links them except row by row: a tensor
-// that one of them writes is touched by any of them only through the very
-// same view, and not as a right operand.  In the llama example's block
-// (attention, add, rmsnorm, MLP, add over 8192 tokens) the five launches took
-// 68 us, 21 and 40 of them the two tile programs; one chain takes 18.
+// Launches items[i], items[i+1], ... as one kernel (RowChain) where they are
+// consecutive launches over the same grid whose rows are independent and no
+// memory links them except row by row: a tensor that one of them writes is
+// touched by any of them only through the very same view, and not as a right
+// operand or a vector that all rows read.  Launches with matmuls run as row
+// blocks, also alone; others as a row program, two or more together, which
+// may loop the same number of times (an in-kernel loop, or an innermost grid
+// variable that the others do not have).  The llama example's block
+// (attention, add, rmsnorm, MLP, add over 8192 tokens): five launches 68 us,
+// 21 and 40 of them the two tile programs, one chain 18.  The three-phase
+// softmax example over [8, 4096, 512]: three passes over the data 67 us, one
+// 26 (134 MB, 5.2 TB/s).
 // Returns the number of items launched (0: none).
-size_t enqueue_rowblock(RunEnv& E, const std::vector<PlanItem>& items, size_t i0, hipStream_t stream, uint64_t& launches) {
+size_t enqueue_chain(RunEnv& E, const std::vector<PlanItem>& items, size_t i0, hipStream_t stream, uint64_t& launches) {
     ptowsp_program* P = E.P;
-    if (!tuning().tile_mma) return 0;
-    auto usable = [&](const PlanItem& it, const LaunchSpec* first, int rows) {
-        if (it.ctl || it.is_loop) return false;
-        const LaunchSpec& L = P->plan.launches[it.launch];
-        const RowBlockInfo& rb = P->ka[L.kernel].rowblock;
-        if (!rb.ok || !L.inner.empty() || !L.masks.empty()) return false;
-        return !first || (L.grid.size() == first->grid.size() && rb.rows == rows);
-    };
-    if (!usable(items[i0], nullptr, 0)) return 0;
-    const LaunchSpec& L0 = P->plan.launches[items[i0].launch];
-    const int ng = static_cast<int>(L0.grid.size()), rows = P->ka[L0.kernel].rowblock.rows;
-    size_t n = 1, last_mm = P->ka[L0.kernel].rowblock.matmul ? 1 : 0;
-    while (i0 + n < items.size() && usable(items[i0 + n], &L0, rows)) {
-        ++n;
-        if (P->ka[P->plan.launches[items[i0 + n - 1].launch].kernel].rowblock.matmul) last_mm = n;
+    auto launch = [&](size_t j) -> const LaunchSpec& { return P->plan.launches[items[j].launch]; };
+    auto kernel = [&](size_t j) -> const KernelAnalysis& { return P->ka[launch(j).kernel]; };
+    auto plain = [&](size_t j) { return j < items.size() && !items[j].ctl && !items[j].is_loop && launch(j).masks.empty(); };
+    // The longest run of launches with fitting shapes.  blocks: row blocks
+    // (up to the first launch that is none); rows: a row program.
+    if (!plain(i0)) return 0;
+    const KernelAnalysis& k0 = kernel(i0);
+    size_t nb = 0, nr = 0;
+    bool matmul = false;
+    if (k0.rowblock.ok && tuning().tile_mma)
+        while (plain(i0 + nb) && launch(i0 + nb).inner.empty() && launch(i0 + nb).grid.size() == launch(i0).grid.size() &&
+               kernel(i0 + nb).rowblock.ok && kernel(i0 + nb).rowblock.rows == k0.rowblock.rows) {
+            matmul = matmul || kernel(i0 + nb).rowblock.matmul;
+            ++nb;
+        }
+    // Grid variables that the launches share: those of a launch that loops.
+    size_t ng = launch(i0).grid.size();
+    if (!matmul) {
+        nb = 0;
+        auto row = [&](size_t j) {
+            return plain(j) && kernel(j).family == Family::RowProgram && kernel(j).rows == k0.rows && kernel(j).cols == k0.cols &&
+                   launch(j).inner.size() <= 1;
+        };
+        while (row(i0 + nr)) {
+            const size_t g = launch(i0 + nr).grid.size();
+            if (g + 1 < ng || g > ng + 1) break;
+            if (g + 1 == ng) {
+                // The launches before it have a grid variable more, their loop.
+                bool all = true;
+                for (size_t j = 0; j < nr; ++j) all = all && launch(i0 + j).grid.size() == ng && launch(i0 + j).inner.empty();
+                if (!all) break;
+                ng = g;
+            }
+            ++nr;
+        }
+        if (nr < 2) return 0;
     }
-    if (!last_mm) return 0;
+    const size_t n = matmul ? nb : nr;
     // Build the launches; the chain ends before one that does not fit it.
     std::vector<BuiltLaunch> B;
     B.reserve(n);
+    int64_t loop = 0;  // iterations of the launches that loop
     for (size_t j = 0; j < n; ++j) {
-        BuiltLaunch b = build_launch(E, P->plan.launches[items[i0 + j].launch]);
-        bool ok = b.ntasks > 0 && b.host_checked && !b.spec.serial && b.ntasks * (rows / 16) < (int64_t(1) << 31);
-        for (int v = 0; v < ng && ok; ++v) ok = j == 0 || b.args.ext[v] == B[0].args.ext[v];
+        const LaunchSpec& L = launch(i0 + j);
+        BuiltLaunch b = build_launch(E, L);
+        bool ok = b.ntasks > 0 && b.host_checked && !b.spec.serial && (L.inner.empty() || b.spec.row_loops);
+        for (size_t v = 0; v < ng && ok; ++v) ok = j == 0 || b.args.ext[v] == B[0].args.ext[v];
+        if (ok && (L.grid.size() > ng || !L.inner.empty())) {
+            ok = L.grid.size() + L.inner.size() == ng + 1;
+            const int64_t e = b.args.ext[ng];
+            ok = ok && e >= 1 && e <= 32 && (loop == 0 || loop == e);
+            if (ok) loop = e;
+        }
         if (!ok) break;
         B.push_back(std::move(b));
     }
-    struct Slot {
-        int tid, launch, p, rows, cols;
-        bool written = false, right = false, row = false;  // stored; a right operand; read or written row by row
+    int64_t tasks = 1;
+    for (size_t v = 0; v < ng && !B.empty(); ++v) tasks *= B[0].args.ext[v];
+    if (B.empty() || tasks * k0.rows >= (int64_t(1) << 31) || tasks * std::max(1, k0.rowblock.rows / 16) >= (int64_t(1) << 31)) return 0;
+    struct Place {
+        int tid, rows, cols;
+        bool shared = false;  // a right operand, or a vector that all rows read
     };
+    const int nvars = static_cast<int>(ng) + 1;
     for (size_t len = B.size(); len > 0; --len) {
         bool mm = false;
-        for (size_t j = 0; j < len; ++j) mm = mm || P->ka[P->plan.launches[items[i0 + j].launch].kernel].rowblock.matmul;
-        if (!mm) return 0;
-        RowBlockChain chain;
-        chain.ng = ng;
-        std::vector<Slot> slots;
+        for (size_t j = 0; j < len; ++j) mm = mm || (matmul && kernel(i0 + j).rowblock.matmul);
+        if (!mm && (matmul || len < 2)) return 0;
+        RowChain chain;
+        chain.ng = static_cast<int>(ng);
+        chain.loop = static_cast<int>(std::max<int64_t>(loop, 1));
+        chain.nontemporal = tuning().nontemporal;
+        chain.vec_width = 4;
+        chain.unit_cols = true;
+        std::vector<Place> places;
         LaunchArgs A{};
         int nscal = 0;
         bool ok = true;
         std::ostringstream key;
+        key << (mm ? "b" : "r") << chain.loop << ";";
         for (size_t j = 0; j < len && ok; ++j) {
-            const int li = items[i0 + j].launch;
-            const LaunchSpec& L = P->plan.launches[li];
-            const KernelAnalysis& a = P->ka[L.kernel];
+            const LaunchSpec& L = launch(i0 + j);
+            const KernelAnalysis& a = kernel(i0 + j);
             const LaunchArgs& X = B[j].args;
-            RowBlockChain::Seg sg;
+            const std::vector<RowClass>& cls = mm ? a.rowblock.cls : a.row_class;
+            RowChain::Seg sg;
             sg.a = &a;
             sg.scal0 = nscal;
-            key << li << ":";
+            sg.loops = L.grid.size() > ng || !L.inner.empty();
+            if (!mm) {
+                chain.vec_width = std::min(chain.vec_width, B[j].spec.vec_width);
+                chain.unit_cols = chain.unit_cols && B[j].spec.row_unit_cols;
+            }
+            key << items[i0 + j].launch << ":";
             for (size_t p = 0; p < a.tensor_param_index.size() && ok; ++p) {
                 const int id = a.def->params[a.tensor_param_index[p]].id;
                 const ValueInfo* v = a.by_id[id];
+                auto coef = [&](int g) { return g < static_cast<int>(ng) || sg.loops ? X.coef[p][g] : 0; };
                 int s = -1;
-                for (size_t q = 0; q < slots.size() && s < 0; ++q) {
-                    const Slot& t = slots[q];
-                    if (t.tid != L.targs[p]->tid || t.rows != v->rows || t.cols != v->cols) continue;
+                for (size_t q = 0; q < places.size() && s < 0; ++q) {
+                    if (places[q].tid != L.targs[p]->tid || places[q].rows != v->rows || places[q].cols != v->cols) continue;
                     if (A.base[q] != X.base[p] || A.s3[q] != X.s3[p] || A.s4[q] != X.s4[p]) continue;
                     bool same = true;
-                    for (int g = 0; g < ng; ++g) same = same && A.coef[q][g] == X.coef[p][g];
+                    for (int g = 0; g < nvars; ++g) same = same && A.coef[q][g] == coef(g);
                     if (same) s = static_cast<int>(q);
                 }
                 if (s < 0) {
-                    s = static_cast<int>(slots.size());
+                    s = static_cast<int>(places.size());
                     if (s >= kMaxParams) {
                         ok = false;
                         break;
                     }
-                    slots.push_back({L.targs[p]->tid, static_cast<int>(j), static_cast<int>(p), v->rows, v->cols});
+                    places.push_back({L.targs[p]->tid, v->rows, v->cols});
                     A.base[s] = X.base[p];
                     A.s3[s] = X.s3[p];
                     A.s4[s] = X.s4[p];
                     A.span[s] = X.span[p];
+                    RowChain::Slot t;
+                    t.dtype = v->dtype;
                     bool aligned = reinterpret_cast<uintptr_t>(X.base[p]) % 16 == 0;
-                    for (int g = 0; g < ng; ++g) {
-                        A.coef[s][g] = X.coef[p][g];
-                        aligned = aligned && X.coef[p][g] % 4 == 0;
+                    for (int g = 0; g < nvars; ++g) {
+                        A.coef[s][g] = coef(g);
+                        aligned = aligned && coef(g) % 4 == 0;
                     }
-                    chain.vec.push_back(aligned && X.s4[p] == 1 && X.s3[p] % 4 == 0);
-                    chain.stage_mode.push_back(chain.vec.back() ? 0 : aligned && X.s3[p] == 1 && X.s4[p] % 4 == 0 ? 1 : 2);
+                    t.moves = A.coef[s][ng] != 0;
+                    t.vec = aligned && X.s4[p] == 1 && X.s3[p] % 4 == 0;
+                    t.stage_mode = t.vec ? 0 : aligned && X.s3[p] == 1 && X.s4[p] % 4 == 0 ? 1 : 2;
+                    chain.slots.push_back(t);
                 }
-                Slot& t = slots[s];
-                t.written = t.written || a.stored[p];
-                t.right = t.right || a.rowblock.right[p];
-                t.row = t.row || a.rowblock.cls[id] != RowClass::None;
-                // A vector broadcast over the rows is read by all of them.
-                if (a.rowblock.cls[id] == RowClass::ColVec || a.rowblock.cls[id] == RowClass::ColVecT) t.right = true;
+                chain.slots[s].written = chain.slots[s].written || a.stored[p];
+                RowClass rc = cls[id];
+                for (const auto& op : a.def->ops)
+                    if (op.kind == OpKind::Load && op.operands[0] == id && op.result > 0) rc = cls[op.result];
+                places[s].shared = places[s].shared || (mm && a.rowblock.right[p]) || rc == RowClass::ColVec || rc == RowClass::ColVecT;
                 sg.slot.push_back(s);
-                key << s << ",";
+                key << s << (mm ? "" : chain.slots[s].moves ? "m" : "f") << ",";
             }
             const size_t ns = L.task->scalar_args.size();
             if (nscal + ns > static_cast<size_t>(kMaxScalars)) ok = false;
@@ -1556,20 +1607,33 @@ size_t enqueue_rowblock(RunEnv& E, const std::vector<PlanItem>& items, size_t i0
             chain.segs.push_back(std::move(sg));
         }
         // Row-by-row dependences only.
-        for (size_t s = 0; s < slots.size() && ok; ++s) {
-            if (!slots[s].written) continue;
-            if (slots[s].right) ok = false;
-            const TensorState& T = E.ts[slots[s].tid];
-            for (size_t q = 0; q < slots.size() && ok; ++q) {
-                const TensorState& U = E.ts[slots[q].tid];
-                if (q != s && T.dev < U.dev + U.span * 4 && U.dev < T.dev + T.span * 4) ok = false;
+        for (size_t s = 0; s < places.size() && ok; ++s) {
+            if (!chain.slots[s].written) continue;
+            if (places[s].shared) ok = false;
+            const TensorState& T = E.ts[places[s].tid];
+            for (size_t q = 0; q < places.size() && ok; ++q) {
+                const TensorState& U = E.ts[places[q].tid];
+                if (q != s && T.dev < U.dev + U.span * dtype_size(chain.slots[q].dtype) &&
+                    U.dev < T.dev + T.span * dtype_size(chain.slots[s].dtype))
+                    ok = false;
             }
+            // Over the grid and the loop its elements never repeat: a tile that
+            // the loop leaves in place is one value per task, which a grid
+            // launch over that variable would write from many tasks.
+            if (ok && loop > 0 && A.coef[s][ng] == 0)
+                for (size_t j = 0; j < len && ok; ++j)
+                    for (size_t p = 0; p < chain.segs[j].slot.size() && ok; ++p)
+                        ok = chain.segs[j].slot[p] != static_cast<int>(s) || !chain.segs[j].loops || !launch(i0 + j).inner.empty() ||
+                             !kernel(i0 + j).stored[p];
         }
         if (!ok) continue;
-        for (size_t s = 0; s < slots.size(); ++s) key << (chain.vec[s] ? "v" : "s") << chain.stage_mode[s];
+        if (mm)
+            for (const auto& t : chain.slots) key << (t.vec ? "v" : "s") << t.stage_mode;
+        else
+            key << "vw" << chain.vec_width << (chain.unit_cols ? "u" : "") << (chain.nontemporal ? "n" : "");
         ChainEntry& e = P->chains.emplace(key.str(), ChainEntry{}).first->second;
         if (!e.ok && e.ek.entry.empty()) {
-            e.ok = emit_rowblock(chain, e.ek);
+            e.ok = mm ? emit_rowblock(chain, e.ek) : emit_rowchain(chain, e.ek);
             if (!e.ok) e.ek.entry = "-";  // refused: remembered
         }
         if (!e.ok) continue;
@@ -1584,11 +1648,12 @@ size_t enqueue_rowblock(RunEnv& E, const std::vector<PlanItem>& items, size_t i0
                 e.jk = &jit_kernel(e.ek.source, e.ek.entry);
             }
         }
-        for (int v = 0; v < ng; ++v) A.ext[v] = B[0].args.ext[v];
-        A.ntasks = B[0].ntasks;
+        for (size_t v = 0; v < ng; ++v) A.ext[v] = B[0].args.ext[v];
+        A.ntasks = tasks;
         A.err = B[0].args.err;
         void* params[] = {&A};
-        launch_kernel(E, e.jk->function, B[0].ntasks * e.ek.blocks_per_task, e.ek.threads, 0, stream, params, "hipModuleLaunchKernel(row blocks)");
+        const int64_t blocks = mm ? tasks * e.ek.blocks_per_task : (tasks * k0.rows + 4 * e.ek.rows_per_chunk - 1) / (4 * e.ek.rows_per_chunk);
+        launch_kernel(E, e.jk->function, blocks, e.ek.threads, 0, stream, params, "hipModuleLaunchKernel(chain)");
         ++launches;
         return len;
     }
@@ -1605,7 +1670,7 @@ void run_items(RunEnv& E, const std::vector<PlanItem>& items, hipStream_t stream
             continue;
         }
         if (!it.is_loop) {
-            if (const size_t n = enqueue_rowblock(E, items, i, stream, launches)) {
+            if (const size_t n = enqueue_chain(E, items, i, stream, launches)) {
                 i += n - 1;
                 continue;
             }
@@ -2116,14 +2181,15 @@ int ptowsp_hip_precompile(ptowsp_program* P, int index, int flags, const char** 
             }
             if ((flags & 64) && a.rowblock.ok && a.rowblock.matmul && L.inner.empty()) {
                 // The launch alone as row blocks, every param a view of its own.
-                RowBlockChain chain;
+                RowChain chain;
                 chain.ng = ng;
-                RowBlockChain::Seg sg;
+                RowChain::Seg sg;
                 sg.a = &a;
                 for (size_t p = 0; p < a.tensor_param_index.size(); ++p) {
                     sg.slot.push_back(static_cast<int>(p));
-                    chain.vec.push_back(true);
-                    chain.stage_mode.push_back(0);
+                    RowChain::Slot t;
+                    t.vec = true;
+                    chain.slots.push_back(t);
                 }
                 chain.segs.push_back(std::move(sg));
                 EmittedKernel ek;
