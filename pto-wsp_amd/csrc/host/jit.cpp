@@ -166,10 +166,11 @@ std::vector<char> jit_compile(const std::string& source) {
 }
 
 namespace {
+// The headers and options are hashed once: they are a hundred times a source.
 std::string source_key(const std::string& source) {
-    std::string h = source + "\n" + options_key() + "\n" + kDeviceHeader + kLaunchHeader;
-    if (source.rfind(kTuMarker, 0) == 0) h += std::string(kKernelAbi) + kPtoisaBridge + kStdTypes;
-    return hex64(fnv1a_64(h));
+    static const std::string fixed = hex64(fnv1a_64(options_key() + kDeviceHeader + kLaunchHeader));
+    static const std::string tu = hex64(fnv1a_64(std::string(kKernelAbi) + kPtoisaBridge + kStdTypes));
+    return hex64(fnv1a_64(source + "\n" + fixed + (source.rfind(kTuMarker, 0) == 0 ? tu : "")));
 }
 }  // namespace
 

@@ -59,9 +59,14 @@ struct TensorState {
     bool written = false;
 };
 
+// The kernels of one launch, by what they were specialized on (a few at most).
 struct LaunchCache {
-    std::map<std::string, const JitKernel*> by_spec;
-    std::map<std::string, EmittedKernel> emitted;
+    struct Entry {
+        EmitSpec spec;
+        EmittedKernel ek;
+        const JitKernel* jk = nullptr;
+    };
+    std::vector<std::unique_ptr<Entry>> entries;
 };
 
 // A chain of this program's launches: its kernel, or that it has none.
@@ -142,6 +147,11 @@ struct ptowsp_program {
     int* noalloc_err = nullptr;
     const int32_t* deferred_dev = nullptr;  // device copy of the deferred extent tensors
     bool timed = false;                     // the run recorded ev0 / ev1
+    // Facts about the module, found once.
+    bool dynamic = false;                   // module_is_dynamic
+    bool loads_slots = false, custom = false;
+    bool fixed_tasks = false;               // no run-time extent: the cycle model has one result
+    std::vector<int> extent_tids;           // tensors that hold loop extents
     uint64_t* slot_stage = nullptr;     // pinned: one element read by a slot load
     std::vector<uint64_t> slot_log;     // values of the run's slot loads, in order
     std::vector<uint64_t> slot_start;   // slots when the run started
@@ -152,15 +162,86 @@ struct ptowsp_program {
             if (c.dev) (void)hipFree(c.dev);
         }
         if (slot_stage) (void)hipHostFree(slot_stage);
-        if (scratch) (void)hipFree(scratch);
         if (gtile) (void)hipFree(gtile);
         for (void* b : stage_buf)
             if (b) (void)hipFree(b);
-        if (h_err) (void)hipHostFree(h_err);
         if (key_stage) (void)hipHostFree(key_stage);
-        if (ev0) (void)hipEventDestroy(ev0);
-        if (ev1) (void)hipEventDestroy(ev1);
+        give_back();
     }
+    // Error flag, events and launch scratch, which every program needs for its
+    // first run, pass from one program to the next (hipMalloc and
+    // hipHostMalloc with their frees take about 20 us each, the frees waiting
+    // for the device).  At most kPoolEntries sets wait, with at most
+    // kPoolScratch bytes each, and go back to the device when an allocation
+    // here fails.
+    struct Resources {
+        int dev = -1;
+        int *h_err = nullptr, *d_err = nullptr;
+        hipEvent_t ev0 = nullptr, ev1 = nullptr;
+        void* scratch = nullptr;
+        size_t scratch_bytes = 0;
+    };
+    static constexpr size_t kPoolEntries = 8, kPoolScratch = size_t(8) << 20;
+    struct Pool {
+        std::mutex mu;
+        std::vector<Resources> free;
+    };
+    static Pool& pool() {
+        static Pool* p = new Pool;  // outlives every program, whatever order static objects end in
+        return *p;
+    }
+    static void release(const Resources& r) {
+        if (r.scratch) (void)hipFree(r.scratch);
+        if (r.h_err) (void)hipHostFree(r.h_err);
+        if (r.ev0) (void)hipEventDestroy(r.ev0);
+        if (r.ev1) (void)hipEventDestroy(r.ev1);
+    }
+    int res_dev = -1;  // device of the error flag, events and scratch
+    void take_resources() {
+        int dev = 0;
+        if (hipGetDevice(&dev) != hipSuccess) return;
+        std::lock_guard<std::mutex> lock(pool().mu);
+        auto& f = pool().free;
+        for (size_t i = f.size(); i-- > 0;) {
+            if (f[i].dev != dev) continue;
+            h_err = f[i].h_err;
+            d_err = f[i].d_err;
+            ev0 = f[i].ev0;
+            ev1 = f[i].ev1;
+            scratch = f[i].scratch;
+            scratch_bytes = f[i].scratch_bytes;
+            have_events = true;
+            res_dev = dev;
+            f.erase(f.begin() + static_cast<std::ptrdiff_t>(i));
+            return;
+        }
+    }
+    void give_back() {
+        Resources r{res_dev, h_err, d_err, ev0, ev1, scratch, scratch_bytes};
+        // Only whole sets whose last run has been waited for and ended well: its
+        // counters are at zero.  A stream that was captured may have put the
+        // events and the scratch into a graph, which can outlive the program.
+        const bool keep = res_dev >= 0 && h_err && have_events && !broken && !pending && !captured && scratch_bytes <= kPoolScratch;
+        if (keep) {
+            __atomic_store_n(h_err, 0, __ATOMIC_RELAXED);
+            std::lock_guard<std::mutex> lock(pool().mu);
+            if (pool().free.size() < kPoolEntries) {
+                pool().free.push_back(r);
+                return;
+            }
+        }
+        release(r);
+    }
+    static void drain_pool() {
+        std::vector<Resources> all;
+        {
+            std::lock_guard<std::mutex> lock(pool().mu);
+            all.swap(pool().free);
+        }
+        for (const Resources& r : all) release(r);
+    }
+    bool broken = false;    // a launch or wait failed: its counters and events are in doubt
+    bool captured = false;  // a run was captured, or went through the no-allocation entry point
 };
 
 struct ptowsp_runtime {
@@ -1182,28 +1263,16 @@ BuiltLaunch build_launch(RunEnv& E, const LaunchSpec& L) {
     return B;
 }
 
-std::string spec_key(const EmitSpec& s) {
-    std::ostringstream o;
-    o << "vw" << s.vec_width << (s.row_unit_cols ? "u" : "") << (s.serial ? ";serial" + std::to_string(s.seq_mask) : "") << (s.task_list ? ";tl" : "") << ";up" << s.row_up << (s.nontemporal ? ";nt" : "")
-      << (s.row_loops ? ";rl" : "") << (s.gemm ? ";gemm" : "") << ";m" << s.gemm_vm << ";n" << s.gemm_vn << ";b" << s.gemm_bm << "x" << s.gemm_bn << "x" << s.gemm_kf << "x" << s.gemm_ring
-      << "s" << s.gemm_split << (s.gemm_edge ? ";edge" : "") << (s.gemm_pingpong ? ";pp" : "")
-      << (s.decode ? ";dec" : "")
-      << (s.decode_norm ? ";norm" : "") << (s.tile_mma ? ";mma" : "") << ";t" << s.threads << ";r" << s.decode_ring << ";w" << s.decode_waves << (s.decode_ordered ? ";ord" : "")
-      << ";i";
-    for (int c : s.indirect_count) o << c << ",";
-    o << ";d";
-    for (int c : s.inner_dyn_term) o << c << ",";
-    return o.str();
-}
-
-const EmittedKernel& emitted_for(ptowsp_program* P, int li, const EmitSpec& spec) {
+LaunchCache::Entry& emitted_for(ptowsp_program* P, int li, const EmitSpec& spec) {
     LaunchCache& c = P->cache[li];
-    const std::string key = spec_key(spec);
-    auto it = c.emitted.find(key);
-    if (it != c.emitted.end()) return it->second;
+    for (auto& e : c.entries)
+        if (e->spec == spec) return *e;
     const LaunchSpec& L = P->plan.launches[li];
-    EmittedKernel ek = emit_launch(P->m, P->ka[L.kernel], L, spec);
-    return c.emitted.emplace(key, std::move(ek)).first->second;
+    auto e = std::make_unique<LaunchCache::Entry>();
+    e->spec = spec;
+    e->ek = emit_launch(P->m, P->ka[L.kernel], L, spec);
+    c.entries.push_back(std::move(e));
+    return *c.entries.back();
 }
 
 // Launch shape of a decode kernel: one 256-thread block per CU.  The
@@ -1254,7 +1323,11 @@ char* launch_scratch(RunEnv& E, size_t need) {
         }
         P->scratch = nullptr;
         P->scratch_bytes = 0;
-        check(hipMalloc(&P->scratch, need), "hipMalloc(launch scratch)");
+        if (hipMalloc(&P->scratch, need) != hipSuccess) {
+            (void)hipGetLastError();
+            ptowsp_program::drain_pool();
+            check(hipMalloc(&P->scratch, need), "hipMalloc(launch scratch)");
+        }
         check(hipMemset(P->scratch, 0, kScratchCounters * sizeof(int32_t)), "hipMemset(scratch counters)");
         check(hipDeviceSynchronize(), "hipDeviceSynchronize");
         P->scratch_bytes = need;
@@ -1294,26 +1367,21 @@ void enqueue_decode(RunEnv& E, int li, BuiltLaunch& B, const EmittedKernel& ek, 
 
 void enqueue_built(RunEnv& E, int li, BuiltLaunch& B, hipStream_t stream, uint64_t& launches) {
     ptowsp_program* P = E.P;
-    const EmittedKernel& ek = emitted_for(P, li, B.spec);
-    LaunchCache& c = P->cache[li];
-    const std::string key = spec_key(B.spec);
-    const JitKernel* jk;
-    auto it = c.by_spec.find(key);
-    if (it == c.by_spec.end()) {
+    LaunchCache::Entry& entry = emitted_for(P, li, B.spec);
+    const EmittedKernel& ek = entry.ek;
+    if (!entry.jk) {
         if (E.nscratch) {
             // A no-allocation run loads no code objects (loading allocates).
-            jk = jit_loaded(ek.source, ek.entry);
-            if (!jk)
+            entry.jk = jit_loaded(ek.source, ek.entry);
+            if (!entry.jk)
                 throw std::runtime_error("ptowsp_hip_launch_noalloc: the kernel of launch " + std::to_string(li) +
                                          " is not loaded yet; run the program once through ptowsp_hip_launch, "
                                          "which builds and loads its kernels");
         } else {
-            jk = &jit_kernel(ek.source, ek.entry);
+            entry.jk = &jit_kernel(ek.source, ek.entry);
         }
-        c.by_spec[key] = jk;
-    } else {
-        jk = it->second;
     }
+    const JitKernel* jk = entry.jk;
     if (B.spec.decode) {
         enqueue_decode(E, li, B, ek, *jk, stream, launches);
         return;
@@ -1448,6 +1516,10 @@ bool enqueue_decode_folded(RunEnv& E, int li, int lj, hipStream_t stream, uint64
     return true;
 }
 
+// Launches that a chain had built and did not take, by plan item: the next
+// ones of the same item list use them instead of building them again.
+using ReadyLaunches = std::map<size_t, BuiltLaunch>;
+
 // Launches items[i], items[i+1], ... as one kernel (RowChain) where they are
 // consecutive launches over the same grid whose rows are independent and no
 // memory links them except row by row: a tensor that one of them writes is
@@ -1461,7 +1533,8 @@ bool enqueue_decode_folded(RunEnv& E, int li, int lj, hipStream_t stream, uint64
 // softmax example over [8, 4096, 512]: three passes over the data 67 us, one
 // 26 (134 MB, 5.2 TB/s).
 // Returns the number of items launched (0: none).
-size_t enqueue_chain(RunEnv& E, const std::vector<PlanItem>& items, size_t i0, hipStream_t stream, uint64_t& launches) {
+size_t enqueue_chain(RunEnv& E, const std::vector<PlanItem>& items, size_t i0, hipStream_t stream, uint64_t& launches,
+                     ReadyLaunches& ready) {
     ptowsp_program* P = E.P;
     auto launch = [&](size_t j) -> const LaunchSpec& { return P->plan.launches[items[j].launch]; };
     auto kernel = [&](size_t j) -> const KernelAnalysis& { return P->ka[launch(j).kernel]; };
@@ -1502,14 +1575,15 @@ size_t enqueue_chain(RunEnv& E, const std::vector<PlanItem>& items, size_t i0, h
     }
     const size_t n = matmul ? nb : nr;
     // Build the launches; the chain ends before one that does not fit it.
-    std::vector<BuiltLaunch> B;
-    B.reserve(n);
+    std::vector<const BuiltLaunch*> B;
     int64_t loop = 0;  // iterations of the launches that loop
     for (size_t j = 0; j < n; ++j) {
         const LaunchSpec& L = launch(i0 + j);
-        BuiltLaunch b = build_launch(E, L);
+        auto r = ready.find(i0 + j);
+        if (r == ready.end()) r = ready.emplace(i0 + j, build_launch(E, L)).first;
+        BuiltLaunch& b = r->second;
         bool ok = b.ntasks > 0 && b.host_checked && !b.spec.serial && (L.inner.empty() || b.spec.row_loops);
-        for (size_t v = 0; v < ng && ok; ++v) ok = j == 0 || b.args.ext[v] == B[0].args.ext[v];
+        for (size_t v = 0; v < ng && ok; ++v) ok = j == 0 || b.args.ext[v] == B[0]->args.ext[v];
         if (ok && (L.grid.size() > ng || !L.inner.empty())) {
             ok = L.grid.size() + L.inner.size() == ng + 1;
             const int64_t e = b.args.ext[ng];
@@ -1517,10 +1591,10 @@ size_t enqueue_chain(RunEnv& E, const std::vector<PlanItem>& items, size_t i0, h
             if (ok) loop = e;
         }
         if (!ok) break;
-        B.push_back(std::move(b));
+        B.push_back(&b);
     }
     int64_t tasks = 1;
-    for (size_t v = 0; v < ng && !B.empty(); ++v) tasks *= B[0].args.ext[v];
+    for (size_t v = 0; v < ng && !B.empty(); ++v) tasks *= B[0]->args.ext[v];
     if (B.empty() || tasks * k0.rows >= (int64_t(1) << 31) || tasks * std::max(1, k0.rowblock.rows / 16) >= (int64_t(1) << 31)) return 0;
     struct Place {
         int tid, rows, cols;
@@ -1546,15 +1620,15 @@ size_t enqueue_chain(RunEnv& E, const std::vector<PlanItem>& items, size_t i0, h
         for (size_t j = 0; j < len && ok; ++j) {
             const LaunchSpec& L = launch(i0 + j);
             const KernelAnalysis& a = kernel(i0 + j);
-            const LaunchArgs& X = B[j].args;
+            const LaunchArgs& X = B[j]->args;
             const std::vector<RowClass>& cls = mm ? a.rowblock.cls : a.row_class;
             RowChain::Seg sg;
             sg.a = &a;
             sg.scal0 = nscal;
             sg.loops = L.grid.size() > ng || !L.inner.empty();
             if (!mm) {
-                chain.vec_width = std::min(chain.vec_width, B[j].spec.vec_width);
-                chain.unit_cols = chain.unit_cols && B[j].spec.row_unit_cols;
+                chain.vec_width = std::min(chain.vec_width, B[j]->spec.vec_width);
+                chain.unit_cols = chain.unit_cols && B[j]->spec.row_unit_cols;
             }
             key << items[i0 + j].launch << ":";
             for (size_t p = 0; p < a.tensor_param_index.size() && ok; ++p) {
@@ -1648,9 +1722,9 @@ size_t enqueue_chain(RunEnv& E, const std::vector<PlanItem>& items, size_t i0, h
                 e.jk = &jit_kernel(e.ek.source, e.ek.entry);
             }
         }
-        for (size_t v = 0; v < ng; ++v) A.ext[v] = B[0].args.ext[v];
+        for (size_t v = 0; v < ng; ++v) A.ext[v] = B[0]->args.ext[v];
         A.ntasks = tasks;
-        A.err = B[0].args.err;
+        A.err = B[0]->args.err;
         void* params[] = {&A};
         const int64_t blocks = mm ? tasks * e.ek.blocks_per_task : (tasks * k0.rows + 4 * e.ek.rows_per_chunk - 1) / (4 * e.ek.rows_per_chunk);
         launch_kernel(E, e.jk->function, blocks, e.ek.threads, 0, stream, params, "hipModuleLaunchKernel(chain)");
@@ -1663,6 +1737,7 @@ size_t enqueue_chain(RunEnv& E, const std::vector<PlanItem>& items, size_t i0, h
 void run_host_step(RunEnv& E, const PlanItem& it, hipStream_t stream, uint64_t& launches);
 
 void run_items(RunEnv& E, const std::vector<PlanItem>& items, hipStream_t stream, uint64_t& launches) {
+    ReadyLaunches ready;
     for (size_t i = 0; i < items.size(); ++i) {
         const PlanItem& it = items[i];
         if (it.ctl) {
@@ -1670,13 +1745,17 @@ void run_items(RunEnv& E, const std::vector<PlanItem>& items, hipStream_t stream
             continue;
         }
         if (!it.is_loop) {
-            if (const size_t n = enqueue_chain(E, items, i, stream, launches)) {
+            if (const size_t n = enqueue_chain(E, items, i, stream, launches, ready)) {
                 i += n - 1;
                 continue;
             }
             if (i + 1 < items.size() && !items[i + 1].is_loop && !items[i + 1].ctl &&
                 enqueue_decode_folded(E, it.launch, items[i + 1].launch, stream, launches)) {
                 ++i;
+                continue;
+            }
+            if (auto r = ready.find(i); r != ready.end()) {
+                if (r->second.ntasks > 0) enqueue_built(E, it.launch, r->second, stream, launches);
                 continue;
             }
             enqueue_launch(E, it.launch, stream, launches);
@@ -1794,6 +1873,7 @@ void resolve_tensors(RunEnv& E, hipStream_t stream) {
 
 CycleResult cycles_for(RunEnv& E) {
     ptowsp_program* P = E.P;
+    if (P->fixed_tasks && P->cycles_valid) return P->cycles;
     CycleEnv env;
     env.axis_size = [&](const std::string& n) { return E.ctx->get_axis_size(E.ctx->ctx, n.c_str()); };
     env.symbol_u64 = [&](uint64_t id) { return E.ctx->get_symbol_u64(E.ctx->ctx, id); };
@@ -1845,7 +1925,7 @@ CycleResult cycles_for(RunEnv& E) {
         for (const auto& c : n->kids) walk(c.get());
     };
     walk(P->m.root.get());
-    const bool dynamic = module_is_dynamic(P->m);
+    const bool dynamic = P->dynamic;
     if (!dynamic && P->cycles_valid && P->cycle_key == key.str()) return P->cycles;
     env.index_value = [&](const IndexExpr& e, const std::vector<std::pair<std::string, int64_t>>& vars) {
         return eval_index_host(E, e, vars);
@@ -1895,17 +1975,30 @@ CycleResult cycles_for(RunEnv& E) {
 // device: the cycle-model key reads their contents.
 std::vector<int> device_extent_tensors(RunEnv& E) {
     std::vector<int> out;
+    for (int tid : E.P->extent_tids)
+        if (!E.ts[tid].host) out.push_back(tid);
+    return out;
+}
+
+// What launch_impl and cycles_for need to know of the module (once).
+void note_module(ptowsp_program* P) {
+    P->dynamic = module_is_dynamic(P->m);
+    P->loads_slots = module_loads_slots(P->m);
+    for (const auto& k : P->m.kernels) P->custom |= k.custom;
+    P->fixed_tasks = !P->dynamic && !P->custom;
     std::function<void(const Node*)> walk = [&](const Node* n) {
         if (!n) return;
-        if ((n->kind == NodeKind::ParallelFor || n->kind == NodeKind::ForEach) && n->axis.kind == AxisKind::DynTensor) {
-            const int tid = n->axis.expr.tid;
-            if (!E.ts[tid].host && std::find(out.begin(), out.end(), tid) == out.end()) out.push_back(tid);
+        if (n->kind == NodeKind::Select) P->fixed_tasks = false;
+        if (n->kind == NodeKind::ParallelFor || n->kind == NodeKind::ForEach) {
+            if (n->axis.kind != AxisKind::Dense) P->fixed_tasks = false;
+            if (n->axis.kind == AxisKind::DynTensor &&
+                std::find(P->extent_tids.begin(), P->extent_tids.end(), n->axis.expr.tid) == P->extent_tids.end())
+                P->extent_tids.push_back(n->axis.expr.tid);
         }
         walk(n->body.get());
         for (const auto& c : n->kids) walk(c.get());
     };
-    walk(E.P->m.root.get());
-    return out;
+    walk(P->m.root.get());
 }
 
 // Copies the device extent tensors into pinned memory on `stream` and keeps
@@ -1962,13 +2055,16 @@ int launch_impl(ptowsp_program* P, RuntimeContext* ctx, void* hip_stream, ptowsp
     if (!P || !ctx) throw std::runtime_error("null argument");
     if (P->pending) throw std::runtime_error("Program already started");
     hipStream_t stream = static_cast<hipStream_t>(hip_stream);
-    bool custom = false;
-    for (const auto& k : P->m.kernels) custom |= k.custom;
+    const bool custom = P->custom;
     RunEnv E{P, ctx, {}, {}, {}};
+    P->broken = true;  // until the run is enqueued
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &capture) != hipSuccess) (void)hipGetLastError();
+    P->captured |= noalloc || capture != hipStreamCaptureStatusNone;
     if (noalloc) {
         const char* who = "ptowsp_hip_launch_noalloc: ";
         if (custom) throw std::runtime_error(std::string(who) + "cpp_src kernels read their per-task cycles back through staging memory");
-        if (module_loads_slots(P->m)) throw std::runtime_error(std::string(who) + "slot loads read tensors back through staging memory");
+        if (P->loads_slots) throw std::runtime_error(std::string(who) + "slot loads read tensors back through staging memory");
         for (const auto& L : P->plan.launches)
             if (!L.masks.empty())
                 throw std::runtime_error(std::string(who) + "masked launches upload task lists through staging memory");
@@ -1988,7 +2084,9 @@ int launch_impl(ptowsp_program* P, RuntimeContext* ctx, void* hip_stream, ptowsp
         E.timing = P->have_events;
     } else {
         noalloc_prepare(stream);
+        if (!P->h_err && !P->have_events) P->take_resources();
         if (!P->h_err) {
+            check(hipGetDevice(&P->res_dev), "hipGetDevice");
             check(hipHostMalloc(reinterpret_cast<void**>(&P->h_err), sizeof(int), hipHostMallocMapped | hipHostMallocCoherent),
                   "hipHostMalloc(err)");
             __atomic_store_n(P->h_err, 0, __ATOMIC_RELAXED);
@@ -2009,11 +2107,13 @@ int launch_impl(ptowsp_program* P, RuntimeContext* ctx, void* hip_stream, ptowsp
     P->custom_runs.clear();
     P->readback.clear();
     P->slot_log.clear();
-    P->slot_start.assign(256, 0);
-    for (uint32_t i = 0; i < 256; ++i) P->slot_start[i] = ctx_slot(E, i);
+    if (P->dynamic || P->loads_slots) {
+        P->slot_start.assign(256, 0);
+        for (uint32_t i = 0; i < 256; ++i) P->slot_start[i] = ctx_slot(E, i);
+    }
     // A slot load reads what the kernels before it wrote: the cycle model
     // replays the values the run read, after the run.
-    const bool slot_loads = module_loads_slots(P->m) || custom;
+    const bool slot_loads = P->loads_slots || custom;
     const std::vector<int> dev_ext = device_extent_tensors(E);
     // The extent copies of a no-allocation run sit at the tail of the scratch;
     // its launches may use everything before them.
@@ -2062,6 +2162,7 @@ int launch_impl(ptowsp_program* P, RuntimeContext* ctx, void* hip_stream, ptowsp
     check(hipGetLastError(), "kernel launch");
     P->stream = stream;
     P->pending = true;
+    P->broken = false;
     P->timed = E.timing;
     P->noalloc_run = noalloc;
     P->noalloc_err = E.err;
@@ -2089,6 +2190,7 @@ int ptowsp_hip_compile(const char* module_text, ptowsp_program** out) {
         P->m = parse_module(module_text);
         for (const auto& k : P->m.kernels) P->ka.push_back(analyze_kernel(k));
         P->plan = build_plan(P->m, P->ka);
+        note_module(P.get());
         P->cache.resize(P->plan.launches.size());
         P->tensor_written.assign(P->m.tensors.size(), false);
         for (const auto& L : P->plan.launches) {
@@ -2199,7 +2301,7 @@ int ptowsp_hip_precompile(ptowsp_program* P, int index, int flags, const char** 
                     continue;
                 }
             }
-            const EmittedKernel& ek = emitted_for(P, static_cast<int>(li), spec);
+            const EmittedKernel& ek = emitted_for(P, static_cast<int>(li), spec).ek;
             (void)jit_compile(ek.source);
             if (static_cast<int>(li) == index) P->precompiled_source = ek.source;
         }
@@ -2270,11 +2372,13 @@ int ptowsp_hip_synchronize(ptowsp_program* P, ptowsp_timing* timing) {
             return 0;
         }
         P->pending = false;
+        P->broken = true;  // until the wait has ended well
         check(hipStreamSynchronize(P->stream), "hipStreamSynchronize");
+        P->broken = false;
         if (P->cycles_deferred) {
             P->cycles_deferred = false;
             RunEnv E{P, P->deferred_ctx, P->deferred_ts, {}, {}};
-            E.replay_slots = module_loads_slots(P->m);
+            E.replay_slots = P->loads_slots;
             for (const auto& [tid, off] : P->deferred_tids) {
                 const size_t n = static_cast<size_t>(std::max<int64_t>(E.ts[tid].span, 0));
                 if (P->deferred_dev) {
