@@ -1198,15 +1198,16 @@ __device__ inline RV<NB> rv_matmul(const RV<KB>& a, const float* b) {
 // (a transposed view); 2: any strides.
 template <int K, int N, int LDN, int MODE, int NT>
 __device__ inline void rv_stage(float* dst, const float* p, i64 s3, i64 s4) {
+    const int tid = threadIdx.x % NT;
     if constexpr (MODE == 0) {
 #pragma unroll 8
-        for (int e = threadIdx.x; e < K * N / 4; e += NT) {
+        for (int e = tid; e < K * N / 4; e += NT) {
             const int k = e / (N / 4), n = e % (N / 4) * 4;
             *reinterpret_cast<f32x4v*>(dst + k * LDN + n) = *reinterpret_cast<const f32x4v*>(p + k * s3 + n);
         }
     } else if constexpr (MODE == 1) {
 #pragma unroll 8
-        for (int e = threadIdx.x; e < K * N / 4; e += NT) {
+        for (int e = tid; e < K * N / 4; e += NT) {
             const int n = e / (K / 4), k = e % (K / 4) * 4;
             const f32x4v x = *reinterpret_cast<const f32x4v*>(p + n * s4 + k);
 #pragma unroll
@@ -1214,8 +1215,87 @@ __device__ inline void rv_stage(float* dst, const float* p, i64 s3, i64 s4) {
         }
     } else {
 #pragma unroll 8
-        for (int e = threadIdx.x; e < K * N; e += NT) dst[(e / N) * LDN + e % N] = p[(e / N) * s3 + (e % N) * s4];
+        for (int e = tid; e < K * N; e += NT) dst[(e / N) * LDN + e % N] = p[(e / N) * s3 + (e % N) * s4];
     }
+}
+
+// KS rows of a right operand on their way to LDS, in registers (MODE as
+// rv_stage).
+template <int KS, int N, int LDN, int MODE, int NT>
+struct RvSlice {
+    static constexpr int E = KS * N / 4, C = (E + NT - 1) / NT;
+    f32x4v x[C];
+    __device__ inline void fetch(const float* p, i64 s3, i64 s4) {
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            const int e = threadIdx.x + c * NT;
+            if (E % NT != 0 && e >= E) break;
+            if constexpr (MODE == 1) {
+                x[c] = *reinterpret_cast<const f32x4v*>(p + e / (KS / 4) * s4 + e % (KS / 4) * 4);
+            } else if constexpr (MODE == 0) {
+                x[c] = *reinterpret_cast<const f32x4v*>(p + e / (N / 4) * s3 + e % (N / 4) * 4);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) x[c][i] = p[e / (N / 4) * s3 + (e % (N / 4) * 4 + i) * s4];
+            }
+        }
+    }
+    __device__ inline void put(float* dst) const {
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            const int e = threadIdx.x + c * NT;
+            if (E % NT != 0 && e >= E) break;
+            if constexpr (MODE == 1) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) dst[(e % (KS / 4) * 4 + i) * LDN + e / (KS / 4)] = x[c][i];
+            } else {
+                *reinterpret_cast<f32x4v*>(dst + e / (N / 4) * LDN + e % (N / 4) * 4) = x[c];
+            }
+        }
+    }
+};
+
+// rv_matmul with b in memory, KS rows at a time through two LDS buffers of
+// KS * LDN floats that the whole workgroup (NT threads, the same b) fills: the
+// next rows are fetched while the MFMAs of these run.  The sums have
+// rv_matmul's order.  For right operands that do not fit LDS whole: an MLP of
+// 128 -> 512 -> 128 columns holds 512 KB of weights: the block around it over
+// 8192 tokens in tasks of 64 rows took 318 us with the MLP as a tile program
+// (its tiles in global scratch), 64 us streamed.
+template <int KB, int NB, int LDN, int KS, int MODE, int NT>
+__device__ inline RV<NB> rv_matmul_stream(const RV<KB>& a, float* buf, const float* p, i64 s3, i64 s4) {
+    constexpr int S = 16 * KB / KS;
+    const int lane = threadIdx.x & 63;
+    const int at = 4 * (lane >> 4) * LDN + (lane & 15);
+    RvSlice<KS, 16 * NB, LDN, MODE, NT> sl;
+    sl.fetch(p, s3, s4);
+    __syncthreads();  // the buffers' readers before this product
+    sl.put(buf);
+    __syncthreads();
+    RV<NB> r;
+#pragma unroll
+    for (int n = 0; n < NB; ++n) r.v[n] = f32x4v{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+        if (s + 1 < S) {
+            sl.fetch(p + (s + 1) * KS * s3, s3, s4);
+            __builtin_amdgcn_sched_barrier(0);  // the fetch ahead of the MFMAs
+        }
+        const float* q = buf + (s & 1) * (KS * LDN) + at;
+#pragma unroll
+        for (int j = 0; j < KS / 16; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int n = 0; n < NB; ++n)
+                    r.v[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(q[(16 * j + e) * LDN + 16 * n], a.v[s * (KS / 16) + j][e], r.v[n], 0, 0, 0);
+        if (s + 1 < S) {
+            // The other buffer's readers passed the barrier of the slice before.
+            sl.put(buf + ((s + 1) & 1) * (KS * LDN));
+            __syncthreads();
+        }
+    }
+    return r;
 }
 
 // ---------------------------------------------------------------------------

@@ -1494,12 +1494,16 @@ static int most_live(const std::vector<ChainLine>& lines, const std::vector<int>
     int live = 0, most = 0;
     for (size_t i = 0; i < lines.size(); ++i) {
         const int d = lines[i].def;
-        if (d >= 0) live += regs[d];
-        most = std::max(most, live);
-        if (d >= 0 && last[d] < 0) live -= regs[d];
+        int dying = 0;
         const std::set<int> u(lines[i].uses.begin(), lines[i].uses.end());
         for (int v : u)
-            if (last[v] == static_cast<int>(i)) live -= regs[v];
+            if (last[v] == static_cast<int>(i)) dying += regs[v];
+        // An elementwise result takes its operands' registers one by one.
+        const bool in_place = d >= 0 && lines[i].text.find("= rv_e") != std::string::npos;
+        if (d >= 0) live += regs[d];
+        most = std::max(most, in_place ? live - std::min(dying, regs[d]) : live);
+        if (d >= 0 && last[d] < 0) live -= regs[d];
+        live -= dying;
     }
     return most;
 }
@@ -1510,14 +1514,16 @@ static int most_live(const std::vector<ChainLine>& lines, const std::vector<int>
 bool emit_rowblock(const RowChain& c, EmittedKernel& ek) {
     const int R = c.segs[0].a->rowblock.rows, nslots = static_cast<int>(c.slots.size());
     // Waves of a workgroup: up to 4 blocks of 16 rows of one task.
-    const int blocks = R / 16, nw = blocks % 4 == 0 ? 4 : blocks % 2 == 0 ? 2 : 1, nt = 64 * nw;
-    // Right operands in LDS, one copy per slot.
+    const int blocks = R / 16, nw = blocks % 4 == 0 ? 4 : blocks % 2 == 0 ? 2 : 1;
+    // Right operands in LDS, one copy per slot.  ks: not whole, but ks rows at
+    // a time.
     struct Right {
-        int k = 0, n = 0;
+        int k = 0, n = 0, ks = 0;
         size_t off = 0;
+        size_t floats() const { return static_cast<size_t>(k) * (n + 4); }
     };
     std::map<int, Right> right;
-    size_t lds = 0;
+    bool uniform = false;  // a right operand that all tasks read
     long mfma = 0;
     for (const auto& sg : c.segs)
         for (const auto& op : sg.a->def->ops) {
@@ -1532,10 +1538,35 @@ bool emit_rowblock(const RowChain& c, EmittedKernel& ek) {
             }
             r.k = b->rows;
             r.n = b->cols;
-            r.off = lds;
-            lds += static_cast<size_t>(r.k) * (r.n + 4);
+            uniform = uniform || c.slots[slot].uniform;
         }
-    if (lds * 4 > 150 * 1024 || mfma > 4096) return false;
+    if (mfma > 4096) return false;
+    // Tasks of 16 or 32 rows share a workgroup of 4 waves where they read the
+    // same right operand: it is staged once for all of them, and a workgroup of
+    // one wave could not stream it (16384 tokens of the block below in tasks of
+    // 16 rows: 172 us as tile programs, 61 so).  Without a shared one a
+    // workgroup per task spreads better.
+    const int tpb = uniform && blocks == nw ? 4 / nw : 1, nt = 64 * nw * tpb;
+    // What does not fit in LDS is streamed through two buffers of ks rows, at
+    // most 8192 floats each (32 registers a thread on the way, 4096 cycles of
+    // MFMAs to cover them), the largest first; all of the workgroup reads it.
+    constexpr size_t kLds = 150 * 1024 / 4;
+    size_t lds = 0, buffer = 0;
+    for (;;) {
+        lds = 2 * buffer;
+        Right* big = nullptr;
+        for (auto& [s, r] : right) {
+            if (r.ks) continue;
+            r.off = lds;
+            lds += r.floats() * (c.slots[s].uniform ? 1 : tpb);
+            if ((tpb == 1 || c.slots[s].uniform) && r.n <= 512 && (!big || r.floats() > big->floats())) big = &r;
+        }
+        if (lds <= kLds) break;
+        if (!big || nt != 256) return false;
+        for (int ks = 16; ks <= big->k && ks * big->n <= 8192; ks += 16)
+            if (big->k % ks == 0) big->ks = ks;
+        buffer = std::max(buffer, static_cast<size_t>(big->ks) * (big->n + 4));
+    }
     // The chain's values in order, each with its registers, and the lines that
     // compute them.  cur: the value a slot holds.
     std::vector<ChainLine> lines;
@@ -1547,6 +1578,8 @@ bool emit_rowblock(const RowChain& c, EmittedKernel& ek) {
         lines.push_back({"  const " + type + " " + vn(v) + " = " + expr + ";\n", std::move(uses), v});
         return v;
     };
+    // Of tasks that share a workgroup the last ones may not exist.
+    const std::string act = tpb > 1 ? "if (act) " : "";
     std::map<int, int> cur;
     std::ostringstream scalars;
     size_t barrier = 0;  // line before which the right operands must be in LDS
@@ -1618,20 +1651,30 @@ bool emit_rowblock(const RowChain& c, EmittedKernel& ek) {
                     const int d = op.operands[0], s = sg.slot[a.tensor_ordinal[a.param_of[d]]], v = get(op.operands[1]);
                     const std::string p = "P" + std::to_string(s), s3 = "A.s3[" + std::to_string(s) + "]", s4 = "A.s4[" + std::to_string(s) + "]";
                     if (rb.cls[d] == RowClass::Full)
-                        lines.push_back({"  rv_store<" + std::to_string(nb(d)) + ", " + (c.slots[s].vec ? "true" : "false") + ">(" + p + " + r0 * " + s3 + ", " + s3 +
+                        lines.push_back({"  " + act + "rv_store<" + std::to_string(nb(d)) + ", " + (c.slots[s].vec ? "true" : "false") + ">(" + p + " + r0 * " + s3 + ", " + s3 +
                                              ", " + s4 + ", " + vn(v) + ");\n",
                                          {v}, -1});
                     else
-                        lines.push_back({"  if (lane < 16) " + p + "[(r0 + row) * " + s3 + "] = " + vn(v) + ";\n", {v}, -1});
+                        lines.push_back({"  " + act + "if (lane < 16) " + p + "[(r0 + row) * " + s3 + "] = " + vn(v) + ";\n", {v}, -1});
                     cur[s] = v;
                     break;
                 }
                 case OpKind::Matmul: {
                     const int x = op.operands[0], y = op.operands[1];
-                    const Right& r = right[sg.slot[a.tensor_ordinal[a.param_of[y]]]];
+                    const int s = sg.slot[a.tensor_ordinal[a.param_of[y]]];
+                    const Right& r = right[s];
                     const std::string xa = use(x);
+                    if (r.ks) {
+                        val[op.result] = emit(r.n / 4, uses, rvt(r.n / 16), "rv_matmul_stream<" + std::to_string(r.k / 16) + ", " + std::to_string(r.n / 16) +
+                                                                                ", " + std::to_string(r.n + 4) + ", " + std::to_string(r.ks) + ", " +
+                                                                                std::to_string(c.slots[s].stage_mode) + ", " + std::to_string(nt) + ">(" + xa +
+                                                                                ", lb, P" + std::to_string(s) + ", A.s3[" + std::to_string(s) + "], A.s4[" +
+                                                                                std::to_string(s) + "])");
+                        break;
+                    }
+                    const std::string rows = c.slots[s].uniform || tpb == 1 ? "" : " + part * " + std::to_string(r.floats());
                     val[op.result] = emit(r.n / 4, uses, rvt(r.n / 16), "rv_matmul<" + std::to_string(r.k / 16) + ", " + std::to_string(r.n / 16) + ", " +
-                                                                            std::to_string(r.n + 4) + ">(" + xa + ", lb + " + std::to_string(r.off) + ")");
+                                                                            std::to_string(r.n + 4) + ">(" + xa + ", lb + " + std::to_string(r.off) + rows + ")");
                     break;
                 }
                 case OpKind::Add: case OpKind::Sub: case OpKind::Mul: case OpKind::Div: case OpKind::Max: case OpKind::Min: {
@@ -1677,6 +1720,7 @@ bool emit_rowblock(const RowChain& c, EmittedKernel& ek) {
     ek.entry = entry_name("block", *c.segs[0].a->def);
     ek.threads = nt;
     ek.blocks_per_task = blocks / nw;
+    ek.tasks_per_block = tpb;
     ek.lds_bytes = lds * 4;
     o << "extern \"C\" __global__ void __launch_bounds__(" << nt << ") " << ek.entry << "(const LaunchArgs A) {\n";
     if (lds) o << "  __shared__ __attribute__((aligned(16))) float lb[" << lds << "];\n";
@@ -1684,15 +1728,23 @@ bool emit_rowblock(const RowChain& c, EmittedKernel& ek) {
     o << scalars.str();
     o << "  i64 vars[" << std::max(1, c.ng) << "];\n  (void)vars;\n";
     // A workgroup's rows are nw blocks of 16 of one task (fewer than 2^31 workgroups).
-    o << "  u32 q_ = blockIdx.x;\n";
-    o << "  const i64 r0 = ((q_ % " << ek.blocks_per_task << "u) * " << nw << " + wave) * 16; q_ /= " << ek.blocks_per_task << "u;\n";
+    if (tpb > 1)
+        o << "  const int part = wave / " << nw << ";\n  u32 q_ = blockIdx.x * " << tpb << "u + part;\n  const bool act = q_ < static_cast<u32>(A.ntasks);\n"
+          << "  if (!act) q_ = static_cast<u32>(A.ntasks) - 1;  // a task to read; nothing is stored\n  const i64 r0 = wave % " << nw << " * 16;\n";
+    else
+        o << "  u32 q_ = blockIdx.x;\n"
+          << "  const i64 r0 = ((q_ % " << ek.blocks_per_task << "u) * " << nw << " + wave) * 16; q_ /= " << ek.blocks_per_task << "u;\n";
     for (int v = c.ng - 1; v >= 0; --v)
         o << "  { const u32 e_ = static_cast<u32>(A.ext[" << v << "]); vars[" << v << "] = q_ % e_; q_ /= e_; }\n";
     for (int s = 0; s < nslots; ++s)
         o << "  float* const P" << s << " = reinterpret_cast<float*>(A.base[" << s << "]) + (" << offset_expr(s, c.ng, 0, 0) << ");\n";
-    for (const auto& [s, r] : right)
-        o << "  rv_stage<" << r.k << ", " << r.n << ", " << r.n + 4 << ", " << c.slots[s].stage_mode << ", " << nt << ">(lb + " << r.off << ", P" << s << ", A.s3["
-          << s << "], A.s4[" << s << "]);\n";
+    for (const auto& [s, r] : right) {
+        if (r.ks) continue;
+        const bool own = tpb > 1 && !c.slots[s].uniform;  // of the task's waves only
+        o << "  rv_stage<" << r.k << ", " << r.n << ", " << r.n + 4 << ", " << c.slots[s].stage_mode << ", " << (own ? 64 * nw : nt) << ">(lb + " << r.off;
+        if (own) o << " + part * " << r.floats();
+        o << ", P" << s << ", A.s3[" << s << "], A.s4[" << s << "]);\n";
+    }
     for (size_t i = 0; i < lines.size(); ++i) {
         if (i == barrier && lds) o << "  __syncthreads();\n";
         o << lines[i].text;

@@ -100,6 +100,7 @@ struct EmittedKernel {
     bool row_program = false;
     int part_floats = 0;        // decode: floats per partial (m, l, o of one unit)
     int blocks_per_task = 1;    // row blocks: workgroups per task
+    int tasks_per_block = 1;    // row blocks: tasks per workgroup
     size_t lds_bytes = 0;
     // Tile programs: bytes of global scratch per workgroup for the tiles that
     // do not fit in LDS (base[ntens] of the launch; the grid is capped so
@@ -127,6 +128,7 @@ struct RowChain {
         bool vec = false;        // unit columns, 16-byte aligned rows
         bool moves = false;      // the loop moves it (coef[slot][ng])
         bool written = false;
+        bool uniform = false;    // all tasks read the same tile
         int stage_mode = 0;      // how rv_stage reads it as a right operand
     };
     std::vector<Seg> segs;

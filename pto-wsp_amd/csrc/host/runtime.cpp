@@ -1662,6 +1662,8 @@ size_t enqueue_chain(RunEnv& E, const std::vector<PlanItem>& items, size_t i0, h
                         aligned = aligned && coef(g) % 4 == 0;
                     }
                     t.moves = A.coef[s][ng] != 0;
+                    t.uniform = true;
+                    for (size_t g = 0; g < ng; ++g) t.uniform = t.uniform && (A.coef[s][g] == 0 || B[0]->args.ext[g] <= 1);
                     t.vec = aligned && X.s4[p] == 1 && X.s3[p] % 4 == 0;
                     t.stage_mode = t.vec ? 0 : aligned && X.s3[p] == 1 && X.s4[p] % 4 == 0 ? 1 : 2;
                     chain.slots.push_back(t);
@@ -1702,7 +1704,7 @@ size_t enqueue_chain(RunEnv& E, const std::vector<PlanItem>& items, size_t i0, h
         }
         if (!ok) continue;
         if (mm)
-            for (const auto& t : chain.slots) key << (t.vec ? "v" : "s") << t.stage_mode;
+            for (const auto& t : chain.slots) key << (t.vec ? "v" : "s") << t.stage_mode << (t.uniform ? "u" : "");
         else
             key << "vw" << chain.vec_width << (chain.unit_cols ? "u" : "") << (chain.nontemporal ? "n" : "");
         ChainEntry& e = P->chains.emplace(key.str(), ChainEntry{}).first->second;
@@ -1726,7 +1728,7 @@ size_t enqueue_chain(RunEnv& E, const std::vector<PlanItem>& items, size_t i0, h
         A.ntasks = tasks;
         A.err = B[0]->args.err;
         void* params[] = {&A};
-        const int64_t blocks = mm ? tasks * e.ek.blocks_per_task : (tasks * k0.rows + 4 * e.ek.rows_per_chunk - 1) / (4 * e.ek.rows_per_chunk);
+        const int64_t blocks = mm ? (tasks + e.ek.tasks_per_block - 1) / e.ek.tasks_per_block * e.ek.blocks_per_task : (tasks * k0.rows + 4 * e.ek.rows_per_chunk - 1) / (4 * e.ek.rows_per_chunk);
         launch_kernel(E, e.jk->function, blocks, e.ek.threads, 0, stream, params, "hipModuleLaunchKernel(chain)");
         ++launches;
         return len;
