@@ -1075,7 +1075,9 @@ __device__ inline float cross4_reduce(float x, Op op) {
 // What bounds it: attention tiles of 64 rows at head dim 64 (4 x 16 x 2048)
 // move 134 MB and need 2.1 GFLOP of fp32 MFMA, 22 and 14 us; as a tile
 // program (values in LDS, a workgroup barrier per op, sequential row
-// reductions on 64 of 256 threads) 86 us, as row blocks 38 us.
+// reductions on 64 of 256 threads) 86 us, as row blocks 34 us: a CU's four
+// workgroups load, compute and store in step, so the two times add up more
+// than they overlap.
 template <int NB>
 struct RV {
     f32x4v v[NB];
@@ -1175,6 +1177,36 @@ __device__ inline float rv_max(const RV<NB>& a) {
     return cross4_reduce(m, [](float x, float y) { return y > x ? y : x; });
 }
 
+// r += columns 16*J0 .. 16*(J0 + KB) - 1 of a times KB*16 rows of b, which
+// start at q (the lane's element) in LDS.  The right operand is read a group
+// of 8 MFMAs (256 cycles) ahead: left to itself the compiler reads two
+// elements, waits for them and issues their two MFMAs, and a wave that has its
+// SIMD to itself spends half of its time in those waits.  Llama block of 8192
+// tokens, width 128, MLP 512: 64 us so, 52 read ahead; attention tiles of 32
+// rows at head dim 64 (134 MB): 32 and 24 us.
+template <int J0, int KB, int LDN, int KA, int NB>
+__device__ inline void rv_mma(RV<NB>& r, const RV<KA>& a, const float* q) {
+    constexpr int T = KB * 4 * NB, G = 8, NG = (T + G - 1) / G;
+    float b[2][G];
+    auto read = [&](int g) {
+#pragma unroll
+        for (int i = 0; i < G; ++i)
+            if (g * G + i < T) b[g & 1][i] = q[((g * G + i) / NB / 4 * 16 + (g * G + i) / NB % 4) * LDN + 16 * ((g * G + i) % NB)];
+    };
+    read(0);
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+        if (g + 1 < NG) read(g + 1);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < G; ++i) {
+            const int t = g * G + i;
+            if (t < T) r.v[t % NB] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[g & 1][i], a.v[J0 + t / NB / 4][t / NB % 4], r.v[t % NB], 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
 // a [16, 16*KB] x b [16*KB, 16*NB], b in LDS with row pitch LDN.
 template <int KB, int NB, int LDN>
 __device__ inline RV<NB> rv_matmul(const RV<KB>& a, const float* b) {
@@ -1183,13 +1215,7 @@ __device__ inline RV<NB> rv_matmul(const RV<KB>& a, const float* b) {
     RV<NB> r;
 #pragma unroll
     for (int n = 0; n < NB; ++n) r.v[n] = f32x4v{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int j = 0; j < KB; ++j)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-#pragma unroll
-            for (int n = 0; n < NB; ++n)
-                r.v[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(q[(16 * j + e) * LDN + 16 * n], a.v[j][e], r.v[n], 0, 0, 0);
+    rv_mma<0, KB, LDN>(r, a, q);
     return r;
 }
 
@@ -1261,12 +1287,23 @@ struct RvSlice {
 // rv_matmul's order.  For right operands that do not fit LDS whole: an MLP of
 // 128 -> 512 -> 128 columns holds 512 KB of weights: the block around it over
 // 8192 tokens in tasks of 64 rows took 318 us with the MLP as a tile program
-// (its tiles in global scratch), 64 us streamed.
+// (its tiles in global scratch), 52 us streamed; 27 are the MFMAs of a wave.
+template <int S, int S_END, int KA, int NB, int LDN, int KS, class Slice>
+__device__ inline void rv_stream_step(RV<NB>& r, const RV<KA>& a, Slice& sl, float* buf, int at, const float* p, i64 s3, i64 s4) {
+    if constexpr (S < S_END) {
+        if constexpr (S + 1 < S_END) sl.fetch(p + (S + 1) * KS * s3, s3, s4);
+        rv_mma<S * (KS / 16), KS / 16, LDN>(r, a, buf + (S & 1) * (KS * LDN) + at);
+        if constexpr (S + 1 < S_END) {
+            // The other buffer's readers passed the barrier of the slice before.
+            sl.put(buf + ((S + 1) & 1) * (KS * LDN));
+            __syncthreads();
+        }
+        rv_stream_step<S + 1, S_END, KA, NB, LDN, KS>(r, a, sl, buf, at, p, s3, s4);
+    }
+}
 template <int KB, int NB, int LDN, int KS, int MODE, int NT>
 __device__ inline RV<NB> rv_matmul_stream(const RV<KB>& a, float* buf, const float* p, i64 s3, i64 s4) {
-    constexpr int S = 16 * KB / KS;
     const int lane = threadIdx.x & 63;
-    const int at = 4 * (lane >> 4) * LDN + (lane & 15);
     RvSlice<KS, 16 * NB, LDN, MODE, NT> sl;
     sl.fetch(p, s3, s4);
     __syncthreads();  // the buffers' readers before this product
@@ -1275,26 +1312,7 @@ __device__ inline RV<NB> rv_matmul_stream(const RV<KB>& a, float* buf, const flo
     RV<NB> r;
 #pragma unroll
     for (int n = 0; n < NB; ++n) r.v[n] = f32x4v{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int s = 0; s < S; ++s) {
-        if (s + 1 < S) {
-            sl.fetch(p + (s + 1) * KS * s3, s3, s4);
-            __builtin_amdgcn_sched_barrier(0);  // the fetch ahead of the MFMAs
-        }
-        const float* q = buf + (s & 1) * (KS * LDN) + at;
-#pragma unroll
-        for (int j = 0; j < KS / 16; ++j)
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-#pragma unroll
-                for (int n = 0; n < NB; ++n)
-                    r.v[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(q[(16 * j + e) * LDN + 16 * n], a.v[s * (KS / 16) + j][e], r.v[n], 0, 0, 0);
-        if (s + 1 < S) {
-            // The other buffer's readers passed the barrier of the slice before.
-            sl.put(buf + ((s + 1) & 1) * (KS * LDN));
-            __syncthreads();
-        }
-    }
+    rv_stream_step<0, 16 * KB / KS, KB, NB, LDN, KS>(r, a, sl, buf, 4 * (lane >> 4) * LDN + (lane & 15), p, s3, s4);
     return r;
 }
 

@@ -1544,7 +1544,7 @@ bool emit_rowblock(const RowChain& c, EmittedKernel& ek) {
     // Tasks of 16 or 32 rows share a workgroup of 4 waves where they read the
     // same right operand: it is staged once for all of them, and a workgroup of
     // one wave could not stream it (16384 tokens of the block below in tasks of
-    // 16 rows: 172 us as tile programs, 61 so).  Without a shared one a
+    // 16 rows: 172 us as tile programs, 50 so).  Without a shared one a
     // workgroup per task spreads better.
     const int tpb = uniform && blocks == nw ? 4 / nw : 1, nt = 64 * nw * tpb;
     // What does not fit in LDS is streamed through two buffers of ks rows, at

@@ -1529,7 +1529,7 @@ using ReadyLaunches = std::map<size_t, BuiltLaunch>;
 // may loop the same number of times (an in-kernel loop, or an innermost grid
 // variable that the others do not have).  The llama example's block
 // (attention, add, rmsnorm, MLP, add over 8192 tokens): five launches 68 us,
-// 21 and 40 of them the two tile programs, one chain 18.  The three-phase
+// 21 and 40 of them the two tile programs, one chain 15.  The three-phase
 // softmax example over [8, 4096, 512]: three passes over the data 67 us, one
 // 26 (134 MB, 5.2 TB/s).
 // Returns the number of items launched (0: none).
