@@ -1075,9 +1075,10 @@ __device__ inline float cross4_reduce(float x, Op op) {
 // What bounds it: attention tiles of 64 rows at head dim 64 (4 x 16 x 2048)
 // move 134 MB and need 2.1 GFLOP of fp32 MFMA, 22 and 14 us; as a tile
 // program (values in LDS, a workgroup barrier per op, sequential row
-// reductions on 64 of 256 threads) 86 us, as row blocks 34 us: a CU's four
-// workgroups load, compute and store in step, so the two times add up more
-// than they overlap.
+// reductions on 64 of 256 threads) 86 us, as row blocks with both operands in
+// LDS 34 us: a CU's four workgroups load, compute and store in step, so the
+// two times add up more than they overlap.  With the operands taking turns in
+// one buffer a CU holds all eight of its workgroups: 31 us.
 template <int NB>
 struct RV {
     f32x4v v[NB];

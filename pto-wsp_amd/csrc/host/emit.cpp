@@ -1520,9 +1520,12 @@ bool emit_rowblock(const RowChain& c, EmittedKernel& ek) {
     struct Right {
         int k = 0, n = 0, ks = 0;
         size_t off = 0;
+        int slice = -1;  // staged late: the value that holds it on its way
         size_t floats() const { return static_cast<size_t>(k) * (n + 4); }
     };
     std::map<int, Right> right;
+    std::vector<int> order;  // slots in `right` by first use
+    bool turns = true;       // no operand is used again once the next one is
     bool uniform = false;  // a right operand that all tasks read
     long mfma = 0;
     for (const auto& sg : c.segs)
@@ -1534,10 +1537,12 @@ bool emit_rowblock(const RowChain& c, EmittedKernel& ek) {
             Right& r = right[slot];
             if (r.k) {
                 if (r.k != b->rows || r.n != b->cols) return false;
+                turns = turns && slot == order.back();
                 continue;
             }
             r.k = b->rows;
             r.n = b->cols;
+            order.push_back(slot);
             uniform = uniform || c.slots[slot].uniform;
         }
     if (mfma > 4096) return false;
@@ -1566,6 +1571,23 @@ bool emit_rowblock(const RowChain& c, EmittedKernel& ek) {
         for (int ks = 16; ks <= big->k && ks * big->n <= 8192; ks += 16)
             if (big->k % ks == 0) big->ks = ks;
         buffer = std::max(buffer, static_cast<size_t>(big->ks) * (big->n + 4));
+    }
+    // Staged late (RowChain::late): the operands take turns in one LDS buffer,
+    // those after the first waiting in registers (at most 32 a thread), so that
+    // a CU holds more workgroups, some loading while others multiply.  Of use
+    // only where LDS is what limits them: 8 workgroups of 4 waves fill a CU,
+    // and chains whose grid leaves one per CU pay for the barriers (llama block
+    // of 8192 tokens, width 64: 36.7 us up front, 37.1 late).
+    bool late = c.late && turns && order.size() > 1 && tpb == 1 && buffer == 0 && nt == 256 && lds * 4 > 160 * 1024 / 8;
+    int on_way = 0;
+    for (size_t i = 1; i < order.size(); ++i) on_way += (right[order[i]].k * right[order[i]].n / 4 + nt - 1) / nt * 4;
+    late = late && on_way <= 32;
+    if (late) {
+        lds = 0;
+        for (auto& [s, r] : right) {
+            r.off = 0;
+            lds = std::max(lds, r.floats());
+        }
     }
     // The chain's values in order, each with its registers, and the lines that
     // compute them.  cur: the value a slot holds.
@@ -1632,6 +1654,17 @@ bool emit_rowblock(const RowChain& c, EmittedKernel& ek) {
         if (si == 0) {
             for (const auto& op : k.ops)  // a left operand read from memory: ahead of the barrier too
                 if (op.kind == OpKind::Matmul && a.param_of[op.operands[0]] >= 0) read(op.operands[0]);
+            for (size_t i = 1; late && i < order.size(); ++i) {
+                const int s = order[i];
+                Right& r = right[s];
+                const std::string st = std::to_string(s);
+                r.slice = static_cast<int>(regs.size());
+                regs.push_back((r.k * r.n / 4 + nt - 1) / nt * 4);
+                lines.push_back({"  RvSlice<" + std::to_string(r.k) + ", " + std::to_string(r.n) + ", " + std::to_string(r.n + 4) + ", " +
+                                     std::to_string(c.slots[s].stage_mode) + ", " + std::to_string(nt) + "> " + vn(r.slice) + ";\n  " + vn(r.slice) +
+                                     ".fetch(P" + st + ", A.s3[" + st + "], A.s4[" + st + "]);\n",
+                                 {}, r.slice});
+            }
             barrier = lines.size();
         }
         auto get = [&](int id) { return val[id] >= 0 ? val[id] : read(id); };
@@ -1662,8 +1695,12 @@ bool emit_rowblock(const RowChain& c, EmittedKernel& ek) {
                 case OpKind::Matmul: {
                     const int x = op.operands[0], y = op.operands[1];
                     const int s = sg.slot[a.tensor_ordinal[a.param_of[y]]];
-                    const Right& r = right[s];
+                    Right& r = right[s];
                     const std::string xa = use(x);
+                    if (r.slice >= 0) {
+                        lines.push_back({"  __syncthreads();\n  " + vn(r.slice) + ".put(lb);\n  __syncthreads();\n", {r.slice}, -1});
+                        r.slice = -2;  // in LDS from here on
+                    }
                     if (r.ks) {
                         val[op.result] = emit(r.n / 4, uses, rvt(r.n / 16), "rv_matmul_stream<" + std::to_string(r.k / 16) + ", " + std::to_string(r.n / 16) +
                                                                                 ", " + std::to_string(r.n + 4) + ", " + std::to_string(r.ks) + ", " +
@@ -1710,7 +1747,12 @@ bool emit_rowblock(const RowChain& c, EmittedKernel& ek) {
     }
     // A wave has 512 registers; half of them leave room for the products'
     // operands, addresses and a second wave.
-    if (most_live(lines, regs) > 224) return false;
+    if (most_live(lines, regs) > 224) {
+        if (!late) return false;
+        RowChain up_front = c;
+        up_front.late = false;
+        return emit_rowblock(up_front, ek);
+    }
 
     std::ostringstream o;
     o << "#include \"ptowsp_device.h\"\nusing namespace ptowsp;\n// row-block program: kernels";
@@ -1739,7 +1781,7 @@ bool emit_rowblock(const RowChain& c, EmittedKernel& ek) {
     for (int s = 0; s < nslots; ++s)
         o << "  float* const P" << s << " = reinterpret_cast<float*>(A.base[" << s << "]) + (" << offset_expr(s, c.ng, 0, 0) << ");\n";
     for (const auto& [s, r] : right) {
-        if (r.ks) continue;
+        if (r.ks || r.slice == -2) continue;
         const bool own = tpb > 1 && !c.slots[s].uniform;  // of the task's waves only
         o << "  rv_stage<" << r.k << ", " << r.n << ", " << r.n + 4 << ", " << c.slots[s].stage_mode << ", " << (own ? 64 * nw : nt) << ">(lb + " << r.off;
         if (own) o << " + part * " << r.floats();

@@ -137,6 +137,7 @@ struct RowChain {
     int loop = 1;
     int vec_width = 1;               // row program: as EmitSpec
     bool unit_cols = false, nontemporal = false;
+    bool late = false;               // row blocks: right operands after the first are staged when they are used
 };
 
 // Emits the kernel of a chain; false when its values need more registers, or

@@ -1520,6 +1520,12 @@ bool enqueue_decode_folded(RunEnv& E, int li, int lj, hipStream_t stream, uint64
 // ones of the same item list use them instead of building them again.
 using ReadyLaunches = std::map<size_t, BuiltLaunch>;
 
+// Workgroups from which a chain's right operands are staged late: four per CU,
+// more than what up-front staging holds at once.  Attention tiles of 64 rows,
+// pass, up front and late: 2048 tasks at head dim 64 53.1 and 49.5 us, 1024 at
+// 128 56.2 and 50.0; 640 at 64 34.6 and 34.5, 512 at 128 38.1 and 38.4.
+constexpr int64_t kLateBlocks = 1024;
+
 // Launches items[i], items[i+1], ... as one kernel (RowChain) where they are
 // consecutive launches over the same grid whose rows are independent and no
 // memory links them except row by row: a tensor that one of them writes is
@@ -1616,7 +1622,8 @@ size_t enqueue_chain(RunEnv& E, const std::vector<PlanItem>& items, size_t i0, h
         int nscal = 0;
         bool ok = true;
         std::ostringstream key;
-        key << (mm ? "b" : "r") << chain.loop << ";";
+        chain.late = mm && tasks * std::max(1, k0.rowblock.rows / 64) >= kLateBlocks;
+        key << (mm ? chain.late ? "bl" : "b" : "r") << chain.loop << ";";
         for (size_t j = 0; j < len && ok; ++j) {
             const LaunchSpec& L = launch(i0 + j);
             const KernelAnalysis& a = kernel(i0 + j);

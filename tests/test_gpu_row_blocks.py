@@ -46,6 +46,23 @@ def test_attention_row_blocks(gpu, ts, D):
     assert _rel(a["o"], ((e / e.sum(-1, keepdims=True)) @ v64).reshape(q.shape)) <= 1e-5
 
 
+def _attention_error(B, S, D, ts):
+    rng = np.random.default_rng(S + D)
+    q, k, v = (rng.standard_normal((B, 4, S, D), dtype=np.float32) for _ in range(3))
+    a = W.attention_arrays(q, k, v, ts)
+    assert _run(W.rr4(W.tiled_attention(a, ts))).stats.launches == 1
+    q, k, v = (x.reshape(B, 4, S // ts, ts, D).astype(np.float64) for x in (q, k, v))
+    s = q @ k.swapaxes(-1, -2) / math.sqrt(D)
+    e = np.exp(s - s.max(-1, keepdims=True))
+    return _rel(a["o"], ((e / e.sum(-1, keepdims=True)) @ v).reshape(B, 4, S, D))
+
+
+# From 1024 workgroups the right operands take turns in one LDS buffer; 128 rows are two workgroups.
+@pytest.mark.parametrize("B,S,D,ts", [(4, 4096, 64, 64), (4, 4032, 128, 64), (4, 4096, 128, 64), (3, 11008, 64, 128)])
+def test_attention_operands_in_turn(gpu, B, S, D, ts):
+    assert _attention_error(B, S, D, ts) <= 1e-5
+
+
 @pytest.mark.parametrize("seq,d,mlp,ts", [(256, 64, 128, 64), (96, 32, 128, 32), (192, 128, 256, 64), (160, 64, 256, 16)])
 def test_llama_chain(gpu, seq, d, mlp, ts):
     """The five launches of the llama block: one chain where every product is of MFMA shape and the
