@@ -425,7 +425,10 @@ RowBlockInfo classify_rowblock(const KernelDef& k, const KernelAnalysis& a) {
             const ValueInfo *x = a.by_id[op.operands[0]], *y = a.by_id[op.operands[1]];
             const int pb = a.param_of[y->id];
             if (op.operands.size() != 2 || pb < 0 || x->rows != R || x->cols % 16 || y->cols % 16) return no;
-            if (!tile_mma_kind(x->rows, x->cols, y->cols)) return no;
+            if (!tile_mma_kind(x->rows, x->cols, y->cols)) {
+                if (x->cols > 32 && x->cols % 32) return no;
+                r.small = true;
+            }
             r.right[a.tensor_ordinal[pb]] = true;
             ++other[x->id];
             continue;

@@ -73,6 +73,7 @@ struct NormInfo {
 struct RowBlockInfo {
     bool ok = false;
     bool matmul = false;           // has matmuls, all of them of MFMA shape
+    bool small = false;            // some of them below 32^3 products (tile_mma_kind 0)
     int rows = 0;                  // a multiple of 16
     std::vector<RowClass> cls;     // value id -> class (Full: [rows, 16*n]); None for right operands only
     std::vector<bool> right;       // tensor ordinal: a matmul's right operand

@@ -1520,6 +1520,14 @@ bool enqueue_decode_folded(RunEnv& E, int li, int lj, hipStream_t stream, uint64
 // ones of the same item list use them instead of building them again.
 using ReadyLaunches = std::map<size_t, BuiltLaunch>;
 
+// Tasks from which matmuls below 32^3 products run as row blocks.  The tile
+// program's scalar loop, which sums in the oracle's order, keeps fewer: a
+// launch of a task per CU is where the products begin to cost more than the
+// launch.  Attention tiles of 16 rows, pass before and after: 8192 tasks at
+// head dim 64 96 -> 46 us, 16384 at 32 107 -> 45, 1024 at 64 32 -> 26, 256 at
+// 64 27 -> 24; the llama block of 8192 tokens, width 64, in 16-row tiles 51 -> 35.
+constexpr int64_t kSmallBlockTasks = 256;
+
 // Workgroups from which a chain's right operands are staged late: four per CU,
 // more than what up-front staging holds at once.  Attention tiles of 64 rows,
 // pass, up front and late: 2048 tasks at head dim 64 53.1 and 49.5 us, 1024 at
@@ -1589,6 +1597,7 @@ size_t enqueue_chain(RunEnv& E, const std::vector<PlanItem>& items, size_t i0, h
         if (r == ready.end()) r = ready.emplace(i0 + j, build_launch(E, L)).first;
         BuiltLaunch& b = r->second;
         bool ok = b.ntasks > 0 && b.host_checked && !b.spec.serial && (L.inner.empty() || b.spec.row_loops);
+        ok = ok && !(matmul && kernel(i0 + j).rowblock.small && b.ntasks < kSmallBlockTasks);
         for (size_t v = 0; v < ng && ok; ++v) ok = j == 0 || b.args.ext[v] == B[0]->args.ext[v];
         if (ok && (L.grid.size() > ng || !L.inner.empty())) {
             ok = L.grid.size() + L.inner.size() == ng + 1;

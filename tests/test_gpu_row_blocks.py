@@ -63,6 +63,12 @@ def test_attention_operands_in_turn(gpu, B, S, D, ts):
     assert _attention_error(B, S, D, ts) <= 1e-5
 
 
+# Products below 32^3 from 256 tasks (fewer in the first case: the scalar loop).
+@pytest.mark.parametrize("B,S,D,ts", [(5, 192, 64, 16), (4, 256, 64, 16), (4, 272, 32, 16), (1, 1040, 16, 16)])
+def test_attention_small_products(gpu, B, S, D, ts):
+    assert _attention_error(B, S, D, ts) <= 1e-5
+
+
 @pytest.mark.parametrize("seq,d,mlp,ts", [(256, 64, 128, 64), (96, 32, 128, 32), (192, 128, 256, 64), (160, 64, 256, 16)])
 def test_llama_chain(gpu, seq, d, mlp, ts):
     """The five launches of the llama block: one chain where every product is of MFMA shape and the
