@@ -714,6 +714,41 @@ struct GemmBlock {
         }
     }
 
+    // C ahead of the epilogue, at most 64 registers beside as many of
+    // accumulators: read under the last two stages, or under the partials of a
+    // split K.  What it saves is the round trips of the epilogue: many for a
+    // block with edges, whose loads sit behind a mask each (15 x 224 x 6144 x
+    // 320 bf16, whole pass: 83.5 -> 70.1 us); one or two otherwise (4 x 1024^3
+    // f16 38.1 -> 37.5), and nothing for one accumulator (1024^3 bf16 29.6
+    // against 29.9) or after a split K (1024^3 f32 46.8 against 47.4).
+    static constexpr bool c_ahead(bool edge, bool split) { return FI * FJ <= 4 && (edge || (!split && FI * FJ >= 2)); }
+    struct CBlock {
+        float v[FI * FJ][16];
+    };
+    template <bool EDGE>
+    __device__ static void c_read(CBlock& c, buf_rsrc rc, int ldc, const GemmOut& g) {
+        const int lane = threadIdx.x & 63, wave = wave_index();
+        const int wm = wave / WN, wn = wave % WN;
+        const int r0 = wm * TM + (lane >> 5) * 4, c0 = wn * TN + (lane & 31);
+        const int vc = ((lane >> 5) * 4 * ldc + (lane & 31)) * 4;
+        const int so = (wm * TM * ldc + wn * TN) * 4;
+#pragma unroll
+        for (int n = 0; n < FI * FJ; ++n)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int i = n / FJ, j = n % FJ, r = i * 32 + (e >> 2) * 8 + (e & 3);
+                c.v[n][e] = 0.0f;
+                if (!EDGE || (r0 + r < g.rows && c0 + j * 32 < g.cols))
+                    c.v[n][e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rc, vc + j * 128, so + r * ldc * 4, 2));
+            }
+    }
+    __device__ static void c_add(Acc& acc, const CBlock& c) {
+#pragma unroll
+        for (int n = 0; n < FI * FJ; ++n)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc.v[n / FJ][n % FJ][e] = c.v[n][e] + acc.v[n / FJ][n % FJ][e];
+    }
+
     // SPLIT: writes this block's partial (128 bits per lane, one accumulator
     // quarter of 1 KiB per instruction) and counts it; true in the last block
     // of the tile to arrive, whose acc then holds the sum of the tile's
@@ -721,7 +756,8 @@ struct GemmBlock {
     // complete (vmcnt 0) in every wave before the workgroup barrier that
     // precedes the count, and agent-coherent loads behind the count's value:
     // the ordering of the decode partials (publish).
-    __device__ static bool reduce_split(Acc& acc, u16* lds, const GemmOut& g) {
+    template <class AtLast>
+    __device__ static bool reduce_split(Acc& acc, u16* lds, const GemmOut& g, AtLast at_last) {
         const int lane = threadIdx.x & 63, wave = wave_index();
         float* tile = g.part + static_cast<i64>(g.tile) * g.ns * (BM * BN);
         const buf_rsrc rp = __builtin_amdgcn_make_buffer_rsrc(tile, 0, -1, 0x00020000);
@@ -746,6 +782,7 @@ struct GemmBlock {
         if (!*last) return false;
         if (threadIdx.x == 0) __hip_atomic_store(g.cnt + g.tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        at_last();
         constexpr int SB = FI * FJ >= 8 ? 1 : 4;  // partials read together
 #pragma unroll
         for (int n = 0; n < FI * FJ; ++n) {
@@ -806,16 +843,40 @@ struct GemmBlock {
 #pragma unroll
         for (int p = 0; p < NS - 1; ++p)
             if (p < nst) issue(p);
-        for (i64 st = 0; st < nst; ++st) {
+        auto head = [&](i64 st) {
             const i64 ahead = nst - 1 - st < NS - 2 ? nst - 1 - st : NS - 2;
             wait_stages(ahead);
             __syncthreads();
             if (st + NS - 1 < nst) issue(st + NS - 1);
+        };
+        constexpr bool AHEAD = ACC && c_ahead(EDGE, SPLIT);
+        CBlock cb;
+        i64 st = 0;
+        for (; st < (AHEAD && !SPLIT ? nst - 2 : nst); ++st) {
+            head(st);
             mma(acc, lds + static_cast<int>(st & (NS - 1)) * STAGE);
         }
-        if constexpr (SPLIT)
-            if (!reduce_split(acc, lds, g)) return;
-        c_out<ACC, EDGE>(acc, rc, ldc, g);
+        if constexpr (AHEAD && !SPLIT) {
+            if (nst > 1) head(st);
+            c_read<EDGE>(cb, rc, ldc, g);
+            __builtin_amdgcn_sched_barrier(0);  // not sunk below the products
+            if (nst > 1) {
+                mma(acc, lds + static_cast<int>(st & (NS - 1)) * STAGE);
+                ++st;
+            }
+            if (nst > 0) {
+                head(st);
+                mma(acc, lds + static_cast<int>(st & (NS - 1)) * STAGE);
+            }
+        }
+        if constexpr (SPLIT) {
+            auto at_last = [&]() {
+                if constexpr (AHEAD) c_read<EDGE>(cb, rc, ldc, g);
+            };
+            if (!reduce_split(acc, lds, g, at_last)) return;
+        }
+        if constexpr (AHEAD) c_add(acc, cb);
+        c_out<ACC && !AHEAD, EDGE>(acc, rc, ldc, g);
     }
 };
 
@@ -948,7 +1009,7 @@ struct GemmF32 {
 #pragma unroll
         for (int p = 0; p < NS - 1; ++p)
             if (p < nst) issue(p);
-        for (i64 st = 0; st < nst; ++st) {
+        auto head = [&](i64 st) {
             const i64 ahead = nst - 1 - st < NS - 2 ? nst - 1 - st : NS - 2;
             if constexpr (NS == 2) {
                 wait_vmcnt<0>();
@@ -959,11 +1020,35 @@ struct GemmF32 {
             }
             __syncthreads();
             if (st + NS - 1 < nst) issue(st + NS - 1);
+        };
+        constexpr bool AHEAD = ACC && Out::c_ahead(EDGE, SPLIT);
+        typename Out::CBlock cb;
+        i64 st = 0;
+        for (; st < (AHEAD && !SPLIT ? nst - 2 : nst); ++st) {
+            head(st);
             mma(acc, ring + static_cast<int>(st & (NS - 1)) * STAGE);
         }
-        if constexpr (SPLIT)
-            if (!Out::reduce_split(acc, lds, g)) return;
-        Out::template c_out<ACC, EDGE>(acc, rc, ldc, g);
+        if constexpr (AHEAD && !SPLIT) {
+            if (nst > 1) head(st);
+            Out::template c_read<EDGE>(cb, rc, ldc, g);
+            __builtin_amdgcn_sched_barrier(0);  // not sunk below the products
+            if (nst > 1) {
+                mma(acc, ring + static_cast<int>(st & (NS - 1)) * STAGE);
+                ++st;
+            }
+            if (nst > 0) {
+                head(st);
+                mma(acc, ring + static_cast<int>(st & (NS - 1)) * STAGE);
+            }
+        }
+        if constexpr (SPLIT) {
+            auto at_last = [&]() {
+                if constexpr (AHEAD) Out::template c_read<EDGE>(cb, rc, ldc, g);
+            };
+            if (!Out::reduce_split(acc, lds, g, at_last)) return;
+        }
+        if constexpr (AHEAD) Out::c_add(acc, cb);
+        Out::template c_out<ACC && !AHEAD, EDGE>(acc, rc, ldc, g);
     }
 };
 
@@ -1078,7 +1163,7 @@ __device__ inline float cross4_reduce(float x, Op op) {
 // reductions on 64 of 256 threads) 86 us, as row blocks with both operands in
 // LDS 34 us: a CU's four workgroups load, compute and store in step, so the
 // two times add up more than they overlap.  With the operands taking turns in
-// one buffer a CU holds all eight of its workgroups: 31 us.
+// one buffer a CU holds all eight of its workgroups: 32 us.
 template <int NB>
 struct RV {
     f32x4v v[NB];
