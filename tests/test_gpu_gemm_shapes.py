@@ -75,6 +75,13 @@ def test_gemm_shape(gpu, dt, B, M, N, K, tile):
         assert bool((buf[:, 0] == 5.0).all()) and bool((buf[:, M + 1] == 5.0).all())
 
 
+# One, two and three stages: C is read ahead of the last two.
+@pytest.mark.parametrize("dt,k", [("bf16", 64), ("bf16", 128), ("f16", 192), ("f32", 32), ("f32", 64), ("f32", 96)])
+@pytest.mark.parametrize("B,M,N", [(3, 80, 144), (512, 64, 128), (64, 176, 208)])
+def test_gemm_few_stages(gpu, dt, k, B, M, N):
+    test_gemm_shape(gpu, dt, B, M, N, k, (16, 16, 32))
+
+
 @pytest.mark.parametrize("M,N,K,tk", [(48, 256, 512, 256), (160, 192, 1024, 1024), (32, 512, 1024, 512)])
 def test_gemm_plain_last_step(gpu, M, N, K, tk):
     """store(c, matmul(a, b)) under a K loop: the last step's product, in stages and parts."""
