@@ -1615,7 +1615,8 @@ size_t enqueue_chain(RunEnv& E, const std::vector<PlanItem>& items, size_t i0, h
         int tid, rows, cols;
         bool shared = false;  // a right operand, or a vector that all rows read
     };
-    const int nvars = static_cast<int>(ng) + 1;
+    // The grid's variables and the loop's (a nest of kMaxVars grid loops has none left for one).
+    const int nvars = std::min(static_cast<int>(ng) + 1, kMaxVars);
     for (size_t len = B.size(); len > 0; --len) {
         bool mm = false;
         for (size_t j = 0; j < len; ++j) mm = mm || (matmul && kernel(i0 + j).rowblock.matmul);
@@ -1677,7 +1678,7 @@ size_t enqueue_chain(RunEnv& E, const std::vector<PlanItem>& items, size_t i0, h
                         A.coef[s][g] = coef(g);
                         aligned = aligned && coef(g) % 4 == 0;
                     }
-                    t.moves = A.coef[s][ng] != 0;
+                    t.moves = loop > 0 && A.coef[s][ng] != 0;
                     t.uniform = true;
                     for (size_t g = 0; g < ng; ++g) t.uniform = t.uniform && (A.coef[s][g] == 0 || B[0]->args.ext[g] <= 1);
                     t.vec = aligned && X.s4[p] == 1 && X.s3[p] % 4 == 0;

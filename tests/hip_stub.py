@@ -1,0 +1,101 @@
+"""Runs programs through the native library's host side on the CPU: its sources linked against a
+HIP runtime without a device (hip_stub.cpp).  Kernels are emitted and built for gfx950 by hiprtc as
+always; launches are recorded instead of run, so tensors may be views of any size over a small
+buffer."""
+
+import ctypes
+import hashlib
+import os
+import subprocess
+import time
+from dataclasses import dataclass
+
+import pto_wsp._hip as _hip
+from pto_wsp import _build
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+LIB = os.path.join(HERE, "_build", "libptowsp_stub.so")
+
+
+def _library():
+    srcs = [os.path.join(_build.CSRC, "host", s) for s in _build.HOST_SOURCES if s.endswith(".cpp")]
+    srcs.append(os.path.join(HERE, "hip_stub.cpp"))
+    _build._write_embedded_headers()
+    host = os.path.join(_build.CSRC, "host")
+    read = srcs + [os.path.join(host, f) for f in sorted(os.listdir(host)) if f.endswith(".hpp")]
+    read += [os.path.join(_build.BUILD_DIR, "device_headers.inc"), os.path.join(_build.INCLUDE, "ptowsp_hip.h"),
+             os.path.join(_build.INCLUDE, "ptowsp_abi.h")]
+    key = hashlib.sha256(b"".join(open(p, "rb").read() for p in read)).hexdigest()[:16]
+    path = LIB.replace(".so", f"_{key}.so")
+    if not os.path.exists(path):
+        os.makedirs(os.path.dirname(path), exist_ok=True)
+        for old in os.listdir(os.path.dirname(path)):
+            if old.startswith("libptowsp_stub"):
+                os.unlink(os.path.join(os.path.dirname(path), old))
+        procs = []
+        for s in srcs:
+            o = f"{path}.{os.path.basename(s)}.o"
+            cmd = ["hipcc", "--offload-host-only", "-O2", "-std=c++17", "-fPIC", "-w", "-I", _build.INCLUDE, "-I", _build.BUILD_DIR, "-I", host,
+                   "-c", s, "-o", o]
+            procs.append((subprocess.Popen(cmd), o))
+        assert all(p.wait() == 0 for p, _ in procs)
+        objs = [o for _, o in procs]
+        subprocess.run(["g++", "-shared", "-Wl,-Bsymbolic", *objs, "-o", path + ".tmp", "-L/opt/rocm/lib", "-lhiprtc",
+                        "-Wl,-rpath,/opt/rocm/lib"], check=True)
+        for o in objs:
+            os.unlink(o)
+        os.replace(path + ".tmp", path)
+    lib = ctypes.CDLL(path)
+    for name, f in vars(_hip._lib).items():
+        if name.startswith("ptowsp_"):
+            getattr(lib, name).argtypes, getattr(lib, name).restype = f.argtypes, f.restype
+    lib.stub_entry.restype = ctypes.c_char_p
+    for name in ("stub_blocks", "stub_threads"):
+        getattr(lib, name).restype = ctypes.c_uint64
+    for name in ("stub_s3", "stub_s4", "stub_coef"):
+        getattr(lib, name).restype = ctypes.c_int64
+    return lib
+
+
+_lib = None
+
+
+@dataclass
+class Launch:
+    entry: str
+    blocks: int
+    threads: int
+    s3: list
+    s4: list
+    coef: list
+
+
+def run(workload, passes=1):
+    """Launches of one pass of `workload` (after `passes` - 1 others), and the last pass's host time in seconds."""
+    global _lib
+    if _lib is None:
+        _lib = _library()
+    real, _hip._lib = _hip._lib, _lib
+    prog = None
+    try:
+        prog = workload.compile(target="hip_gfx950")
+        best = 1e9
+        for i in range(passes):
+            _lib.stub_clear()
+            t = time.perf_counter()
+            prog.execute()
+            prog.synchronize()
+            if i > 0 or passes == 1:
+                best = min(best, time.perf_counter() - t)
+        out = []
+        for i in range(_lib.stub_num_launches()):
+            out.append(Launch(_lib.stub_entry(i).decode(), _lib.stub_blocks(i), _lib.stub_threads(i),
+                              [_lib.stub_s3(i, p) for p in range(12)], [_lib.stub_s4(i, p) for p in range(12)],
+                              [[_lib.stub_coef(i, p, v) for v in range(8)] for p in range(12)]))
+        assert prog.stats.launches == len(out)
+        return out, best
+    finally:
+        if prog is not None:
+            prog._native = None
+        del prog
+        _hip._lib = real
