@@ -1730,6 +1730,11 @@ size_t enqueue_chain(RunEnv& E, const std::vector<PlanItem>& items, size_t i0, h
             if (!e.ok) e.ek.entry = "-";  // refused: remembered
         }
         if (!e.ok) continue;
+        const int64_t blocks = mm ? (tasks + e.ek.tasks_per_block - 1) / e.ek.tasks_per_block * e.ek.blocks_per_task
+                                  : (tasks * k0.rows + 4 * e.ek.rows_per_chunk - 1) / (4 * e.ek.rows_per_chunk);
+        // A launch takes fewer than 2^32 work-items, and a chain's waves do not
+        // loop over their rows as the launches' own kernels do.
+        if (blocks * e.ek.threads >= (int64_t(1) << 32)) return 0;
         if (!e.jk) {
             if (E.nscratch) {
                 e.jk = jit_loaded(e.ek.source, e.ek.entry);
@@ -1745,7 +1750,6 @@ size_t enqueue_chain(RunEnv& E, const std::vector<PlanItem>& items, size_t i0, h
         A.ntasks = tasks;
         A.err = B[0]->args.err;
         void* params[] = {&A};
-        const int64_t blocks = mm ? (tasks + e.ek.tasks_per_block - 1) / e.ek.tasks_per_block * e.ek.blocks_per_task : (tasks * k0.rows + 4 * e.ek.rows_per_chunk - 1) / (4 * e.ek.rows_per_chunk);
         launch_kernel(E, e.jk->function, blocks, e.ek.threads, 0, stream, params, "hipModuleLaunchKernel(chain)");
         ++launches;
         return len;
