@@ -69,11 +69,24 @@ struct LaunchCache {
     std::vector<std::unique_ptr<Entry>> entries;
 };
 
-// A chain of this program's launches: its kernel, or that it has none.
-struct ChainEntry {
-    bool ok = false;
+// A chain of this program's launches: its kernel, and the chains with one
+// launch more, by what they add to it.
+struct ChainNode {
+    bool tried = false, ok = false;
     EmittedKernel ek;
     const JitKernel* jk = nullptr;
+    // The emitter refused this chain, and so every longer one: its first
+    // `best` launches run as one (0: none).
+    bool refused = false;
+    size_t best = 0;
+    std::vector<std::pair<std::string, std::unique_ptr<ChainNode>>> next;
+
+    ChainNode& child(const std::string& key) {
+        for (auto& n : next)
+            if (n.first == key) return *n.second;
+        next.emplace_back(key, std::make_unique<ChainNode>());
+        return *next.back().second;
+    }
 };
 
 }  // namespace
@@ -83,7 +96,7 @@ struct ptowsp_program {
     std::vector<KernelAnalysis> ka;
     Plan plan;
     std::vector<LaunchCache> cache;
-    std::map<std::string, ChainEntry> chains;  // by launches, slots and access modes
+    std::vector<ChainNode> chains;  // by first launch, and whether its right operands are staged late
     std::vector<bool> tensor_written;
     std::vector<void*> stage_buf;
     std::vector<size_t> stage_bytes;
@@ -152,6 +165,10 @@ struct ptowsp_program {
     bool loads_slots = false, custom = false;
     bool fixed_tasks = false;               // no run-time extent: the cycle model has one result
     std::vector<int> extent_tids;           // tensors that hold loop extents
+    // By launch: how many launches ahead the first one with matmuls is, all of
+    // them consecutive launches of the same rows over as many grid variables
+    // that a row-block chain takes (-1: none).
+    std::vector<int> matmul_ahead;
     uint64_t* slot_stage = nullptr;     // pinned: one element read by a slot load
     std::vector<uint64_t> slot_log;     // values of the run's slot loads, in order
     std::vector<uint64_t> slot_start;   // slots when the run started
@@ -1534,6 +1551,178 @@ constexpr int64_t kSmallBlockTasks = 256;
 // 128 56.2 and 50.0; 640 at 64 34.6 and 34.5, 512 at 128 38.1 and 38.4.
 constexpr int64_t kLateBlocks = 1024;
 
+// Whether item j is a launch without masks.
+bool chain_plain(const Plan& plan, const std::vector<PlanItem>& items, size_t j) {
+    return j < items.size() && !items[j].ctl && !items[j].is_loop && plan.launches[items[j].launch].masks.empty();
+}
+
+// A chain as it grows, one launch at a time: its slots, and what the next
+// launch has to fit.
+struct GrowingChain {
+    struct Place {
+        int tid = -1, rows = 0, cols = 0;
+        bool shared = false;  // a right operand, or a vector that all rows read
+        bool written = false;
+        RowChain::Slot slot;
+    };
+    struct Step {
+        std::array<signed char, kMaxParams> slot{};  // by tensor ordinal
+        int launch = -1;
+        int places = 0, scal0 = 0;                   // slots in use with this launch; its first scalar argument
+        size_t ng = 0;                               // grid variables that the launches share
+        int64_t loop = 0;                            // iterations of the launches that loop (0: none does)
+        int vec_width = 4;
+        bool unit_cols = true;
+    };
+    bool matmul = false;  // as row blocks
+    std::vector<Step> steps;
+    std::vector<const BuiltLaunch*> built;
+    std::array<Place, kMaxParams> places;
+    LaunchArgs A{};
+    int nscal = 0;
+};
+
+// Launches of one chain at most: far more than its registers hold, and a
+// bound on what each start of a chain can cost the host.
+constexpr size_t kChainLaunches = 64;
+
+// Adds launch L, built as b, to the chain; false where it does not fit.  key:
+// what the chain's kernel depends on of this launch and its views.
+bool chain_join(RunEnv& E, GrowingChain& C, const LaunchSpec& L, const KernelAnalysis& a, int index, const BuiltLaunch& b,
+                std::string& key) {
+    const bool first = C.steps.empty(), mm = C.matmul;
+    if (b.ntasks <= 0 || !b.host_checked || b.spec.serial || !(L.inner.empty() || b.spec.row_loops)) return false;
+    if (mm && a.rowblock.small && b.ntasks < kSmallBlockTasks) return false;
+    const LaunchArgs& X = b.args;
+    const size_t g = L.grid.size();
+    GrowingChain::Step S;
+    if (!first) S = C.steps.back();
+    // Grid variables that the launches share; the variable after them is the
+    // loop's, in the kernel or in the grid.
+    bool dropped = false;
+    if (first) {
+        S.ng = g;
+    } else if (g + 1 == S.ng) {
+        // The launches before it have a grid variable more, their loop.
+        if (S.loop) return false;
+        dropped = true;
+        S.ng = g;
+        S.loop = C.built[0]->args.ext[g];
+        if (S.loop < 1 || S.loop > 32) return false;
+    }
+    for (size_t v = 0; v < S.ng && !first; ++v)
+        if (X.ext[v] != C.built[0]->args.ext[v]) return false;
+    const bool loops = g + L.inner.size() > S.ng;
+    if (loops) {
+        if (g + L.inner.size() != S.ng + 1) return false;
+        const int64_t e = X.ext[S.ng];
+        if (e < 1 || e > 32 || (S.loop && S.loop != e)) return false;
+        S.loop = e;
+    }
+    S.launch = index;
+    S.scal0 = C.nscal;
+    if (!mm) {
+        S.vec_width = std::min(S.vec_width, b.spec.vec_width);
+        S.unit_cols = S.unit_cols && b.spec.row_unit_cols;
+    }
+    auto put = [&key](int x) { key.push_back(static_cast<char>(x)); };
+    for (int i = 0; i < 4; ++i) put(index >> (8 * i));
+    put(static_cast<int>(S.loop));
+    put(S.vec_width * 2 + S.unit_cols);
+    bool check_deps = false;
+    LaunchArgs& A = C.A;
+    for (size_t p = 0; p < a.tensor_param_index.size(); ++p) {
+        const int id = a.def->params[a.tensor_param_index[p]].id;
+        const ValueInfo* v = a.by_id[id];
+        int s = -1;
+        for (int q = 0; q < S.places && s < 0; ++q) {
+            const GrowingChain::Place& O = C.places[q];
+            if (O.tid != L.targs[p]->tid || O.rows != v->rows || O.cols != v->cols) continue;
+            if (A.base[q] != X.base[p] || A.s3[q] != X.s3[p] || A.s4[q] != X.s4[p]) continue;
+            if (std::equal(A.coef[q], A.coef[q] + kMaxVars, X.coef[p])) s = q;
+        }
+        if (s < 0) {
+            s = S.places;
+            if (s >= kMaxParams) return false;
+            ++S.places;
+            check_deps = true;
+            A.base[s] = X.base[p];
+            A.s3[s] = X.s3[p];
+            A.s4[s] = X.s4[p];
+            A.span[s] = X.span[p];
+            GrowingChain::Place& O = C.places[s];
+            O = GrowingChain::Place{};
+            O.tid = L.targs[p]->tid;
+            O.rows = v->rows;
+            O.cols = v->cols;
+            RowChain::Slot& t = O.slot;
+            t.dtype = v->dtype;
+            t.uniform = true;
+            bool aligned = reinterpret_cast<uintptr_t>(X.base[p]) % 16 == 0;
+            int moved = 0;
+            for (int i = 0; i < kMaxVars; ++i) {
+                A.coef[s][i] = X.coef[p][i];
+                aligned = aligned && X.coef[p][i] % 4 == 0;
+                moved |= (X.coef[p][i] != 0) << i;
+                if (static_cast<size_t>(i) < S.ng) t.uniform = t.uniform && (X.coef[p][i] == 0 || X.ext[i] <= 1);
+            }
+            t.vec = aligned && X.s4[p] == 1 && X.s3[p] % 4 == 0;
+            t.stage_mode = t.vec ? 0 : aligned && X.s3[p] == 1 && X.s4[p] % 4 == 0 ? 1 : 2;
+            put(s);
+            put(t.vec + 2 * t.stage_mode + 8 * t.uniform);
+            put(mm ? 0 : moved);
+        } else {
+            put(s);
+        }
+        S.slot[p] = static_cast<signed char>(s);
+        GrowingChain::Place& O = C.places[s];
+        RowClass rc = (mm ? a.rowblock.cls : a.row_class)[id];
+        for (const auto& op : a.def->ops)
+            if (op.kind == OpKind::Load && op.operands[0] == id && op.result > 0) rc = (mm ? a.rowblock.cls : a.row_class)[op.result];
+        const bool shared = (mm && a.rowblock.right[p]) || rc == RowClass::ColVec || rc == RowClass::ColVecT;
+        check_deps = check_deps || (shared && !O.shared) || (a.stored[p] && !O.written);
+        O.shared = O.shared || shared;
+        O.written = O.written || a.stored[p];
+    }
+    const size_t ns = L.task->scalar_args.size();
+    if (C.nscal + ns > static_cast<size_t>(kMaxScalars)) return false;
+    for (size_t q = 0; q < ns; ++q) A.scal[C.nscal + q] = X.scal[q];
+    C.nscal += static_cast<int>(ns);
+    C.steps.push_back(S);
+    C.built.push_back(&b);
+    // Row-by-row dependences only.
+    bool ok = true;
+    for (int s = 0; s < S.places && check_deps && ok; ++s) {
+        const GrowingChain::Place& O = C.places[s];
+        if (!O.written) continue;
+        if (O.shared) ok = false;
+        const TensorState& T = E.ts[O.tid];
+        for (int q = 0; q < S.places && ok; ++q) {
+            const TensorState& U = E.ts[C.places[q].tid];
+            if (q != s && T.dev < U.dev + U.span * dtype_size(C.places[q].slot.dtype) &&
+                U.dev < T.dev + T.span * dtype_size(O.slot.dtype))
+                ok = false;
+        }
+    }
+    // Over the grid and the loop a stored tile's elements never repeat: one
+    // that the loop leaves in place is one value per task, which a grid launch
+    // over that variable would write from many tasks.
+    auto in_place = [&](size_t j) {
+        const LaunchSpec& M = E.P->plan.launches[C.steps[j].launch];
+        const KernelAnalysis& k = E.P->ka[M.kernel];
+        if (!M.inner.empty() || M.grid.size() <= S.ng) return false;
+        for (size_t p = 0; p < k.tensor_param_index.size(); ++p)
+            if (k.stored[p] && A.coef[C.steps[j].slot[p]][S.ng] == 0) return true;
+        return false;
+    };
+    for (size_t j = dropped ? 0 : C.steps.size() - 1; j < C.steps.size() && S.loop && ok; ++j) ok = !in_place(j);
+    if (!ok) {
+        C.steps.pop_back();
+        C.built.pop_back();
+    }
+    return ok;
+}
+
 // Launches items[i], items[i+1], ... as one kernel (RowChain) where they are
 // consecutive launches over the same grid whose rows are independent and no
 // memory links them except row by row: a tensor that one of them writes is
@@ -1546,215 +1735,131 @@ constexpr int64_t kLateBlocks = 1024;
 // 21 and 40 of them the two tile programs, one chain 15.  The three-phase
 // softmax example over [8, 4096, 512]: three passes over the data 67 us, one
 // 26 (134 MB, 5.2 TB/s).
+//
+// The chain grows one launch at a time, each built when the chain reaches it,
+// until one does not fit.  Where the emitter refuses what has grown, its
+// longest part is searched once (a longer chain needs no fewer registers, LDS
+// and code); the node behind that part remembers it, so that the next passes
+// stop there.  Host time is so linear in a program's launches (64 llama blocks
+// of five launches in one workload, host side alone: 1.9 ms; 42 with every
+// length tried from every start, on every pass).
 // Returns the number of items launched (0: none).
 size_t enqueue_chain(RunEnv& E, const std::vector<PlanItem>& items, size_t i0, hipStream_t stream, uint64_t& launches,
                      ReadyLaunches& ready) {
     ptowsp_program* P = E.P;
     auto launch = [&](size_t j) -> const LaunchSpec& { return P->plan.launches[items[j].launch]; };
     auto kernel = [&](size_t j) -> const KernelAnalysis& { return P->ka[launch(j).kernel]; };
-    auto plain = [&](size_t j) { return j < items.size() && !items[j].ctl && !items[j].is_loop && launch(j).masks.empty(); };
-    // The longest run of launches with fitting shapes.  blocks: row blocks
-    // (up to the first launch that is none); rows: a row program.
-    if (!plain(i0)) return 0;
+    if (!chain_plain(P->plan, items, i0)) return 0;
     const KernelAnalysis& k0 = kernel(i0);
-    size_t nb = 0, nr = 0;
-    bool matmul = false;
-    if (k0.rowblock.ok && tuning().tile_mma)
-        while (plain(i0 + nb) && launch(i0 + nb).inner.empty() && launch(i0 + nb).grid.size() == launch(i0).grid.size() &&
-               kernel(i0 + nb).rowblock.ok && kernel(i0 + nb).rowblock.rows == k0.rowblock.rows) {
-            matmul = matmul || kernel(i0 + nb).rowblock.matmul;
-            ++nb;
-        }
-    // Grid variables that the launches share: those of a launch that loops.
-    size_t ng = launch(i0).grid.size();
-    if (!matmul) {
-        nb = 0;
-        auto row = [&](size_t j) {
-            return plain(j) && kernel(j).family == Family::RowProgram && kernel(j).rows == k0.rows && kernel(j).cols == k0.cols &&
-                   launch(j).inner.size() <= 1;
-        };
-        while (row(i0 + nr)) {
-            const size_t g = launch(i0 + nr).grid.size();
-            if (g + 1 < ng || g > ng + 1) break;
-            if (g + 1 == ng) {
-                // The launches before it have a grid variable more, their loop.
-                bool all = true;
-                for (size_t j = 0; j < nr; ++j) all = all && launch(i0 + j).grid.size() == ng && launch(i0 + j).inner.empty();
-                if (!all) break;
-                ng = g;
-            }
-            ++nr;
-        }
-        if (nr < 2) return 0;
-    }
-    const size_t n = matmul ? nb : nr;
-    // Build the launches; the chain ends before one that does not fit it.
-    std::vector<const BuiltLaunch*> B;
-    int64_t loop = 0;  // iterations of the launches that loop
-    for (size_t j = 0; j < n; ++j) {
-        const LaunchSpec& L = launch(i0 + j);
-        auto r = ready.find(i0 + j);
-        if (r == ready.end()) r = ready.emplace(i0 + j, build_launch(E, L)).first;
-        BuiltLaunch& b = r->second;
-        bool ok = b.ntasks > 0 && b.host_checked && !b.spec.serial && (L.inner.empty() || b.spec.row_loops);
-        ok = ok && !(matmul && kernel(i0 + j).rowblock.small && b.ntasks < kSmallBlockTasks);
-        for (size_t v = 0; v < ng && ok; ++v) ok = j == 0 || b.args.ext[v] == B[0]->args.ext[v];
-        if (ok && (L.grid.size() > ng || !L.inner.empty())) {
-            ok = L.grid.size() + L.inner.size() == ng + 1;
-            const int64_t e = b.args.ext[ng];
-            ok = ok && e >= 1 && e <= 32 && (loop == 0 || loop == e);
-            if (ok) loop = e;
-        }
-        if (!ok) break;
-        B.push_back(&b);
-    }
-    int64_t tasks = 1;
-    for (size_t v = 0; v < ng && !B.empty(); ++v) tasks *= B[0]->args.ext[v];
-    if (B.empty() || tasks * k0.rows >= (int64_t(1) << 31) || tasks * std::max(1, k0.rowblock.rows / 16) >= (int64_t(1) << 31)) return 0;
-    struct Place {
-        int tid, rows, cols;
-        bool shared = false;  // a right operand, or a vector that all rows read
+    // Launches to the first with a matmul, along which all have the same rows:
+    // row blocks, which need one; else a row program, of two launches or more.
+    const int ahead = P->matmul_ahead[items[i0].launch];
+    GrowingChain C;
+    C.matmul = ahead >= 0 && tuning().tile_mma;
+    const bool mm = C.matmul;
+    const size_t least = mm ? static_cast<size_t>(ahead) + 1 : 2;
+    auto fits = [&](size_t j) {
+        if (!chain_plain(P->plan, items, j)) return false;
+        const KernelAnalysis& k = kernel(j);
+        if (mm) return launch(j).inner.empty() && launch(j).grid.size() == launch(i0).grid.size() && k.rowblock.ok && k.rowblock.rows == k0.rowblock.rows;
+        return k.family == Family::RowProgram && k.rows == k0.rows && k.cols == k0.cols && launch(j).inner.size() <= 1;
     };
-    // The grid's variables and the loop's (a nest of kMaxVars grid loops has none left for one).
-    const int nvars = std::min(static_cast<int>(ng) + 1, kMaxVars);
-    for (size_t len = B.size(); len > 0; --len) {
-        bool mm = false;
-        for (size_t j = 0; j < len; ++j) mm = mm || (matmul && kernel(i0 + j).rowblock.matmul);
-        if (!mm && (matmul || len < 2)) return 0;
-        RowChain chain;
-        chain.ng = static_cast<int>(ng);
-        chain.loop = static_cast<int>(std::max<int64_t>(loop, 1));
-        chain.nontemporal = tuning().nontemporal;
-        chain.vec_width = 4;
-        chain.unit_cols = true;
-        std::vector<Place> places;
-        LaunchArgs A{};
-        int nscal = 0;
-        bool ok = true;
-        std::ostringstream key;
-        chain.late = mm && tasks * std::max(1, k0.rowblock.rows / 64) >= kLateBlocks;
-        key << (mm ? chain.late ? "bl" : "b" : "r") << chain.loop << ";";
-        for (size_t j = 0; j < len && ok; ++j) {
-            const LaunchSpec& L = launch(i0 + j);
-            const KernelAnalysis& a = kernel(i0 + j);
-            const LaunchArgs& X = B[j]->args;
-            const std::vector<RowClass>& cls = mm ? a.rowblock.cls : a.row_class;
-            RowChain::Seg sg;
-            sg.a = &a;
-            sg.scal0 = nscal;
-            sg.loops = L.grid.size() > ng || !L.inner.empty();
-            if (!mm) {
-                chain.vec_width = std::min(chain.vec_width, B[j]->spec.vec_width);
-                chain.unit_cols = chain.unit_cols && B[j]->spec.row_unit_cols;
-            }
-            key << items[i0 + j].launch << ":";
-            for (size_t p = 0; p < a.tensor_param_index.size() && ok; ++p) {
-                const int id = a.def->params[a.tensor_param_index[p]].id;
-                const ValueInfo* v = a.by_id[id];
-                auto coef = [&](int g) { return g < static_cast<int>(ng) || sg.loops ? X.coef[p][g] : 0; };
-                int s = -1;
-                for (size_t q = 0; q < places.size() && s < 0; ++q) {
-                    if (places[q].tid != L.targs[p]->tid || places[q].rows != v->rows || places[q].cols != v->cols) continue;
-                    if (A.base[q] != X.base[p] || A.s3[q] != X.s3[p] || A.s4[q] != X.s4[p]) continue;
-                    bool same = true;
-                    for (int g = 0; g < nvars; ++g) same = same && A.coef[q][g] == coef(g);
-                    if (same) s = static_cast<int>(q);
-                }
-                if (s < 0) {
-                    s = static_cast<int>(places.size());
-                    if (s >= kMaxParams) {
-                        ok = false;
-                        break;
-                    }
-                    places.push_back({L.targs[p]->tid, v->rows, v->cols});
-                    A.base[s] = X.base[p];
-                    A.s3[s] = X.s3[p];
-                    A.s4[s] = X.s4[p];
-                    A.span[s] = X.span[p];
-                    RowChain::Slot t;
-                    t.dtype = v->dtype;
-                    bool aligned = reinterpret_cast<uintptr_t>(X.base[p]) % 16 == 0;
-                    for (int g = 0; g < nvars; ++g) {
-                        A.coef[s][g] = coef(g);
-                        aligned = aligned && coef(g) % 4 == 0;
-                    }
-                    t.moves = loop > 0 && A.coef[s][ng] != 0;
-                    t.uniform = true;
-                    for (size_t g = 0; g < ng; ++g) t.uniform = t.uniform && (A.coef[s][g] == 0 || B[0]->args.ext[g] <= 1);
-                    t.vec = aligned && X.s4[p] == 1 && X.s3[p] % 4 == 0;
-                    t.stage_mode = t.vec ? 0 : aligned && X.s3[p] == 1 && X.s4[p] % 4 == 0 ? 1 : 2;
-                    chain.slots.push_back(t);
-                }
-                chain.slots[s].written = chain.slots[s].written || a.stored[p];
-                RowClass rc = cls[id];
-                for (const auto& op : a.def->ops)
-                    if (op.kind == OpKind::Load && op.operands[0] == id && op.result > 0) rc = cls[op.result];
-                places[s].shared = places[s].shared || (mm && a.rowblock.right[p]) || rc == RowClass::ColVec || rc == RowClass::ColVecT;
-                sg.slot.push_back(s);
-                key << s << (mm ? "" : chain.slots[s].moves ? "m" : "f") << ",";
-            }
-            const size_t ns = L.task->scalar_args.size();
-            if (nscal + ns > static_cast<size_t>(kMaxScalars)) ok = false;
-            for (size_t q = 0; q < ns && ok; ++q) A.scal[nscal + q] = X.scal[q];
-            nscal += static_cast<int>(ns);
-            chain.segs.push_back(std::move(sg));
+    if (least > kChainLaunches || !fits(i0) || (!mm && !fits(i0 + 1))) return 0;
+    std::vector<ChainNode*> path;
+    size_t best = SIZE_MAX;  // launches to run as one, once known
+    std::string key;
+    bool late = false;
+    for (size_t j = i0; j < i0 + kChainLaunches && fits(j); ++j) {
+        auto r = ready.find(j);
+        if (r == ready.end()) r = ready.emplace(j, build_launch(E, launch(j))).first;
+        key.clear();
+        if (!chain_join(E, C, launch(j), kernel(j), items[j].launch, r->second, key)) break;
+        if (j == i0) {
+            late = mm && r->second.ntasks * std::max(1, k0.rowblock.rows / 64) >= kLateBlocks;
+            path.push_back(&P->chains[items[i0].launch * 2 + late]);
         }
-        // Row-by-row dependences only.
-        for (size_t s = 0; s < places.size() && ok; ++s) {
-            if (!chain.slots[s].written) continue;
-            if (places[s].shared) ok = false;
-            const TensorState& T = E.ts[places[s].tid];
-            for (size_t q = 0; q < places.size() && ok; ++q) {
-                const TensorState& U = E.ts[places[q].tid];
-                if (q != s && T.dev < U.dev + U.span * dtype_size(chain.slots[q].dtype) &&
-                    U.dev < T.dev + T.span * dtype_size(chain.slots[s].dtype))
-                    ok = false;
-            }
-            // Over the grid and the loop its elements never repeat: a tile that
-            // the loop leaves in place is one value per task, which a grid
-            // launch over that variable would write from many tasks.
-            if (ok && loop > 0 && A.coef[s][ng] == 0)
-                for (size_t j = 0; j < len && ok; ++j)
-                    for (size_t p = 0; p < chain.segs[j].slot.size() && ok; ++p)
-                        ok = chain.segs[j].slot[p] != static_cast<int>(s) || !chain.segs[j].loops || !launch(i0 + j).inner.empty() ||
-                             !kernel(i0 + j).stored[p];
+        path.push_back(&path.back()->child(key));
+        if (path.back()->refused) {
+            best = path.back()->best;
+            break;
         }
-        if (!ok) continue;
-        if (mm)
-            for (const auto& t : chain.slots) key << (t.vec ? "v" : "s") << t.stage_mode << (t.uniform ? "u" : "");
-        else
-            key << "vw" << chain.vec_width << (chain.unit_cols ? "u" : "") << (chain.nontemporal ? "n" : "");
-        ChainEntry& e = P->chains.emplace(key.str(), ChainEntry{}).first->second;
-        if (!e.ok && e.ek.entry.empty()) {
-            e.ok = mm ? emit_rowblock(chain, e.ek) : emit_rowchain(chain, e.ek);
-            if (!e.ok) e.ek.entry = "-";  // refused: remembered
-        }
-        if (!e.ok) continue;
-        const int64_t blocks = mm ? (tasks + e.ek.tasks_per_block - 1) / e.ek.tasks_per_block * e.ek.blocks_per_task
-                                  : (tasks * k0.rows + 4 * e.ek.rows_per_chunk - 1) / (4 * e.ek.rows_per_chunk);
-        // A launch takes fewer than 2^32 work-items, and a chain's waves do not
-        // loop over their rows as the launches' own kernels do.
-        if (blocks * e.ek.threads >= (int64_t(1) << 32)) return 0;
-        if (!e.jk) {
-            if (E.nscratch) {
-                e.jk = jit_loaded(e.ek.source, e.ek.entry);
-                if (!e.jk)
-                    throw std::runtime_error("ptowsp_hip_launch_noalloc: the kernel of launch " + std::to_string(items[i0].launch) +
-                                             " is not loaded yet; run the program once through ptowsp_hip_launch, "
-                                             "which builds and loads its kernels");
-            } else {
-                e.jk = &jit_kernel(e.ek.source, e.ek.entry);
-            }
-        }
-        for (size_t v = 0; v < ng; ++v) A.ext[v] = B[0]->args.ext[v];
-        A.ntasks = tasks;
-        A.err = B[0]->args.err;
-        void* params[] = {&A};
-        launch_kernel(E, e.jk->function, blocks, e.ek.threads, 0, stream, params, "hipModuleLaunchKernel(chain)");
-        ++launches;
-        return len;
     }
-    return 0;
+    const size_t grown = C.steps.size();
+    // The kernel of the first n launches: built once, or refused.
+    auto emitted = [&](size_t n) {
+        ChainNode& node = *path[n];
+        if (!node.tried) {
+            const GrowingChain::Step& S = C.steps[n - 1];
+            RowChain c;
+            c.ng = static_cast<int>(S.ng);
+            c.loop = static_cast<int>(std::max<int64_t>(S.loop, 1));
+            c.vec_width = S.vec_width;
+            c.unit_cols = S.unit_cols;
+            c.nontemporal = tuning().nontemporal;
+            c.late = late;
+            for (int s = 0; s < S.places; ++s) {
+                c.slots.push_back(C.places[s].slot);
+                c.slots.back().moves = S.loop && C.A.coef[s][S.ng] != 0;
+            }
+            for (size_t j = 0; j < n; ++j) {
+                const LaunchSpec& L = launch(i0 + j);
+                RowChain::Seg sg;
+                sg.a = &kernel(i0 + j);
+                sg.slot.assign(C.steps[j].slot.begin(), C.steps[j].slot.begin() + sg.a->tensor_param_index.size());
+                sg.scal0 = C.steps[j].scal0;
+                sg.loops = L.grid.size() + L.inner.size() > S.ng;
+                c.segs.push_back(std::move(sg));
+            }
+            node.tried = true;
+            node.ok = mm ? emit_rowblock(c, node.ek) : emit_rowchain(c, node.ek);
+        }
+        return node.ok;
+    };
+    if (best == SIZE_MAX) {
+        if (grown < least) return 0;
+        best = grown;
+        if (!emitted(grown)) {
+            size_t refused = grown;
+            best = least - 1;
+            while (refused - best > 1) {
+                const size_t n = (refused + best) / 2;
+                (emitted(n) ? best : refused) = n;
+            }
+            if (best < least) best = 0;
+            path[refused]->refused = true;
+            path[refused]->best = best;
+        }
+    }
+    if (best == 0) return 0;
+    const GrowingChain::Step& S = C.steps[best - 1];
+    ChainNode& e = *path[best];
+    int64_t tasks = 1;
+    for (size_t v = 0; v < S.ng; ++v) tasks *= C.built[0]->args.ext[v];
+    if (tasks * k0.rows >= (int64_t(1) << 31) || tasks * std::max(1, k0.rowblock.rows / 16) >= (int64_t(1) << 31)) return 0;
+    const int64_t blocks = mm ? (tasks + e.ek.tasks_per_block - 1) / e.ek.tasks_per_block * e.ek.blocks_per_task
+                              : (tasks * k0.rows + 4 * e.ek.rows_per_chunk - 1) / (4 * e.ek.rows_per_chunk);
+    // A launch takes fewer than 2^32 work-items, and a chain's waves do not
+    // loop over their rows as the launches' own kernels do.
+    if (blocks * e.ek.threads >= (int64_t(1) << 32)) return 0;
+    if (!e.jk) {
+        if (E.nscratch) {
+            e.jk = jit_loaded(e.ek.source, e.ek.entry);
+            if (!e.jk)
+                throw std::runtime_error("ptowsp_hip_launch_noalloc: the kernel of launch " + std::to_string(items[i0].launch) +
+                                         " is not loaded yet; run the program once through ptowsp_hip_launch, "
+                                         "which builds and loads its kernels");
+        } else {
+            e.jk = &jit_kernel(e.ek.source, e.ek.entry);
+        }
+    }
+    LaunchArgs& A = C.A;
+    for (size_t v = 0; v < S.ng; ++v) A.ext[v] = C.built[0]->args.ext[v];
+    A.ntasks = tasks;
+    A.err = C.built[0]->args.err;
+    void* params[] = {&A};
+    launch_kernel(E, e.jk->function, blocks, e.ek.threads, 0, stream, params, "hipModuleLaunchKernel(chain)");
+    ++launches;
+    return best;
 }
 
 void run_host_step(RunEnv& E, const PlanItem& it, hipStream_t stream, uint64_t& launches);
@@ -2003,8 +2108,30 @@ std::vector<int> device_extent_tensors(RunEnv& E) {
     return out;
 }
 
+// ptowsp_program::matmul_ahead of the launches among `items`.
+void note_matmuls(ptowsp_program* P, const std::vector<PlanItem>& items) {
+    auto block = [&](size_t j) -> const RowBlockInfo* {
+        if (!chain_plain(P->plan, items, j) || !P->plan.launches[items[j].launch].inner.empty()) return nullptr;
+        const RowBlockInfo& r = P->ka[P->plan.launches[items[j].launch].kernel].rowblock;
+        return r.ok ? &r : nullptr;
+    };
+    for (size_t j = items.size(); j-- > 0;) {
+        note_matmuls(P, items[j].body);
+        note_matmuls(P, items[j].alt);
+        const RowBlockInfo *r = block(j), *n = block(j + 1);
+        if (!r) continue;
+        int& d = P->matmul_ahead[items[j].launch];
+        if (r->matmul) d = 0;
+        else if (n && n->rows == r->rows && P->matmul_ahead[items[j + 1].launch] >= 0 &&
+                 P->plan.launches[items[j + 1].launch].grid.size() == P->plan.launches[items[j].launch].grid.size())
+            d = P->matmul_ahead[items[j + 1].launch] + 1;
+    }
+}
+
 // What launch_impl and cycles_for need to know of the module (once).
 void note_module(ptowsp_program* P) {
+    P->matmul_ahead.assign(P->plan.launches.size(), -1);
+    note_matmuls(P, P->plan.items);
     P->dynamic = module_is_dynamic(P->m);
     P->loads_slots = module_loads_slots(P->m);
     for (const auto& k : P->m.kernels) P->custom |= k.custom;
@@ -2215,6 +2342,7 @@ int ptowsp_hip_compile(const char* module_text, ptowsp_program** out) {
         P->plan = build_plan(P->m, P->ka);
         note_module(P.get());
         P->cache.resize(P->plan.launches.size());
+        P->chains.resize(P->plan.launches.size() * 2);
         P->tensor_written.assign(P->m.tensors.size(), false);
         for (const auto& L : P->plan.launches) {
             const KernelAnalysis& a = P->ka[L.kernel];

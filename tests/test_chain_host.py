@@ -1,11 +1,13 @@
 """Chains of launches as the host side forms them (enqueue_chain), on the CPU: launches are recorded
 instead of run (hip_stub)."""
 
+import math
 import mmap
 
 import numpy as np
 
 import hip_stub
+import pytest
 import workloads as W
 from pto_wsp import Dense, In, Out, P, Tile, kernel, pto, workload
 
@@ -100,3 +102,73 @@ def test_more_row_blocks_than_a_launch_takes():
     over = launches(1 << 24)
     assert [x.entry.split("_")[1] for x in over] == ["tile"]
     assert over[0].blocks * over[0].threads < 1 << 32
+
+
+def _llama_blocks(n, d, mlp, st=128, ts=64):
+    """n llama blocks (attention, add, rmsnorm, MLP, add), each reading what the one before it wrote."""
+    def new(*shape):
+        return np.zeros(shape, np.float32)
+
+    xs = [new(st, ts, d) for _ in range(n + 1)]
+    X, KT = [W.T(x) for x in xs], [W.T(x.transpose(0, 2, 1)) for x in xs]
+    W1, W2 = ([W.T(new(*s)) for _ in range(n)] for s in ((d, mlp), (mlp, d)))
+    Attn, Res, Xn, Mlp = (W.T(new(st, ts, d)) for _ in range(4))
+
+    @kernel
+    def attn(q: In[Tile[ts, d, F32]], k_t: In[Tile[d, ts, F32]], v: In[Tile[ts, d, F32]], out: Out[Tile[ts, d, F32]]):
+        s = pto.mul(pto.matmul(q, k_t), pto.constant(1.0 / math.sqrt(d), F32))
+        e = pto.exp(pto.sub(s, pto.rowmax(s)))
+        pto.store(out, pto.matmul(pto.div(e, pto.rowsum(e)), v))
+
+    @kernel
+    def add(a: In[Tile[ts, d, F32]], b: In[Tile[ts, d, F32]], out: Out[Tile[ts, d, F32]]):
+        pto.store(out, pto.add(a, b))
+
+    @kernel
+    def rmsnorm(x: In[Tile[ts, d, F32]], out: Out[Tile[ts, d, F32]]):
+        pto.store(out, pto.mul(x, pto.rsqrt(pto.rowmean(pto.mul(x, x)))))
+
+    @kernel
+    def mlp_relu(x: In[Tile[ts, d, F32]], w1: In[Tile[d, mlp, F32]], w2: In[Tile[mlp, d, F32]], out: Out[Tile[ts, d, F32]]):
+        pto.store(out, pto.matmul(pto.max(pto.matmul(x, w1), pto.constant(0.0, F32)), w2))
+
+    @workload
+    def wl():
+        for s in P(Dense[st]()):
+            for i in range(n):
+                attn[s](q=X[i][s], k_t=KT[i][s], v=X[i][s], out=Attn[s])
+                add[s](a=X[i][s], b=Attn[s], out=Res[s])
+                rmsnorm[s](x=Res[s], out=Xn[s])
+                mlp_relu[s](x=Xn[s], w1=W1[i], w2=W2[i], out=Mlp[s])
+                add[s](a=Res[s], b=Mlp[s], out=X[i + 1][s])
+
+    return W.rr4(wl())
+
+
+def _norms(n, C):
+    X = [W.T(np.zeros((4, 16, C), np.float32)) for _ in range(n + 1)]
+
+    @kernel
+    def rmsnorm(x: In[Tile[16, C, F32]], out: Out[Tile[16, C, F32]]):
+        pto.store(out, pto.mul(x, pto.rsqrt(pto.rowmean(pto.mul(x, x)))))
+
+    @workload
+    def wl():
+        for s in P(Dense[4]()):
+            for i in range(n):
+                rmsnorm[s](x=X[i][s], out=X[i + 1][s])
+
+    return W.rr4(wl())
+
+
+# Chained whole, in part (the MLP's width refused), not at all (a row's registers), and by as many
+# views as a chain has slots.
+@pytest.mark.parametrize("make,per_8", [(lambda n: _llama_blocks(n, 64, 128), 8), (lambda n: _llama_blocks(n, 256, 512), 16),
+                                        (lambda n: _norms(n, 4096), 8), (lambda n: _norms(n, 128), 1)])
+def test_host_time_is_linear_in_launches(make, per_8):
+    """Eight times the launches cost about eight times the host time (the search that tried every
+    length from every start: 50 times and more)."""
+    few, t_few = hip_stub.run(make(8), passes=20)
+    many, t_many = hip_stub.run(make(64), passes=20)
+    assert len(few) == per_8
+    assert t_many <= 20 * t_few
