@@ -1771,7 +1771,14 @@ size_t enqueue_chain(RunEnv& E, const std::vector<PlanItem>& items, size_t i0, h
     bool late = false;
     for (size_t j = i0; j < i0 + kChainLaunches && fits(j); ++j) {
         auto r = ready.find(j);
-        if (r == ready.end()) r = ready.emplace(j, build_launch(E, launch(j))).first;
+        if (r == ready.end()) {
+            try {
+                r = ready.emplace(j, build_launch(E, launch(j))).first;
+            } catch (const std::exception&) {
+                if (j == i0) throw;
+                break;  // thrown again at its own turn, after the launches before it
+            }
+        }
         key.clear();
         if (!chain_join(E, C, launch(j), kernel(j), items[j].launch, r->second, key)) break;
         if (j == i0) {

@@ -172,3 +172,23 @@ def test_host_time_is_linear_in_launches(make, per_8):
     many, t_many = hip_stub.run(make(64), passes=20)
     assert len(few) == per_8
     assert t_many <= 20 * t_few
+
+
+def test_error_comes_after_the_launches_before_it():
+    """A launch whose tiles leave their tensor is an error at its own turn: those before it run."""
+    R, C = 16, 32
+    X, Y, Z = (W.T(np.zeros((4, R, C), np.float32)) for _ in range(3))
+    scale = _scale_kernel(R, C)
+
+    @workload
+    def wl():
+        for t in P(Dense[4]()):
+            scale[t](x=X[t], y=Y[t])
+        for t in P(Dense[4]()):
+            scale[t](x=Y[t], y=Z[t])
+        for t in P(Dense[4]()):
+            scale[t](x=Z[t], y=Y[t + 1])
+
+    with pytest.raises(RuntimeError, match="tiles of param y"):
+        hip_stub.run(W.rr4(wl()))
+    assert hip_stub.recorded() == ["ptowsp_rows_scale"]  # the first two, chained
