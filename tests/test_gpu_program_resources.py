@@ -1,11 +1,12 @@
 """Programs made and dropped in turn: the error flag, events and launch scratch of one pass to the
 next (ptowsp_program::take_resources), whatever kind of launch left its partials there.
 
-Against float64 with the GEMM tests' 1e-5 relative Frobenius (exact products, fp32 sums of K terms),
-and the error flag of a run that failed against the run after it."""
+Against float64 with the GEMM tests' 1e-5 relative Frobenius (exact products, fp32 sums of K terms).
+A run that ended with an error leaves flag and counters clear for the program after it."""
 
 import gc
 
+import numpy as np
 import pytest
 
 import workloads as W
@@ -58,3 +59,46 @@ def test_live_programs_do_not_share(gpu):
         for prog, t, c0, st in runs:
             prog.synchronize()
             _check(t["c"], t, c0)
+
+
+@pytest.mark.parametrize("fault", ["pages", "index"])
+def test_resources_of_a_failed_run(gpu, fault):
+    """A decode that ends with an error (a page count above its maximum, a page index out of range:
+    both cut by the kernel's own checks) passes its flag and counters on; the runs after it find
+    neither an error nor a count."""
+    from pto_wsp import ExecutionError
+
+    a = W.paged_decode_arrays([2100], 1, 1, 128, seed=1)
+    if fault == "pages":
+        a["npages"][0] = a["page_table"].shape[1] + 1
+    else:
+        a["page_table"][0, 70] = a["k_cache"].shape[0]
+    prog = W.rr4(W.paged_decode(a)).compile(target="hip_gfx950")
+    assert prog._native.kernel_family("decode_page") == "decode"
+    prog.execute()
+    with pytest.raises(ExecutionError, match="declared maximum" if fault == "pages" else "out of range"):
+        prog.synchronize()
+    del prog
+    gc.collect()
+    decode_many_partials(gpu, [2100], 1, 1, 128, 16, "bf16")
+    gc.collect()
+    _gemm(gpu, 16, 512, 1024)
+
+
+def test_failed_run_then_the_same_program(gpu):
+    """The program whose run failed runs again with its tensors put right."""
+    from pto_wsp import ExecutionError
+
+    a = W.paged_decode_arrays([2100], 1, 1, 128, seed=1)
+    good = a["page_table"].copy()
+    a["page_table"][0, 70] = a["k_cache"].shape[0]
+    prog = W.rr4(W.paged_decode(a)).compile(target="hip_gfx950")
+    prog.execute()
+    with pytest.raises(ExecutionError, match="out of range"):
+        prog.synchronize()
+    a["page_table"][:] = good
+    a["m"][:], a["l"][:], a["o"][:] = -np.inf, 0.0, 0.0
+    prog.execute()
+    prog.synchronize()
+    ref = W.paged_decode_ref(a)
+    assert np.linalg.norm(a["out"] - ref) <= 1e-5 * np.linalg.norm(ref)
