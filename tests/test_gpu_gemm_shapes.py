@@ -82,6 +82,28 @@ def test_gemm_few_stages(gpu, dt, k, B, M, N):
     test_gemm_shape(gpu, dt, B, M, N, k, (16, 16, 32))
 
 
+@pytest.mark.parametrize("dt,M,N,K", [("bf16", 80, 144, 320), ("f32", 80, 144, 320), ("bf16", 80, 144, 4096)])
+def test_gemm_edges_special_values(gpu, dt, M, N, K):
+    """Blocks with edges, K whole and in parts: what is not finite in A's last row or B's first column
+    (which the rows and columns past the edges read again) stays in its own row and column."""
+    import torch
+
+    t = _data(gpu, dt, 1, M, N, K, seed=3)
+    t["a"][0, M - 1, 5] = float("inf")
+    t["a"][0, 3, K - 1] = float("nan")
+    t["b"][0, 7, 0] = float("-inf")
+    c = t["c"].clone()
+    wdt = {"bf16": W.BF16, "f32": W.F32}[dt]
+    prog = W.rr4(W.bgemm({"a": t["a"], "b": t["b"], "c": c}, 16, 16, 16, wdt)).compile(target="hip_gfx950")
+    prog.execute()
+    prog.synchronize()
+    want = t["c"].double() + t["a"].double() @ t["b"].double()
+    assert torch.equal(torch.isnan(c), torch.isnan(want)) and torch.equal(torch.isinf(c), torch.isinf(want))
+    ok = torch.isfinite(want)
+    assert int(ok.sum()) == (M - 2) * (N - 1)
+    assert float((c[ok].double() - want[ok]).norm() / want[ok].norm()) <= 1e-5
+
+
 @pytest.mark.parametrize("M,N,K,tk", [(48, 256, 512, 256), (160, 192, 1024, 1024), (32, 512, 1024, 512)])
 def test_gemm_plain_last_step(gpu, M, N, K, tk):
     """store(c, matmul(a, b)) under a K loop: the last step's product, in stages and parts."""
