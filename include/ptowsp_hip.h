@@ -70,11 +70,12 @@ int ptowsp_hip_launch(ptowsp_program* prog, RuntimeContext* ctx, void* hip_strea
 /* No counterpart in the reference.  For callers that cannot allocate memory
  * (tight serving loops, harnesses that forbid hipMalloc): the same run as
  * ptowsp_hip_launch, allocating no device or pinned memory and loading no
- * code objects.  The decode kernels' unit counters and partials, the
- * kernels' error flag and the copy of device-resident loop-extent tensors
- * use a fixed device scratch of 16 MiB per GPU (held until the process
- * ends); a run that needs more is refused with an error before its decode
- * launch.  Requirements: every tensor is device memory; each launch's
+ * code objects.  The counters and partials of decode launches and of GEMM
+ * launches that sum K in parts, the kernels' error flag and the copy of
+ * device-resident loop-extent tensors (at its tail) use a fixed device
+ * scratch of 16 MiB per GPU (held until the process ends); a run whose decode
+ * needs more is refused with an error before that launch, and a GEMM sums K
+ * in as many parts as the scratch holds.  Requirements: every tensor is device memory; each launch's
  * kernel was already built and loaded by an earlier ptowsp_hip_launch of
  * the same program (same bindings), which also resolves the device's
  * scratch and loads the kernel that clears it (without one on this device
@@ -82,8 +83,9 @@ int ptowsp_hip_launch(ptowsp_program* prog, RuntimeContext* ctx, void* hip_strea
  * (cond-on-grid) launches or tile programs whose tiles exceed LDS (those
  * keep tiles in an allocated global scratch).  It is not made for HIP stream capture: it
  * records timing events and may read index tensors with synchronous
- * copies.  All no-allocation runs on one GPU share its scratch: runs that
- * overlap in time on one GPU race and must not be issued.  Finish with
+ * copies.  All no-allocation runs on one GPU share its scratch, whatever
+ * kernels they launch: runs that overlap in time on one GPU race and must not
+ * be issued.  Finish with
  * ptowsp_hip_synchronize as usual; device time is reported only when an
  * earlier ptowsp_hip_launch created the program's timing events. */
 int ptowsp_hip_launch_noalloc(ptowsp_program* prog, RuntimeContext* ctx, void* hip_stream, ptowsp_run_info* info);

@@ -9,9 +9,10 @@ namespace ptowsp {
 
 // Size of the per-device scratch array.  Layout used by a no-allocation run:
 //   [0, 256)            the kernels' error flag (int at offset 0);
-//   [256, 256 + 16 KiB) decode unit counters (kDecodeMaxUnits int32);
-//   then the device-resident loop-extent tensors the cycle model reads;
-//   then the decode partials.
+//   [256, 256 + 16 KiB) counters (kScratchCounters int32): one per decode unit,
+//                       or per C block of a GEMM launch that splits K;
+//   then the partials of those launches;
+//   at the tail, the device-resident loop-extent tensors the cycle model reads.
 constexpr size_t kNoAllocScratchBytes = size_t(16) << 20;
 constexpr size_t kNoAllocHeaderBytes = 256;
 

@@ -129,7 +129,7 @@ struct ptowsp_program {
     size_t key_stage_elems = 0;
     ptowsp_run_info last_run{};  // cycle model result of the last synchronized run
     std::string precompiled_source;
-    void* scratch = nullptr;  // decode: unit counters and partials
+    void* scratch = nullptr;  // counters and partials of decode and split-K GEMM launches
     size_t scratch_bytes = 0;
     void* gtile = nullptr;    // tile programs: tiles beyond LDS, one region per workgroup
     size_t gtile_bytes = 0;
@@ -326,7 +326,7 @@ struct RunEnv {
     bool replay_slots = false;                     // cycle model: slot loads replay P->slot_log
     bool timing = true;                            // record ev0 / ev1 (the program's events exist)
     // No-allocation run: the kernels' error flag, and the device scratch that
-    // replaces the program's hipMalloc'd decode scratch (counters at
+    // replaces the program's hipMalloc'd launch scratch (counters at
     // nscratch + kNoAllocHeaderBytes, partials after them, nscratch_limit
     // bytes usable from nscratch).
     int* err = nullptr;
@@ -2205,7 +2205,7 @@ void defer_cycles(RunEnv& E, const std::vector<int>& tids, hipStream_t stream) {
 
 // Both launch entry points.  noalloc: the run allocates no device or pinned
 // memory: every tensor must already be in device memory, the kernels' error
-// flag and the decode scratch live in the fixed device scratch of
+// flag and the launch scratch live in the fixed device scratch of
 // noalloc.hip, the deferred cycle-model input is copied there too, and
 // features whose host steps need staging buffers are refused.
 int launch_impl(ptowsp_program* P, RuntimeContext* ctx, void* hip_stream, ptowsp_run_info* info, bool noalloc) {

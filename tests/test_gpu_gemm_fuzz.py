@@ -2,13 +2,12 @@
 
 Each seed draws a task tile (tm, tn in {64, 128, 256}, tk in {16, 32, 64,
 128}, within the LDS budget of the GEMM family), a batch, tile counts along
-M, N and K (odd counts leave the 2x2 block merge half used or off), the
+M, N and K (C is cut into blocks of its own, which odd counts leave partial), the
 input dtype (f16 / bf16, or f32 for about a third of the seeds: the f32
 block on v_mfma_f32_32x32x2_f32), the InOut accumulate form or the plain store, the
 order of the m and n loops, and seeded inputs with a random initial C (a
-second set of seeds draws tiles of 16 / 32, merged into MFMA blocks or run
-as tile programs, and of 512, split into 256-wide blocks, with K steps up to
-256).  The
+second set of seeds draws tiles of 16 / 32, covered by MFMA blocks or run
+as tile programs, and of 512, cut into blocks too, with K steps up to 256).  The
 GPU result must equal the oracle's within a relative Frobenius error of 1e-5
 (both accumulate exact products in fp32, in different orders), with equal
 cycle counts.
