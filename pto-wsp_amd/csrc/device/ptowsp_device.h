@@ -1841,7 +1841,7 @@ struct GemmPingPong {
 //    lanes l%16 + 16*i with two lane swaps (v_permlane32_swap,
 //    v_permlane16_swap), so every lane of the row ends with the result;
 //  * p @ v on the matrix cores (v_mfma_f32_16x16x16, p split into two
-//    16-bit parts), lane l supplying tokens 4*(l/16)..+3 of every page for
+//    or three 16-bit parts, split4), lane l supplying tokens 4*(l/16)..+3 of every page for
 //    head dims (D/16)*(l%16)+e and accumulating query rows 4*(l/16)..+3.
 
 
@@ -1879,10 +1879,11 @@ __device__ inline void reset_count(int* cnt) {
 // F32: f32 q, K and V (the reference's own dtype): scores on
 // v_mfma_f32_16x16x4_f32 with lane l holding head dims 16*j + 4*(l/16) .. +3
 // of its token for j < D/16 (the K order of a product is free), p @ v on the same MFMA
-// with p as it is (no hi / lo split); F16 is then unused.
+// with p as it is (no split); F16 is then unused.
 // RM: the [1, 16] mask is a row broadcast (the reference's rule for a square
 // score tile): one value per query row, mask[r] for row r, G == 16.
-template <int G, int D, bool F16, bool MASK, bool H8 = false, bool F32 = false, bool RM = false>
+// FEW: a launch of few units (see kParts).
+template <int G, int D, bool F16, bool MASK, bool H8 = false, bool F32 = false, bool RM = false, bool FEW = false>
 struct DecodeWave {
     static_assert(G >= 1 && G <= 48 && (D == 64 || D == 128 || D == 256), "decode shape");
     static_assert(!F32 || D <= 128 || G <= 16, "f32 decode shape");
@@ -2021,19 +2022,42 @@ struct DecodeWave {
     };
 
     typedef float f32x2_t __attribute__((ext_vector_type(2)));
-    // hi + lo == x for four fp32 values x to about 2^-17 (bf16) / 2^-22 (f16)
-    // relative: hi = x rounded to 16 bits, lo = (x - hi) rounded (x - hi is
-    // exact in fp32).  Packed two per dword, element 0 in the low half.
+    // Four fp32 values x >= 0 as the sum of kParts values of 16 bits, packed
+    // two per dword, element 0 in the low half.  Two parts: x rounded, then the
+    // rest (exact in fp32) rounded, x to about 2^-18 (bf16) / 2^-22 (f16).
+    // Three bf16 parts, 8 of x's 24 bits each: x itself.
+    // bf16 takes three: 2^-18 of x is far above the error of the fp32 sums, and
+    // more of it is left the fewer waves share a unit (x is exactly 1 for the
+    // tokens that set a wave's maximum).  Two sequences of 512-8192 tokens at
+    // the C5 heads, error against 64 bits: two parts 1.8e-6 over 1024 waves and
+    // 2.0e-6 over those that waves_for takes, three 2.5e-7; the pass 72.2 and
+    // 72.9 us, 64 sequences level.  Beyond 16 query rows, where the fold bounds
+    // the launch, the third product costs (48 rows 240 us, 252 with it): there
+    // it is taken only where the host knows that the units are few (FEW; two
+    // sequences with 32 rows 115 us over fewer waves, 184 over all), and a
+    // launch with two parts uses all waves.
+    static constexpr int kParts = F16 || (RB > 1 && !FEW) ? 2 : 3;
+    static constexpr bool kAllWaves = !F32 && !F16 && kParts == 2;
     template <bool H, class A, class B> struct Pick { typedef B type; };
     template <class A, class B> struct Pick<true, A, B> { typedef A type; };
-    __device__ static void split4(f32x4v_t x, u32x2& hi, u32x2& lo) {
-        typedef typename Pick<F16, _Float16, __bf16>::type h_t;
-        typedef h_t h2_t __attribute__((ext_vector_type(2)));
-        const f32x2_t x0 = {x[0], x[1]}, x1 = {x[2], x[3]};
-        const h2_t a = __builtin_convertvector(x0, h2_t), b = __builtin_convertvector(x1, h2_t);
-        const f32x2_t r0 = x0 - __builtin_convertvector(a, f32x2_t), r1 = x1 - __builtin_convertvector(b, f32x2_t);
-        hi = u32x2{__builtin_bit_cast(u32, a), __builtin_bit_cast(u32, b)};
-        lo = u32x2{__builtin_bit_cast(u32, __builtin_convertvector(r0, h2_t)), __builtin_bit_cast(u32, __builtin_convertvector(r1, h2_t))};
+    __device__ static void split4(f32x4v_t x, u32x2 (&p)[kParts]) {
+        if constexpr (kParts == 2) {
+            typedef typename Pick<F16, _Float16, __bf16>::type h_t;
+            typedef h_t h2_t __attribute__((ext_vector_type(2)));
+            const f32x2_t x0 = {x[0], x[1]}, x1 = {x[2], x[3]};
+            const h2_t a = __builtin_convertvector(x0, h2_t), b = __builtin_convertvector(x1, h2_t);
+            const f32x2_t r0 = x0 - __builtin_convertvector(a, f32x2_t), r1 = x1 - __builtin_convertvector(b, f32x2_t);
+            p[0] = u32x2{__builtin_bit_cast(u32, a), __builtin_bit_cast(u32, b)};
+            p[1] = u32x2{__builtin_bit_cast(u32, __builtin_convertvector(r0, h2_t)), __builtin_bit_cast(u32, __builtin_convertvector(r1, h2_t))};
+        } else {
+#pragma unroll
+            for (int i = 0; i < kParts; ++i) {
+                p[i] = u32x2{__builtin_amdgcn_perm(__float_as_uint(x[1]), __float_as_uint(x[0]), 0x07060302u),
+                             __builtin_amdgcn_perm(__float_as_uint(x[3]), __float_as_uint(x[2]), 0x07060302u)};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[e] = x[e] - __uint_as_float(__float_as_uint(x[e]) & 0xFFFF0000u);
+            }
+        }
     }
     // v_mfma_f32_16x16x16 (bf16 / f16): lane l holds A[l%16][4*(l/16)..+3],
     // B[4*(l/16)..+3][l%16] and D[4*(l/16)..+3][l%16].
@@ -2078,7 +2102,7 @@ struct DecodeWave {
         auto fmax_ = [](float x, float y) { return fmaxf(x, y); };
         auto fadd_ = [](float x, float y) { return x + y; };
         float a[RB];
-        u32x2 ph[RB], pl[RB];
+        u32x2 pp[RB][kParts];
         f32x4v_t pf[RB];
         bool rescale[RB];
 #pragma unroll
@@ -2100,12 +2124,12 @@ struct DecodeWave {
             st.m[rb] = mn;
             rescale[rb] = __builtin_amdgcn_ballot_w64(16 * rb + t < G && a[rb] != 1.0f) != 0;
             if constexpr (F32) pf[rb] = pr;
-            else split4(pr, ph[rb], pl[rb]);
+            else split4(pr, pp[rb]);
         }
         // o <- o * a + p @ v on the matrix cores: v_mfma_f32_16x16x16 with
         // M = query rows, K = the page's 16 tokens, N = 16 head dims.  p is
-        // fp32 and enters as hi + lo (split4), two products per MFMA step;
-        // the lane's scores are already its A operand (query row l%16,
+        // fp32 and enters in parts of 16 bits (split4), a product per part and
+        // MFMA step; the lane's scores are already its A operand (query row l%16,
         // tokens 4*(l/16)..+3).  MFMA e covers head dims DV*n + e (n = l%16):
         // lane (n, l/16) supplies V[tokens 4*(l/16)..+3][DV*n + e] straight
         // from its page registers (one 16-bit half of pg.v[i][e/2] per token)
@@ -2145,10 +2169,9 @@ struct DecodeWave {
                 const u32x2 bv = {__builtin_amdgcn_perm(pg.v[1][e >> 1], pg.v[0][e >> 1], sel),
                                   __builtin_amdgcn_perm(pg.v[3][e >> 1], pg.v[2][e >> 1], sel)};
 #pragma unroll
-                for (int rb = 0; rb < RB; ++rb) {
-                    st.o[rb][e] = mfma16(ph[rb], bv, st.o[rb][e]);
-                    st.o[rb][e] = mfma16(pl[rb], bv, st.o[rb][e]);
-                }
+                for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+                    for (int i = 0; i < kParts; ++i) st.o[rb][e] = mfma16(pp[rb][i], bv, st.o[rb][e]);
             }
         }
     }

@@ -1116,8 +1116,8 @@ EmittedKernel emit_decode(const Module& m, const KernelAnalysis& a, const Launch
     auto nterms = [&](int p) { return spec.indirect_count[p]; };
     const std::string tmpl = "DecodeWave<" + std::to_string(d.g) + ", " + std::to_string(d.d) + ", " +
                              (d.f16 ? "true" : "false") + ", " + (d.mask >= 0 ? "true" : "false") + ", " +
-                             (d.pg == 8 ? "true" : "false") + (d.f32 || d.row_mask ? (d.f32 ? ", true" : ", false") : "") +
-                             (d.row_mask ? ", true" : "") + ">";
+                             (d.pg == 8 ? "true" : "false") + (d.f32 || d.row_mask || spec.decode_few ? (d.f32 ? ", true" : ", false") : "") +
+                             (d.row_mask || spec.decode_few ? (d.row_mask ? ", true" : ", false") : "") + (spec.decode_few ? ", true" : "") + ">";
     const int es = d.f32 ? 4 : 2;  // bytes per q / K / V element
     std::ostringstream scale;
     scale.precision(9);
@@ -1248,7 +1248,7 @@ EmittedKernel emit_decode(const Module& m, const KernelAnalysis& a, const Launch
     // page, returns here; a unit's partials fill consecutive slots).  When not
     // all are active they are spread over the blocks.
     o << "  const int AW = static_cast<int>(gridDim.x) * " << nw << ";\n";
-    o << "  const i64 W = DecodeSplit::waves_for(TC, U, AW);\n";
+    o << "  const i64 W = DW::kAllWaves ? (AW < TC ? AW : TC) : DecodeSplit::waves_for(TC, U, AW);\n";
     o << "  const i64 w = W < AW ? static_cast<int>(blockIdx.x + gridDim.x * wave) : static_cast<int>(blockIdx.x * " << nw << " + wave);\n";
     o << "  if (w < W) {\n";
     o << "  const i64 s = DecodeSplit::page_at(pre, cpre, U, w * TC / W);\n";

@@ -64,13 +64,14 @@ struct EmitSpec {
     int decode_ring = 4;
     int decode_waves = 4;
     bool decode_ordered = false;  // release / acquire fences around the unit completion count
+    bool decode_few = false;      // bf16, more than 16 query rows: so few units that the launch uses fewer waves
 
     bool operator==(const EmitSpec& o) const {
         auto all = [](const EmitSpec& s) {
             return std::tie(s.vec_width, s.row_unit_cols, s.indirect_count, s.inner_dyn_term, s.threads, s.serial, s.row_loops, s.seq_mask,
                             s.task_list, s.row_up, s.nontemporal, s.tile_mma, s.gemm, s.gemm_vm, s.gemm_vn, s.gemm_bm, s.gemm_bn, s.gemm_kf,
                             s.gemm_ring, s.gemm_split, s.gemm_edge, s.gemm_pingpong, s.decode, s.decode_norm, s.decode_ring, s.decode_waves,
-                            s.decode_ordered);
+                            s.decode_ordered, s.decode_few);
         };
         return all(*this) == all(o);
     }

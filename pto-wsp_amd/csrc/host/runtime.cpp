@@ -1268,6 +1268,14 @@ BuiltLaunch build_launch(RunEnv& E, const LaunchSpec& L) {
     B.spec.decode_ring = tuning().decode_ring ? tuning().decode_ring : decode_ring_for(a.decode.d, a.decode.g, a.decode.f32);
     B.spec.decode_waves = tuning().decode_waves ? tuning().decode_waves : decode_waves_for(a.decode.d, a.decode.g, a.decode.f32);
     B.spec.decode_ordered = tuning().decode_ordered;
+    if (B.spec.decode && a.decode.g > 16 && !a.decode.f16 && !a.decode.f32) {
+        // However long the units are, DecodeSplit::waves_for takes fewer than
+        // the waves of 256 CUs.
+        const Axis& ax = *L.inner[0].axis;
+        const int64_t sub = std::max(1, a.decode.pg / 16), waves = 256 * B.spec.decode_waves;
+        const int64_t cost = std::max<int64_t>(0, ax.kind == AxisKind::DynTensor ? ax.max : A.ext[ng]) * sub + kDecodeUnitCost;
+        B.spec.decode_few = cost * B.ntasks < waves * waves / std::max<int64_t>(1, B.ntasks);
+    }
     B.spec.vec_width = a.family == Family::RowProgram ? pick_vec_width(a, A, nvars) : 1;
     B.spec.row_unit_cols = a.family == Family::RowProgram && row_unit_columns(a, A);
     B.spec.threads = tuning().tile_threads;

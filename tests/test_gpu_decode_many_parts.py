@@ -1,9 +1,9 @@
 """Paged decode with few units over all the waves: each unit is split into many partials, which
 one wave folds after its stream (DecodeCombine::run_many, DecodeSplit::waves_for).
 
-Against float64 attention.  A page's scores and p @ v carry about 2^-17 relative for 16-bit pages
-(p enters as two 16-bit parts) and 2^-24 for f32, and the fold of n partials adds a rounding per
-partial, so the decode tests' bound of 1e-5 relative Frobenius holds whatever the split."""
+Against float64 attention.  p @ v carries at least 2^-18 relative (p enters in 16-bit parts), and the
+fold of n partials adds a rounding per partial, so the decode tests' bound of 1e-5 relative Frobenius
+holds whatever the split."""
 
 import numpy as np
 import pytest
@@ -56,10 +56,33 @@ def test_many_partials(gpu, lengths, hkv, G, D, page, kind):
     np.testing.assert_array_equal(got[live], o / l)
 
 
+def _error(gpu, lengths, G, D):
+    import torch
+
+    a = W.paged_decode_arrays(lengths, 8, G, D, 16, seed=7)
+    t = {k: torch.from_numpy(v.view(np.int16)).to(gpu).view(torch.bfloat16) if v.dtype == np.uint16 else torch.from_numpy(v).to(gpu)
+         for k, v in a.items() if k != "lengths"}
+    prog = W.rr4(W.paged_decode(t)).compile(target="hip_gfx950")
+    prog.execute()
+    prog.synchronize()
+    ref = W.paged_decode_ref(a)
+    return np.linalg.norm(t["out"].cpu().numpy() - ref) / np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("G,D", [(1, 128), (4, 128), (7, 64), (12, 256), (20, 128), (48, 64)])
+def test_few_units_are_as_exact_as_many(gpu, G, D):
+    """bf16 p @ v takes the whole of p: what is left are the roundings of the fp32 sums, about
+    sqrt(100) * 2^-24 = 6e-7 for a wave's pages and the fold.  Two bf16 parts of p would leave
+    2^-18 / sqrt(3) = 2.2e-6, and the more of it the fewer waves share a unit."""
+    assert _error(gpu, [6000, 3111], G, D) <= 1e-6
+    if G <= 16:  # beyond, launches over all waves keep two parts
+        assert _error(gpu, [700] * 40, G, D) <= 1e-6
+
+
 def test_many_partials_special_values(gpu):
     """A value that is not finite in one page of one head, the lowest mask over whole runs of pages:
-    only that head's value column is not finite (infinity or NaN: p enters as two 16-bit parts, the second
-    of either sign), and masked pages weigh nothing."""
+    only that head's value column is not finite (infinity or NaN: p enters in 16-bit parts, and a part may
+    be zero), and masked pages weigh nothing."""
     import torch
 
     a = W.paged_decode_arrays([2100, 1900], 2, 4, 128, seed=5)
