@@ -1086,6 +1086,18 @@ EmittedKernel emit_gemm(const Module& m, const KernelAnalysis& a, const LaunchSp
     }
     o << "}\n";
     ek.source = o.str();
+    if (split) {
+        // The same blocks with K whole, for launches that are captured; a kernel
+        // of its own in the module, since one kernel with both forms held more
+        // registers in its split path (16 x 8192 x 4096 bf16, a pass: 37.2 us,
+        // 38.6 with the choice inside the block, 46.6 with a path for each).
+        EmitSpec whole = spec;
+        whole.gemm_split = 1;
+        std::string w = emit_gemm(m, a, L, whole).source;
+        w = w.substr(w.find("extern \"C\""));
+        ek.whole_entry = ek.entry + "_whole";
+        ek.source += w.replace(w.find(ek.entry), ek.entry.size(), ek.whole_entry);
+    }
     ek.lds_bytes = pp ? static_cast<size_t>((bk == 64 ? 2 : 4) * 512 * bk * 2 + 256) : static_cast<size_t>(ns * (bm + bn) * bk * es);
     return ek;
 }

@@ -94,6 +94,7 @@ inline int gemm_waves_m(int bm) { return bm == 32 ? 1 : 2; }
 
 struct EmittedKernel {
     std::string source;
+    std::string whole_entry;    // GEMM with K in parts: the kernel that takes K whole
     std::string entry;          // kernel symbol
     int threads = 256;
     int rows_per_chunk = 0;     // row programs: rows handled per wave iteration

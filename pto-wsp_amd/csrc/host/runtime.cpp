@@ -65,6 +65,7 @@ struct LaunchCache {
         EmitSpec spec;
         EmittedKernel ek;
         const JitKernel* jk = nullptr;
+        hipFunction_t whole = nullptr;  // EmittedKernel::whole_entry
     };
     std::vector<std::unique_ptr<Entry>> entries;
 };
@@ -236,8 +237,8 @@ struct ptowsp_program {
     void give_back() {
         Resources r{res_dev, h_err, d_err, ev0, ev1, scratch, scratch_bytes};
         // Only whole sets whose last run has been waited for and ended well: its
-        // counters are at zero.  A stream that was captured may have put the
-        // events and the scratch into a graph, which can outlive the program.
+        // counters are at zero.  A captured run has put the error flag and a
+        // decode's scratch into a graph.
         const bool keep = res_dev >= 0 && h_err && have_events && !broken && !pending && !captured && scratch_bytes <= kPoolScratch;
         if (keep) {
             __atomic_store_n(h_err, 0, __ATOMIC_RELAXED);
@@ -332,6 +333,7 @@ struct RunEnv {
     int* err = nullptr;
     char* nscratch = nullptr;
     size_t nscratch_limit = 0;
+    bool capturing = false;  // the stream is being captured into a graph
     // Bytes of launch scratch that a no-allocation run of the program would
     // have: every run stays below it where it has a choice, so that both
     // entry points run the same kernels.
@@ -1406,6 +1408,8 @@ void enqueue_built(RunEnv& E, int li, BuiltLaunch& B, hipStream_t stream, uint64
             entry.jk = &jit_kernel(ek.source, ek.entry);
         }
     }
+    if (!ek.whole_entry.empty() && !entry.whole)
+        check(hipModuleGetFunction(&entry.whole, entry.jk->module, ek.whole_entry.c_str()), "hipModuleGetFunction");
     const JitKernel* jk = entry.jk;
     if (B.spec.decode) {
         enqueue_decode(E, li, B, ek, *jk, stream, launches);
@@ -1413,7 +1417,11 @@ void enqueue_built(RunEnv& E, int li, BuiltLaunch& B, hipStream_t stream, uint64
     }
     if (B.spec.task_list) B.args.tlist = reinterpret_cast<const i64*>(upload_task_list(E, B.tasks, stream));
     const LaunchSpec& L = P->plan.launches[li];
-    if (B.spec.gemm && B.spec.gemm_split > 1) {
+    // A captured GEMM takes K whole: a graph may be replayed beside others of the
+    // same program, or after its scratch has gone.
+    const bool split = B.spec.gemm && B.spec.gemm_split > 1 && (!E.capturing || E.nscratch);
+    const bool whole = B.spec.gemm && B.spec.gemm_split > 1 && !split;
+    if (split) {
         const size_t need = gemm_scratch_bytes(B.gemm_tiles, B.spec.gemm_split, B.spec.gemm_bm, B.spec.gemm_bn);
         const int ntens = static_cast<int>(P->ka[L.kernel].tensor_param_index.size());
         B.args.base[ntens] = launch_scratch(E, need);
@@ -1452,7 +1460,7 @@ void enqueue_built(RunEnv& E, int li, BuiltLaunch& B, hipStream_t stream, uint64
     } else {
         blocks = B.ntasks;
     }
-    if (B.spec.gemm && !B.spec.serial) blocks = B.gemm_tiles * B.spec.gemm_split;  // exactly one block per workgroup
+    if (B.spec.gemm && !B.spec.serial) blocks = B.gemm_tiles * (split ? B.spec.gemm_split : 1);  // exactly one block per workgroup
     else blocks = std::min<int64_t>(blocks, int64_t(1) << 20);
     blocks = std::max<int64_t>(1, blocks);
     if (ek.gtile_bytes > 0) {
@@ -1480,7 +1488,7 @@ void enqueue_built(RunEnv& E, int li, BuiltLaunch& B, hipStream_t stream, uint64
         B.args.span[ntens] = static_cast<int64_t>(need / sizeof(float));
     }
     void* params[] = {&B.args};
-    launch_kernel(E, jk->function, blocks, ek.threads, 0, stream, params, "hipModuleLaunchKernel");
+    launch_kernel(E, whole ? entry.whole : jk->function, blocks, ek.threads, 0, stream, params, "hipModuleLaunchKernel");
     ++launches;
 }
 
@@ -2225,6 +2233,7 @@ int launch_impl(ptowsp_program* P, RuntimeContext* ctx, void* hip_stream, ptowsp
     P->broken = true;  // until the run is enqueued
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(stream, &capture) != hipSuccess) (void)hipGetLastError();
+    E.capturing = capture != hipStreamCaptureStatusNone;
     P->captured |= noalloc || capture != hipStreamCaptureStatusNone;
     if (noalloc) {
         const char* who = "ptowsp_hip_launch_noalloc: ";

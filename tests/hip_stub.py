@@ -3,6 +3,7 @@ HIP runtime without a device (hip_stub.cpp).  Kernels are emitted and built for 
 always; launches are recorded instead of run, so tensors may be views of any size over a small
 buffer."""
 
+import contextlib
 import ctypes
 import hashlib
 import os
@@ -52,6 +53,8 @@ def _library():
     lib.stub_entry.restype = ctypes.c_char_p
     for name in ("stub_blocks", "stub_threads"):
         getattr(lib, name).restype = ctypes.c_uint64
+    lib.stub_base.restype = ctypes.c_void_p
+    lib.stub_freed.argtypes = [ctypes.c_void_p]
     for name in ("stub_s3", "stub_s4", "stub_coef"):
         getattr(lib, name).restype = ctypes.c_int64
     return lib
@@ -68,6 +71,7 @@ class Launch:
     s3: list
     s4: list
     coef: list
+    base: list
 
 
 def recorded():
@@ -75,32 +79,58 @@ def recorded():
     return [_lib.stub_entry(i).decode() for i in range(_lib.stub_num_launches())]
 
 
-def run(workload, passes=1):
-    """Launches of one pass of `workload` (after `passes` - 1 others), and the last pass's host time in seconds."""
+def _launches(prog):
+    out = []
+    for i in range(_lib.stub_num_launches()):
+        out.append(Launch(_lib.stub_entry(i).decode(), _lib.stub_blocks(i), _lib.stub_threads(i),
+                          [_lib.stub_s3(i, p) for p in range(12)], [_lib.stub_s4(i, p) for p in range(12)],
+                          [[_lib.stub_coef(i, p, v) for v in range(8)] for p in range(12)], [_lib.stub_base(i, p) for p in range(12)]))
+    assert prog.stats.launches == len(out)
+    return out
+
+
+def freed(pointer):
+    """Whether device memory that a launch was given has been freed."""
+    return bool(_lib.stub_freed(pointer))
+
+
+@contextlib.contextmanager
+def program(workload):
+    """`workload` compiled for the recorded runtime: a function that runs it once (capture: on a stream
+    that is being captured) and returns its launches."""
     global _lib
     if _lib is None:
         _lib = _library()
     real, _hip._lib = _hip._lib, _lib
     prog = None
+
+    def once(capture=False):
+        _lib.stub_clear()
+        _lib.stub_capture(int(capture))
+        try:
+            prog.execute()
+        finally:
+            _lib.stub_capture(0)
+        prog.synchronize()
+        return _launches(prog)
+
     try:
         prog = workload.compile(target="hip_gfx950")
-        best = 1e9
-        for i in range(passes):
-            _lib.stub_clear()
-            t = time.perf_counter()
-            prog.execute()
-            prog.synchronize()
-            if i > 0 or passes == 1:
-                best = min(best, time.perf_counter() - t)
-        out = []
-        for i in range(_lib.stub_num_launches()):
-            out.append(Launch(_lib.stub_entry(i).decode(), _lib.stub_blocks(i), _lib.stub_threads(i),
-                              [_lib.stub_s3(i, p) for p in range(12)], [_lib.stub_s4(i, p) for p in range(12)],
-                              [[_lib.stub_coef(i, p, v) for v in range(8)] for p in range(12)]))
-        assert prog.stats.launches == len(out)
-        return out, best
+        yield once
     finally:
         if prog is not None:
             prog._native = None
-        del prog
+        prog = None
         _hip._lib = real
+
+
+def run(workload, passes=1):
+    """Launches of one pass of `workload`, and the host time in seconds of the fastest pass after the first."""
+    with program(workload) as once:
+        best = 1e9
+        for i in range(passes):
+            t = time.perf_counter()
+            launches = once()
+            if i > 0 or passes == 1:
+                best = min(best, time.perf_counter() - t)
+        return launches, best
