@@ -132,6 +132,7 @@ struct ptowsp_program {
     std::string precompiled_source;
     void* scratch = nullptr;  // counters and partials of decode and split-K GEMM launches
     size_t scratch_bytes = 0;
+    std::vector<void*> retired;  // launch scratch outgrown after a captured run
     void* gtile = nullptr;    // tile programs: tiles beyond LDS, one region per workgroup
     size_t gtile_bytes = 0;
     // Task lists of masked launches: pinned host chunks copied into device
@@ -184,6 +185,7 @@ struct ptowsp_program {
         for (void* b : stage_buf)
             if (b) (void)hipFree(b);
         if (key_stage) (void)hipHostFree(key_stage);
+        for (void* b : retired) (void)hipFree(b);
         give_back();
     }
     // Error flag, events and launch scratch, which every program needs for its
@@ -1343,7 +1345,9 @@ char* launch_scratch(RunEnv& E, size_t need) {
     if (E.nscratch) return E.nscratch + kNoAllocHeaderBytes;
     ptowsp_program* P = E.P;
     if (need > P->scratch_bytes) {
-        if (P->scratch) {
+        if (P->scratch && P->captured) {
+            P->retired.push_back(P->scratch);  // a graph may hold it
+        } else if (P->scratch) {
             // Earlier launches of this run may still use the smaller one.
             check(hipDeviceSynchronize(), "hipDeviceSynchronize");
             check(hipFree(P->scratch), "hipFree(scratch)");

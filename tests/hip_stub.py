@@ -116,11 +116,12 @@ def program(workload):
 
     try:
         prog = workload.compile(target="hip_gfx950")
+        once.prog = prog
         yield once
     finally:
         if prog is not None:
             prog._native = None
-        prog = None
+        once.prog = prog = None
         _hip._lib = real
 
 
