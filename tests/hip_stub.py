@@ -120,8 +120,7 @@ def program(workload):
         yield once
     finally:
         if prog is not None:
-            prog._native = None
-        once.prog = prog = None
+            prog._native.__del__()  # here and now: an exception's traceback may hold it beyond this library
         _hip._lib = real
 
 
