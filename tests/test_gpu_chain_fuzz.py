@@ -115,3 +115,91 @@ def test_random_chain(gpu, seed):
     for k, v in want.items():
         x = got[k].cpu().numpy().astype(np.float64)
         assert np.linalg.norm(x - v) <= 1e-5 * np.linalg.norm(v), (k, prog.stats.launches)
+
+
+def _make_loops(seed, arrs):
+    """Launches over a grid and in-kernel loops of the same extents, over arrs: t0..t3 [n, L, R, C],
+    v [1, C], accumulators s0, s1 [n, R, 1]."""
+    rng = np.random.default_rng(seed)
+    n, L, R, C = arrs["t0"].shape
+    T_, S, V = [W.T(arrs[f"t{i}"]) for i in range(4)], [W.T(arrs["s0"]), W.T(arrs["s1"])], W.T(arrs["v"])
+
+    @kernel
+    def halve(x: In[Tile[R, C, F32]], y: Out[Tile[R, C, F32]]):
+        pto.store(y, pto.add(pto.mul(x, pto.constant(0.5, F32)), pto.constant(0.25, F32)))
+
+    @kernel
+    def mean2(x: In[Tile[R, C, F32]], z: In[Tile[R, C, F32]], y: Out[Tile[R, C, F32]]):
+        pto.store(y, pto.mul(pto.add(x, z), pto.constant(0.5, F32)))
+
+    @kernel
+    def scale(x: In[Tile[R, C, F32]], v: In[Tile[1, C, F32]], y: InOut[Tile[R, C, F32]]):
+        pto.store(y, pto.mul(pto.add(x, y), v))
+
+    @kernel
+    def shift(x: In[Tile[R, C, F32]], s: In[Tile[R, 1, F32]], y: Out[Tile[R, C, F32]]):
+        pto.store(y, pto.mul(pto.sub(x, s), pto.constant(0.5, F32)))
+
+    @kernel
+    def fold_max(x: In[Tile[R, C, F32]], s: InOut[Tile[R, 1, F32]]):
+        pto.store(s, pto.max(s, pto.rowmax(x)))
+
+    @kernel
+    def fold_mean(x: In[Tile[R, C, F32]], s: InOut[Tile[R, 1, F32]]):
+        pto.store(s, pto.add(pto.mul(s, pto.constant(0.5, F32)), pto.rowmean(x)))
+
+    steps = []
+    for _ in range(int(rng.integers(2, 7))):
+        x, z, y = (int(i) for i in rng.integers(0, 4, 3))
+        if x == y:
+            y = (y + 1) % 4
+        op = str(rng.choice(["halve", "mean2", "scale", "shift", "fold_max", "fold_mean"]))
+        seq = op.startswith("fold") or rng.random() < 0.5
+        steps.append((op, x, z if z != y else x, y, seq, bool(rng.random() < 0.1), int(rng.integers(0, 2))))
+
+    def call(i, j, op, x, z, y, seq, first, s):
+        X, Y = T_[x][i][0 if first else j], T_[y][i][j]
+        if op == "halve":
+            halve[i, j](x=X, y=Y)
+        elif op == "mean2":
+            mean2[i, j](x=X, z=T_[z][i][j], y=Y)
+        elif op == "scale":
+            scale[i, j](x=X, v=V, y=Y)
+        elif op == "shift":
+            shift[i, j](x=X, s=S[s][i], y=Y)
+        elif op == "fold_max":
+            fold_max[i, j](x=X, s=S[s][i])
+        else:
+            fold_mean[i, j](x=X, s=S[s][i])
+
+    @workload
+    def wl():
+        for st in steps:
+            for i in P(Dense[n](), names=["outer"]):
+                for j in P.seq(Dense[L](), name="step") if st[4] else P(Dense[L](), names=["step"]):
+                    call(i, j, *st)
+
+    return W.rr4(wl())
+
+
+@pytest.mark.parametrize("seed", range(20))
+def test_random_loops(gpu, seed):
+    """Grid loops and in-kernel loops in turn over the same tiles, with accumulators in place."""
+    import torch
+
+    n, L, R, C = 3, (3, 5, 2, 1)[seed % 4], (4, 16, 3)[seed % 3], (32, 48, 19, 64)[seed % 4]
+    rng = np.random.default_rng(5000 + seed)
+    base = {f"t{i}": rng.standard_normal((n, L, R, C)) for i in range(4)}
+    base |= {f"s{i}": rng.standard_normal((n, R, 1)) for i in range(2)}
+    base["v"] = rng.uniform(0.3, 0.6, (1, C))
+    base = {k: v.astype(np.float32) for k, v in base.items()}
+    want = {k: v.copy() for k, v in base.items()}
+    ref = run_workload(_make_loops(seed, want))
+    got = {k: torch.from_numpy(v.copy()).to(gpu) for k, v in base.items()}
+    prog = _make_loops(seed, got).compile(target="hip_gfx950")
+    prog.execute()
+    prog.synchronize()
+    assert prog.stats.total_cycles == ref.total_cycles and prog.stats.task_count == ref.task_count
+    for k, v in want.items():
+        x = got[k].cpu().numpy().astype(np.float64)
+        assert np.linalg.norm(x - v) <= 1e-5 * np.linalg.norm(v), (k, prog.stats.launches)
