@@ -64,7 +64,10 @@ uint64_t ptowsp_hip_workload_main(ptowsp_program* prog, RuntimeContext* ctx, CSP
  * UINT64_MAX and ptowsp_hip_run_result gives it after the synchronize (the
  * reference also fills ProgramStats.total_cycles only when the run thread
  * ends, python/pto_wsp/program.py:721-733).  `ctx` must stay valid until
- * the synchronize. */
+ * the synchronize.  The launches of a program that has run with the same
+ * bindings may be captured into a HIP graph.  The graph then holds the
+ * tensors, the program's error flag and the scratch of its decode launches
+ * (keep the program); GEMM launches sum K whole in it and hold no scratch. */
 int ptowsp_hip_launch(ptowsp_program* prog, RuntimeContext* ctx, void* hip_stream, ptowsp_run_info* info);
 
 /* No counterpart in the reference.  For callers that cannot allocate memory

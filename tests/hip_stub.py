@@ -31,21 +31,21 @@ def _library():
     if not os.path.exists(path):
         os.makedirs(os.path.dirname(path), exist_ok=True)
         for old in os.listdir(os.path.dirname(path)):
-            if old.startswith("libptowsp_stub"):
+            if old.startswith("libptowsp_stub") and old.endswith(".so"):
                 os.unlink(os.path.join(os.path.dirname(path), old))
         procs = []
         for s in srcs:
-            o = f"{path}.{os.path.basename(s)}.o"
+            o = f"{path}.{os.getpid()}.{os.path.basename(s)}.o"
             cmd = ["hipcc", "--offload-host-only", "-O2", "-std=c++17", "-fPIC", "-w", "-I", _build.INCLUDE, "-I", _build.BUILD_DIR, "-I", host,
                    "-c", s, "-o", o]
             procs.append((subprocess.Popen(cmd), o))
         assert all(p.wait() == 0 for p, _ in procs)
         objs = [o for _, o in procs]
-        subprocess.run(["g++", "-shared", "-Wl,-Bsymbolic", *objs, "-o", path + ".tmp", "-L/opt/rocm/lib", "-lhiprtc",
+        subprocess.run(["g++", "-shared", "-Wl,-Bsymbolic", *objs, "-o", f"{path}.{os.getpid()}.tmp", "-L/opt/rocm/lib", "-lhiprtc",
                         "-Wl,-rpath,/opt/rocm/lib"], check=True)
         for o in objs:
             os.unlink(o)
-        os.replace(path + ".tmp", path)
+        os.replace(f"{path}.{os.getpid()}.tmp", path)
     lib = ctypes.CDLL(path)
     for name, f in vars(_hip._lib).items():
         if name.startswith("ptowsp_"):
