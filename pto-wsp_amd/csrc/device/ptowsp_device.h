@@ -2129,7 +2129,9 @@ struct DecodeWave {
         // o <- o * a + p @ v on the matrix cores: v_mfma_f32_16x16x16 with
         // M = query rows, K = the page's 16 tokens, N = 16 head dims.  p is
         // fp32 and enters in parts of 16 bits (split4), a product per part and
-        // MFMA step; the lane's scores are already its A operand (query row l%16,
+        // MFMA step, all of one shape (two parts side by side in a 16x16x32
+        // MFMA, with the third in a 16x16x16 one right behind it on the same
+        // accumulator, gave wrong sums); the lane's scores are already its A operand (query row l%16,
         // tokens 4*(l/16)..+3).  MFMA e covers head dims DV*n + e (n = l%16):
         // lane (n, l/16) supplies V[tokens 4*(l/16)..+3][DV*n + e] straight
         // from its page registers (one 16-bit half of pg.v[i][e/2] per token)
